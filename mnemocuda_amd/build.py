@@ -23,7 +23,7 @@ CALLER = PKG / "engine_calls"  # tests/c_caller/engine_calls.c, linked against L
 GRAPH_CALLER = PKG / "attn_graph"  # tests/c_caller/attn_graph.c, linked against LIB
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 
-HIP_SOURCES = ["abi.hip", "gemv_launch.hip", "router.hip", "gemm.hip", "moe.hip", "sample.hip", "attn.hip", "attn_decode.hip", "embed.hip"]
+HIP_SOURCES = ["abi.hip", "gemv_launch.hip", "router.hip", "gemm.hip", "gemm_grouped.hip", "moe.hip", "sample.hip", "attn.hip", "attn_decode.hip", "embed.hip"]
 C_SOURCES = ["host/mnemo_host.c", "host/mnemo_model.c"]
 
 HIPCC_FLAGS = [

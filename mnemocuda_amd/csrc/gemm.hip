@@ -40,123 +40,11 @@
 // scales, the fma) where the exact f16 form needs one.
 #include <algorithm>
 
+#include "gemm_ops.hpp"
 #include "mnemo_common.hpp"
 #include "mnemo_internal.hpp"
 
 namespace mnemo {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-// ------------------------------------------------------------------ operand conversions
-// Byte selectors placing bytes (0, 1) / (2, 3) of a dword under the f16 exponent byte 0x64:
-// the pair (1024 + b0, 1024 + b1) exactly.
-constexpr uint32_t kSelLo = 0x04010400u, kSelHi = 0x04030402u;
-
-__device__ __forceinline__ h2 magic_pair(uint32_t v, uint32_t sel) {
-    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, sel));
-}
-// q * sc for two 4-bit quants: (1024 + q) * sc - 1024 * sc in one fused f16 fma, whose
-// result q * sc <= 945 is an integer f16 holds exactly
-__device__ __forceinline__ uint32_t q4_scaled(uint32_t v, uint32_t sel, h2 sc, h2 nsc) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(v, sel), sc, nsc));
-}
-// q8 as f16 integers: q8 ^ 0x80 under 0x64 is 1152 + q8 exactly
-__device__ __forceinline__ void q8x4_exact(uint32_t v, uint32_t &o0, uint32_t &o1) {
-    const h2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const uint32_t u = v ^ 0x80808080u;
-    o0 = __builtin_bit_cast(uint32_t, magic_pair(u, kSelLo) + off);
-    o1 = __builtin_bit_cast(uint32_t, magic_pair(u, kSelHi) + off);
-}
-// Q6_K: two 6-bit quant bytes as the f16 pair (q - 32), exactly
-__device__ __forceinline__ h2 q6_centered(uint32_t v, uint32_t sel) {
-    const h2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-    return magic_pair(v, sel) + off;
-}
-__device__ __forceinline__ uint32_t h2u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
-
-// byte i of the 12 packed scale bytes held in three dwords
-__device__ __forceinline__ uint32_t sbyte(uint32_t s0, uint32_t s1, uint32_t s2, int i) {
-    const uint32_t w = i < 4 ? s0 : (i < 8 ? s1 : s2);
-    return (w >> (8 * (i & 3))) & 0xFFu;
-}
-// (sc, m) of sub-block j (get_scale_min_k4, kernels.cu:45-53)
-__device__ __forceinline__ void q4k_scale_min(uint32_t s0, uint32_t s1, uint32_t s2, int j, uint32_t &sc,
-                                              uint32_t &m) {
-    if (j < 4) {
-        sc = sbyte(s0, s1, s2, j) & 63;
-        m = sbyte(s0, s1, s2, j + 4) & 63;
-    } else {
-        sc = (sbyte(s0, s1, s2, j + 4) & 15) | ((sbyte(s0, s1, s2, j - 4) >> 6) << 4);
-        m = (sbyte(s0, s1, s2, j + 4) >> 4) | ((sbyte(s0, s1, s2, j) >> 6) << 4);
-    }
-}
-
-// The 8 six-bit mins of a Q4_K super-block as bytes, sub-blocks 0-3 / 4-7 (the packed form of
-// get_scale_min_k4, kernels.cu:45-53: m_j = scales[j+4] & 63 for j < 4, else
-// (scales[j+4] >> 4) | ((scales[j] >> 6) << 4)); hdr.z, hdr.w hold scale bytes 4-7, 8-11.
-__device__ __forceinline__ uint2 q4k_mins(const uint4 &hdr) {
-    return make_uint2(hdr.z & 0x3F3F3F3Fu, ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u));
-}
-// Q4_K min-term operand of one super-block: for its 8 sub-blocks, -dmin * m_s as an exact
-// f16 hi + lo pair (dmin is an f16, m a 6-bit integer: 17 significant bits), in packed f16:
-// hi = the product rounded, lo = fma(m, -dmin, -hi), the remainder (at most 6 significant
-// bits, a multiple of dmin's last place: exact, also in the subnormal range)
-__device__ __forceinline__ void q4k_min_operand_m(uint2 mins, uint32_t dmin_bits, h8 &hi, h8 &lo) {
-    const _Float16 nd = -__builtin_bit_cast(_Float16, (uint16_t)dmin_bits);
-    const h2 ndd = {nd, nd};
-    const h2 off = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    uint32_t H[4], L[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const h2 m = magic_pair(i < 2 ? mins.x : mins.y, (i & 1) ? kSelHi : kSelLo) + off;  // exact
-        const h2 h = m * ndd;
-        H[i] = h2u(h);
-        L[i] = h2u(__builtin_elementwise_fma(m, ndd, -h));
-    }
-    hi = __builtin_bit_cast(h8, make_uint4(H[0], H[1], H[2], H[3]));
-    lo = __builtin_bit_cast(h8, make_uint4(L[0], L[1], L[2], L[3]));
-}
-__device__ __forceinline__ void q4k_min_operand(const uint4 &hdr, h8 &hi, h8 &lo) {
-    q4k_min_operand_m(q4k_mins(hdr), hdr.x >> 16, hi, lo);
-}
-// the ds halves of the 8 sub-blocks of a super-block: two Q8_1 block headers
-__device__ __forceinline__ h8 ds_operand(const uint4 &b0, const uint4 &b1) {
-    const uint32_t sel = 0x07060302u;  // the high halves of two dwords
-    const uint4 u = make_uint4(__builtin_amdgcn_perm(b0.y, b0.x, sel), __builtin_amdgcn_perm(b0.w, b0.z, sel),
-                               __builtin_amdgcn_perm(b1.y, b1.x, sel), __builtin_amdgcn_perm(b1.w, b1.z, sel));
-    return __builtin_bit_cast(h8, u);
-}
-
-// Copies 16 bytes per lane from global memory straight into LDS: lane i's bytes land at
-// dst + 16 i (dst wave-uniform).  The instruction is written out because the compiler, which
-// cannot tell the copies' LDS targets from other LDS buffers, otherwise puts a wait for all
-// of them in front of the next LDS read, and the copies never overlap anything (MoE prefill
-// 856 -> 772 us at 512 tokens, 376 -> 327 us at 37; 128 experts of 4096 -> 1536, top-8).
-// Nothing waits for these copies but the explicit vmcnt waits below.
-__device__ __forceinline__ void lds_copy16(const void *src, void *dst) {
-    const uint32_t l = __builtin_amdgcn_readfirstlane(
-        (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)dst);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(src) : "memory", "m0");
-}
-
-// The same after LDS writes made by global_load_lds: those complete with the wave's vector
-// memory counter, so the wave waits until at most N vector memory operations (the ones it
-// issued after the LDS loads) are outstanding.
-template <int N>
-__device__ __forceinline__ void lds_dma_barrier() {
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-    lds_barrier();
-}
-
-__device__ __forceinline__ f4 mfma(const h8 &a, const h8 &b, const f4 &c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4 mfma0(const h8 &a, const h8 &b) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-}
 
 // ------------------------------------------------------------------ tiled kernel
 // A workgroup computes a 128 x 128 tile (weight rows x tokens) over one K slice (blockIdx.z
@@ -436,20 +324,11 @@ __device__ __forceinline__ void mfma_step(const Frags<TYPE> &f, const Stage<TYPE
 }
 
 struct GemmArgs {
-    const uint8_t *W;   // weights [M][K] (plain); expert table base (grouped)
-    const void *A;      // Q8_1 MMQ rows (plain); staged q8 rows, f16 integers (grouped)
-    const float *a_rho;      // grouped: [rows][K/32] token scale ratios
-    const uint16_t *a_ds;    // grouped: [rows][K/32] f16 ds
-    const float *a_dlast;    // grouped: [rows] last nonzero d8 (1 if none)
+    const uint8_t *W;  // weights [M][K]
+    const uint8_t *A;  // Q8_1 MMQ rows [N]
     float *out;
     int M, K, N, splits;
     int out_ld;
-    // grouped launches
-    size_t expert_stride, w_off, w_off2;  // expert e's matrix at W + e*stride + w_off (up: w_off2)
-    const int *counts;                   // [n_experts] rows per expert
-    const int *offsets;                  // [n_experts] first expert-sorted row
-    const int *perm;                     // [rows] expert-sorted row -> token (SwiGLU gather)
-    const int *tiles;                    // [max_tiles] (expert << 16) | n_tile; tiles[-1] = count
 };
 
 template <int TYPE, bool ATOMIC>
@@ -480,7 +359,7 @@ __global__ void __launch_bounds__(kThreads) gemm_q8_1_kernel(GemmArgs g) {
     // loader role: thread -> (row / token lr, part lp); rows past the end re-read the last
     const int lr = tid / kParts, lp = tid % kParts;
     const uint8_t *wrow = g.W + (size_t)min(i0 + lr, g.M - 1) * wrow_bytes;
-    const uint8_t *arow = (const uint8_t *)g.A + (size_t)min(j0 + lr, g.N - 1) * (K / 128) * kQ81Bytes;
+    const uint8_t *arow = g.A + (size_t)min(j0 + lr, g.N - 1) * (K / 128) * kQ81Bytes;
     LoaderState ls{1.0f, 1.0f};
 
     f4 acc[4][kNB];
@@ -592,7 +471,7 @@ __global__ void __launch_bounds__(kThreads) gemm_q8_1_kernel(GemmArgs g) {
             }
 #pragma unroll
             for (int b = 0; b < kNB; b++) {
-                const uint8_t *ap = (const uint8_t *)g.A +
+                const uint8_t *ap = g.A +
                                     (size_t)min(j0 + wj + 16 * b + (lane & 15), g.N - 1) * (K / 128) * kQ81Bytes;
                 blk[b][0] = valid ? ld16(ap + (size_t)(2 * sb) * kQ81Bytes) : make_uint4(0, 0, 0, 0);
                 blk[b][1] = valid ? ld16(ap + (size_t)(2 * sb + 1) * kQ81Bytes) : make_uint4(0, 0, 0, 0);
@@ -672,8 +551,9 @@ __global__ void __launch_bounds__(kThreads) gemm_q8_1_kernel(GemmArgs g) {
 // fp32 rows [N][K] -> the grouped kernel's operand form of cuda_quantize_mmq_q8_1's output
 // (per 32 values d = amax/127, q = rint(x*127/amax) clamped to +-127, ds = f16(d * sum x);
 // gemm_q4k.cu:327-358): q8 as f16 integers [N][K], the f16 ds [N][K/32], the running-scale
-// ratio rho_s = d8eff_{s-1} / d8eff_s [N][K/32] (d8eff: the last nonzero f16 d8 at or before
-// s, 1 before the first) and the last d8eff of the row [N].  One wave per row.
+// ratio rho_s = d8eff_{s-1} / d8eff_s [N][K/32] and d8eff at the end of every window of 32
+// sub-blocks (1024 values) [N][ceil(K/1024)].  d8eff is the last nonzero f16 d8 at or before s
+// in s's window, 1 before the window's first.  One wave per row.
 constexpr int kStageThreads = 256;
 
 __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *__restrict__ x, int K, int N,
@@ -686,8 +566,8 @@ __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *_
     const int nsub = K / 32;
     const float4 *xr = (const float4 *)(x + (size_t)row * K);
     _Float16 *qrow = q8 + (size_t)row * K;
-    float carry = 1.0f;  // d8eff before this pass's first block
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint64_t below = (1ull << lane) - 1;                       // the lanes before this one ..
+    const uint64_t window = lane < 32 ? 0xFFFFFFFFull : ~0xFFFFFFFFull;  // .. and those of its window
     for (int b0 = 0; b0 < nsub; b0 += 64) {
         const int b = b0 + lane;
         float d8 = 0.0f;
@@ -730,17 +610,16 @@ __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *_
             for (int i = 0; i < 4; i++)
                 dst[i] = make_uint4(o[4 * i] & keep, o[4 * i + 1] & keep, o[4 * i + 2] & keep, o[4 * i + 3] & keep);
         }
-        // running scale: the last nonzero d8 before each block (the carry if none in this pass)
-        const uint64_t nz = __ballot(d8 != 0.0f);
-        const uint64_t m = nz & below;
-        const int src = m ? 63 - __builtin_clzll(m) : 0;
-        const float prev_in = __shfl(d8, src);
-        const float prev = m ? prev_in : carry;
+        // running scale: the last nonzero d8 before each block in its window
+        const uint64_t m = __ballot(d8 != 0.0f) & below & window;
+        const float prev_in = __shfl(d8, m ? 63 - __builtin_clzll(m) : 0);
+        const float prev = m ? prev_in : 1.0f;
         const float cur = d8 != 0.0f ? d8 : prev;
-        if (b < nsub) rho[(size_t)row * nsub + b] = prev / cur;
-        carry = __shfl(cur, 63);
+        if (b < nsub) {
+            rho[(size_t)row * nsub + b] = prev / cur;
+            if ((b & 31) == 31 || b == nsub - 1) dlast[(size_t)row * ((nsub + 31) / 32) + b / 32] = cur;
+        }
     }
-    if (lane == 0) dlast[row] = carry;
 }
 
 int launch_stage_f32(const float *x, int K, int N, StagedAct sa, hipStream_t s) {
@@ -785,7 +664,7 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
     // the call may sit inside a graph capture
     GemmArgs g{};
     g.W = (const uint8_t *)w;
-    g.A = act;
+    g.A = (const uint8_t *)act;
     g.out = out;
     g.M = M;
     g.K = K;
@@ -808,642 +687,6 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
     }
 #undef MNEMO_GEMM_LAUNCH
     return check_launch("gemm_q8_1");
-}
-
-// ------------------------------------------------------------------ skinny grouped kernel
-// The grouped expert GEMMs of the MoE prefill: an expert receives a few tens of tokens, so a
-// tile is at most kGroupTile (64) token rows and the weights dominate the traffic.  A
-// workgroup of 8 waves multiplies one token tile with 8 x 16R weight rows; every wave owns R
-// row tiles of 16 and converts its own A operands in registers, and the tile's staged
-// activation rows are shared through LDS.  Each MFMA covers one sub-block (the running scale
-// needs the exact per-sub-block sums): lane group q = lane/16 holds values 8q .. 8q+7 of the
-// sub-block, i.e.
-//   Q4_K sub-block j = 2g + h: qs bytes 32g + 8q .. +7, nibble h;
-//   Q6_K sub-block j = 4H + grp: ql bytes 64H + 32(grp%2) + 8q .. +7 (nibble grp/2), qh bytes
-//        32H + 8q .. +7 (bits 2grp), scale 8H + 2grp + q/2;
-// and the activation fragment is the staged row's values 32j + 8q .. +7 (natural order).
-// Q4_K weights reach the wave through its own LDS area: the 16 rows x 144 B of a tile's
-// block are 144 row-contiguous 16-byte chunks copied with global_load_lds (whole cache lines
-// per request, no registers held while they are in flight -- lanes loading their own 8-byte
-// pieces touch 16 rows per instruction and kept the L1 busy at ~3 TB/s in a read test
-// against ~4.8 TB/s for the copies), then read back per lane.  Q6_K blocks (210 B, 2-byte
-// aligned) are copied as dwords (sk_copy_q6).
-constexpr int kSkTok = kGroupTile;  // token rows per tile: up to 4 column tiles of 16
-// weight rows per wave: SwiGLU one gate and one up tile of 16 (same features); grouped two
-// tiles of 16 (Q4_K) or one (Q6_K, whose raw blocks take more registers)
-template <int TYPE, int MODE>
-constexpr int sk_rows_per_wave() { return MODE == 1 || TYPE == kTypeQ4K ? 32 : 16; }
-// waves per workgroup: Q4_K 8 (one workgroup per CU: its double-buffered weight areas fill
-// the LDS), Q6_K 16 (single-buffered weight areas, four waves per SIMD within 128 registers)
-template <int TYPE>
-constexpr int sk_waves() { return TYPE == kTypeQ6K ? 16 : 8; }
-// activation staging passes of a workgroup of W waves (2W rows of 32 chunks per pass); rows
-// past NB 16 repeat the tile's last token into the unused rest of the buffer
-template <int NB, int W>
-constexpr int sk_passes() { return (NB * 16 + 2 * W - 1) / (2 * W); }
-// One block of a 16-row tile is 2304 B = 144 chunks of 16 B.  Every copy instruction is
-// issued by the whole wave (a lane-predicated copy invites the compiler to merge it with its
-// neighbour and derive the wave-uniform LDS address from the wrong lane): chunks 0-127 of
-// tile a go to bytes 2048a .. of the wave's area with two copies, chunks 128-143 of all
-// tiles to the tail at 2048R + 256a with one copy, whose lanes past 16R repeat a chunk into
-// the unused rest of the tail.
-template <int R>
-constexpr int sk_q4_area() { return 2048 * R + 1024; }
-template <int R>
-constexpr int sk_q4_copies() { return 2 * R + 1; }
-
-// Q6_K raw bytes of one row tile's lane values for one block
-struct SkRaw6 {
-    uint2 ql[4];  // ql bytes 64H + 32p + 8q .. +7 (index 2H + p)
-    uint2 qh[2];  // qh bytes 32H + 8q .. +7
-    uint32_t sc[2];  // the lane's scale bytes of halves 0 / 1 (byte grp: scale 8H + 2grp + q/2)
-    uint32_t d;      // f16 d
-};
-// Q6_K blocks reach the wave through its LDS area by 16-byte copies (lanes loading their
-// own 8-byte pieces touch 16 rows per instruction; with those loads replaced by constants the
-// cfg5 prefill took 0.75 instead of 1.01 ms).  A block is 210 B, so every other one starts at
-// 2 mod 4: row r's window starts at the dword that holds the block's first byte (sh = block
-// offset & 2 bytes before it) and occupies chunk slots 15 r .. 15 r + 14 of the area (240 B
-// per row: the 16 rows' reads fall in distinct banks).  Chunks 0-12 are window bytes
-// 16 ch ..; chunk 13 is window bytes 196-211 when sh = 2 (block bytes 194-209) and a repeat of
-// chunk 12 when sh = 0; chunk 14 repeats chunk 12.  So no copy reads past its block, and the
-// block's bytes 0-207 are in the area; d (bytes 208-209) is loaded by the lanes themselves.
-// Slot t = 64 i + lane is written by copy i; slots past 239 repeat row 15's chunk 12.
-constexpr int kSk6Slots = 15;
-constexpr int kSk6Copies = 4;
-constexpr int kSk6Area = kSk6Copies * 1024;
-// vector memory instructions per block: the copies and the 2-byte d
-constexpr int kSk6Loads = kSk6Copies + 1;
-
-// the copies of block k: x6[i] = (offset of the slot's row from the tile's 4-byte aligned
-// start) + window offset of the chunk, bit 0 set for chunk 13 (moved 4 bytes on when sh = 2)
-__device__ __forceinline__ void sk_copy_q6(const uint8_t *tile, const uint32_t (&x6)[kSk6Copies], int k,
-                                           uint8_t *dst) {
-#pragma unroll
-    for (int i = 0; i < kSk6Copies; i++) {
-        const uint32_t a = x6[i] + (uint32_t)(kQ6KBytes * k);
-        const uint32_t o = (a & ~3u) + ((a & 1u) ? (a & 2u) << 1 : 0u);
-        lds_copy16(tile + o, (dst + 1024 * i));
-    }
-}
-
-// the lane's raw values of row c's block from the wave's LDS area (sh: the block's
-// misalignment, 0 or 2 bytes); d arrives separately
-__device__ __forceinline__ void sk_read6(const uint8_t *area, int c, int q, uint32_t sh, SkRaw6 &r) {
-    const uint32_t *a = (const uint32_t *)area + 4 * kSk6Slots * c;
-    auto rd8 = [&](int o) {  // block bytes o .. o + 7, o a multiple of 8
-        const uint32_t w0 = a[o >> 2], w1 = a[(o >> 2) + 1], w2 = a[(o >> 2) + 2];
-        return make_uint2(__builtin_amdgcn_alignbyte(w1, w0, sh), __builtin_amdgcn_alignbyte(w2, w1, sh));
-    };
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.ql[i] = rd8(64 * (i >> 1) + 32 * (i & 1) + 8 * q);
-#pragma unroll
-    for (int H = 0; H < 2; H++) r.qh[H] = rd8(128 + 32 * H + 8 * q);
-    // of the 16 scale bytes the lane needs 8H + 2grp + q/2: bytes q/2, 2 + q/2, .. of each
-    // dword, packed per half; window dword 52 (sh = 2 only) is the last of chunk 13
-    uint32_t w[5];
-#pragma unroll
-    for (int i = 0; i < 4; i++) w[i] = a[48 + i];
-    w[4] = a[sh ? 55 : 52];
-    uint4 sc;
-    sc.x = __builtin_amdgcn_alignbyte(w[1], w[0], sh);
-    sc.y = __builtin_amdgcn_alignbyte(w[2], w[1], sh);
-    sc.z = __builtin_amdgcn_alignbyte(w[3], w[2], sh);
-    sc.w = __builtin_amdgcn_alignbyte(w[4], w[3], sh);
-    const uint32_t sel = 0x06040200u + 0x01010101u * (uint32_t)(q >> 1);
-    r.sc[0] = __builtin_amdgcn_perm(sc.y, sc.x, sel);
-    r.sc[1] = __builtin_amdgcn_perm(sc.w, sc.z, sel);
-}
-
-// Q4_K lane view of a tile's block: the header (d, dmin, scales) and the lane's qs bytes
-struct SkQ4 {
-    uint4 h;
-    uint2 a[4];  // qs bytes 32g + 8q .. +7
-};
-// byte o of tile a's block in the wave's LDS area (reads of 8 or 16 aligned bytes never
-// straddle the split at 2048)
-template <int R>
-__device__ __forceinline__ const uint8_t *sk_q4_at(const uint8_t *area, int a, int o) {
-    return o < 2048 ? area + 2048 * a + o : area + 2048 * R + 256 * a + (o - 2048);
-}
-template <int R>
-__device__ __forceinline__ SkQ4 sk_read_q4(const uint8_t *area, int a, int c, int q) {
-    SkQ4 r;
-    const int row = c * kQ4KBytes;
-    r.h = *(const uint4 *)sk_q4_at<R>(area, a, row);
-#pragma unroll
-    for (int g = 0; g < 4; g++) r.a[g] = *(const uint2 *)sk_q4_at<R>(area, a, row + 16 + 32 * g + 8 * q);
-    return r;
-}
-// the 8 six-bit scales of a Q4_K block as bytes (get_scale_min_k4, kernels.cu:45-53): sub-blocks
-// 0-3 are the low 6 bits of bytes 0-3, 4-7 the low nibbles of bytes 8-11 with bits 6-7 of
-// bytes 0-3 above them (the packed form of gemm_q4k.cu:53-56)
-__device__ __forceinline__ void q4k_scales8(const uint4 &h, uint32_t &lo, uint32_t &hi) {
-    lo = h.y & 0x3F3F3F3Fu;
-    hi = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-}
-// sub-block j's A operand, sc*q for its 8 values: the pair (1024 + sc) from the scale byte
-// under 0x64, so that (sc, -1024 sc) cost three packed operations
-// the scales of sub-blocks 4H + g as f16 pairs (g = 0, 1 | 2, 3) and their products with -1024
-// (odd sub-blocks, the high nibbles, are taken in place as bytes 16 q: their pair is
-// (sc / 16, -64 sc), and (1024 + 16 q) * sc / 16 - 64 sc = q * sc in the same exact fma)
-struct Sk4Scales {
-    h2 s[2], n[2];
-};
-__device__ __forceinline__ Sk4Scales sk_scales4(uint32_t sc4) {
-    Sk4Scales o;
-    const h2 m = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const h2 f = {(_Float16)1.0f, (_Float16)0.0625f};
-    o.s[0] = (magic_pair(sc4, kSelLo) + m) * f;
-    o.s[1] = (magic_pair(sc4, kSelHi) + m) * f;
-    o.n[0] = o.s[0] * m;
-    o.n[1] = o.s[1] * m;
-    return o;
-}
-__device__ __forceinline__ h8 sk_operand4(const SkQ4 &r, const Sk4Scales &T, int j) {
-    const _Float16 sj = T.s[(j & 3) >> 1][j & 1], nj = T.n[(j & 3) >> 1][j & 1];
-    const h2 S = {sj, sj}, N = {nj, nj};
-    const uint2 c = r.a[j >> 1];
-    const uint32_t msk = (j & 1) ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-    const uint32_t w0 = c.x & msk, w1 = c.y & msk;
-    return __builtin_bit_cast(h8, make_uint4(q4_scaled(w0, kSelLo, S, N), q4_scaled(w0, kSelHi, S, N),
-                                             q4_scaled(w1, kSelLo, S, N), q4_scaled(w1, kSelHi, S, N)));
-}
-// Q6_K: the two factors of the lane's 4 scales of half H (sc - b and b, b = sc & 1) as f16
-// pairs, for the half's four sub-blocks at once: e6[g/2] / b6[g/2] hold those of sub-blocks
-// 4H + g (g even, g + 1); zero when d is zero
-struct Sk6Scales {
-    uint32_t e6[2], b6[2];
-};
-__device__ __forceinline__ Sk6Scales sk_scales6(const SkRaw6 &r, int H, bool dzero) {
-    Sk6Scales o;
-    const h2 off = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const uint32_t sc = dzero ? 0u : r.sc[H];
-    q8x4_exact(sc & 0xFEFEFEFEu, o.e6[0], o.e6[1]);  // the even parts of the signed bytes
-    const uint32_t b = sc & 0x01010101u;
-    o.b6[0] = h2u(magic_pair(b, kSelLo) + off);
-    o.b6[1] = h2u(magic_pair(b, kSelHi) + off);
-    return o;
-}
-// Q6_K: the planes (sc - b)(q - 32) and b(q - 32) of sub-block j (S: its half's scales)
-__device__ __forceinline__ void sk_operand6(const SkRaw6 &r, const Sk6Scales &S, int j, h8 &a1, h8 &a2) {
-    const int H = j >> 2, grp = j & 3;
-    const h2 ep = __builtin_bit_cast(h2, S.e6[grp >> 1]);
-    const h2 bp = __builtin_bit_cast(h2, S.b6[grp >> 1]);
-    const h2 E = {ep[grp & 1], ep[grp & 1]}, B = {bp[grp & 1], bp[grp & 1]};
-    const uint2 l = r.ql[2 * H + (grp & 1)], hq = r.qh[H];
-    const int shl = 4 * (grp >> 1), shh = 2 * grp;
-    const uint32_t v0 = ((l.x >> shl) & 0x0F0F0F0Fu) | (((hq.x >> shh) & 0x03030303u) << 4);
-    const uint32_t v1 = ((l.y >> shl) & 0x0F0F0F0Fu) | (((hq.y >> shh) & 0x03030303u) << 4);
-    const h2 c0 = q6_centered(v0, kSelLo), c1 = q6_centered(v0, kSelHi), c2 = q6_centered(v1, kSelLo),
-             c3 = q6_centered(v1, kSelHi);
-    a1 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * E), h2u(c1 * E), h2u(c2 * E), h2u(c3 * E)));
-    a2 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * B), h2u(c1 * B), h2u(c2 * B), h2u(c3 * B)));
-}
-
-// staged activation chunk u (16 B = 8 values) of token row r, XOR-swizzled by the row so
-// that the 16 rows of a fragment read hit distinct banks
-__device__ __forceinline__ int sk_slot(int r, int u) { return r * 256 + ((u ^ (r & 31)) << 3); }
-
-template <int TYPE, int R>
-struct SkLds {
-    static constexpr int kW = TYPE == kTypeQ4K ? sk_q4_area<R>() : kSk6Area;
-    static constexpr int kWBufs = TYPE == kTypeQ4K ? 2 : 1;
-    _Float16 b[2][kSkTok * 256];               // staged q8 of one 256-value block, double-buffered
-    float rho[2][kSkTok * 8];                  // the rows' scale ratios of that block's 8 sub-blocks
-    uint8_t w[kWBufs][sk_waves<TYPE>()][kW];   // each wave's row tiles of one block (Q4_K double-buffered)
-};
-
-// the running row scales at a block start: lane c owns A row c of each tile (its running d
-// and the ratio for this block); the lane's outputs are rows 4q + e, whose ratios come from
-// lanes 4q + e
-template <int NB, int R>
-__device__ __forceinline__ void sk_row_scales(const float (&d)[R], int q, float (&deff)[R], f4 (&acc)[R][NB]) {
-#pragma unroll
-    for (int a = 0; a < R; a++) {
-        const float nd = d[a] == 0.0f ? deff[a] : d[a];
-        const float sg = deff[a] * __builtin_amdgcn_rcpf(nd);
-        deff[a] = nd;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float se = __shfl(sg, 4 * q + e);
-#pragma unroll
-            for (int b = 0; b < NB; b++) acc[a][b][e] *= se;
-        }
-    }
-}
-
-// copies of block kb of the wave's Q4_K row tiles into its LDS area: copy 2a + i moves
-// chunk 64i + lane of tile a, copy 2R the tail chunks (sources from sk_tile's tile_src)
-template <int R>
-__device__ __forceinline__ void sk_copy_q4(const uint8_t *const (&src)[sk_q4_copies<R>()], int kb, uint8_t *dst) {
-#pragma unroll
-    for (int i = 0; i < sk_q4_copies<R>(); i++)
-        lds_copy16(src[i] + (size_t)kb * kQ4KBytes, (dst + 1024 * i));
-}
-
-// One 256-value block k: the activations (and ratios) of block k+1 are copied into the other
-// LDS buffer, the weights of block k+1 into the wave's other LDS area (Q4_K) or into its
-// single area (Q6_K, once the lanes have read block k out of it), then block k is
-// multiplied.  The barrier at the end waits for the activation copies only (they were issued
-// first; memory operations complete in issue order): the weights stay in flight until the
-// next block needs them.
-// Q6_K copy state of a wave: the 4-byte aligned address at or below its first row, the
-// copies' lane offsets (sk_copy_q6), their clamp, row c's offset and the next block's d
-struct Sk6 {
-    const uint8_t *tile;
-    uint32_t x6[kSk6Copies];
-    uint32_t roff, dn;
-};
-template <int TYPE, int NB, int R>
-__device__ __forceinline__ void sk_block(int k, int nkb, int q, int c, int wave, int lane, int tid,
-                                         const uint8_t *const (&tile_src)[sk_q4_copies<R>()],
-                                         const _Float16 *const (&arow)[sk_passes<NB, sk_waves<TYPE>()>()],
-                                         const float *rrow, SkLds<TYPE, R> &L, Sk6 &st, float (&deff)[R],
-                                         f4 (&acc)[R][NB], bool late_min, uint32_t (&mring)[4][R][2]) {
-    constexpr int W = sk_waves<TYPE>();
-    // past the end the last block is copied again (into the idle buffers)
-    const int kn = min(k + 1, nkb - 1);
-    // block k's weights have landed in the wave's LDS area (the memory clobber keeps the
-    // compiler from moving the LDS reads above the wait)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    SkRaw6 cur[R];
-    if constexpr (TYPE == kTypeQ6K) {
-        sk_read6(L.w[0][wave], c, q, (st.roff + (uint32_t)(kQ6KBytes * k)) & 2u, cur[0]);
-        cur[0].d = st.dn;
-        // the reads have returned before the area is refilled below
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-#pragma unroll
-    for (int i = 0; i < sk_passes<NB, W>(); i++)
-        lds_copy16(arow[i] + kn * 256, &L.b[(k + 1) & 1][(2 * wave + 2 * W * i) * 256]);
-    if (wave < (NB * 32 + 63) / 64)  // the ratios: two 16-byte chunks per row, whole waves
-        lds_copy16(rrow + kn * 8, &L.rho[(k + 1) & 1][(tid & ~63) * 4]);
-    __builtin_amdgcn_sched_barrier(0);  // the shared copies go first (the barrier below counts on it)
-    if constexpr (TYPE == kTypeQ4K) {
-        sk_copy_q4<R>(tile_src, kn, L.w[(k + 1) & 1][wave]);
-    } else {
-        sk_copy_q6(st.tile, st.x6, kn, L.w[0][wave]);
-        uint16_t dd;
-        __builtin_memcpy(&dd, st.tile + st.roff + (size_t)kn * kQ6KBytes + 208, 2);
-        st.dn = dd;
-    }
-    // keep the loads here, ahead of the multiplication (the scheduler would otherwise sink
-    // them past it to save registers, and nothing would be in flight during the MFMAs)
-    __builtin_amdgcn_sched_barrier(0);
-
-    SkQ4 w4[R];
-    uint32_t slo[R], shi[R];
-    Sk6Scales s6[R];
-    Sk4Scales s4[R];
-    float d[R];
-#pragma unroll
-    for (int a = 0; a < R; a++) {
-        if constexpr (TYPE == kTypeQ4K) {
-            w4[a] = sk_read_q4<R>(L.w[k & 1][wave], a, c, q);
-            if (late_min) {
-                // the min term's operand of row c: lane group q keeps super-block k when k % 4 == q,
-                // in a ring of four (window order: the newest in slot 0), moved up one slot at
-                // each window's first block (a uniform branch)
-                if ((k & 3) == 0) {
-#pragma unroll
-                    for (int i = 0; i < 2; i++)
-#pragma unroll
-                        for (int j = 3; j > 0; j--) mring[j][a][i] = mring[j - 1][a][i];
-                }
-                const bool cap = (k & 3) == q;
-                // the 8 six-bit mins in 48 bits (m_j at bit 6j) and dmin in the top 16
-                const uint2 mn = q4k_mins(w4[a].h);
-                const uint32_t p0 = (mn.x & 0x3Fu) | ((mn.x >> 2) & 0xFC0u) | ((mn.x >> 4) & 0x3F000u) |
-                                    ((mn.x >> 6) & 0xFC0000u) | ((mn.y & 0x3Fu) << 24) | ((mn.y & 0x300u) << 22);
-                const uint32_t p1 = ((mn.y >> 10) & 0xFu) | ((mn.y >> 12) & 0x3F0u) | ((mn.y >> 14) & 0xFC00u) |
-                                    (w4[a].h.x & 0xFFFF0000u);
-                mring[0][a][0] = cap ? p0 : mring[0][a][0];
-                mring[0][a][1] = cap ? p1 : mring[0][a][1];
-            }
-            d[a] = h2f(w4[a].h.x & 0xFFFFu);
-            q4k_scales8(w4[a].h, slo[a], shi[a]);
-            if (d[a] == 0.0f) slo[a] = shi[a] = 0u;  // the block's products are zero
-        } else {
-            d[a] = h2f(cur[a].d);
-        }
-    }
-    sk_row_scales<NB, R>(d, q, deff, acc);
-    const _Float16 *bb = L.b[k & 1];
-    const float *rb = L.rho[k & 1];
-    // the 8 ratios of each token column: two 16-byte reads (Q4_K); Q6_K reads each where it
-    // is used, to fit its 128-register budget
-    f4 rr[NB][2];
-    if constexpr (TYPE == kTypeQ4K) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            rr[b][0] = *(const f4 *)(rb + (16 * b + c) * 8);
-            rr[b][1] = *(const f4 *)(rb + (16 * b + c) * 8 + 4);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        h8 bf[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) bf[b] = *(const h8 *)(bb + sk_slot(16 * b + c, 4 * j + q));
-#pragma unroll
-        for (int a = 0; a < R; a++) {
-            if (TYPE == kTypeQ6K && (j & 3) == 0) s6[a] = sk_scales6(cur[a], j >> 2, d[a] == 0.0f);
-            h8 a1, a2;
-            if constexpr (TYPE == kTypeQ4K) {
-                if ((j & 3) == 0) s4[a] = sk_scales4(j < 4 ? slo[a] : shi[a]);
-                a1 = sk_operand4(w4[a], s4[a], j);
-            }
-            else sk_operand6(cur[a], s6[a], j, a1, a2);
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                if constexpr (TYPE == kTypeQ4K) acc[a][b] *= rr[b][j >> 2][j & 3];
-                else acc[a][b] *= rb[(16 * b + c) * 8 + j];
-                acc[a][b] = mfma(a1, bf[b], acc[a][b]);
-                if constexpr (TYPE == kTypeQ6K) acc[a][b] = mfma(a2, bf[b], acc[a][b]);
-            }
-        }
-        // Q6_K: one sub-block's fragment reads at a time (fewer spills under the budget)
-        if constexpr (TYPE == kTypeQ6K) __builtin_amdgcn_sched_barrier(0);
-    }
-    lds_dma_barrier<TYPE == kTypeQ4K ? sk_q4_copies<R>() : R * kSk6Loads>();
-}
-
-template <int TYPE, int MODE, int NB>
-__device__ __forceinline__ void sk_tile(const GemmArgs &g, SkLds<TYPE, sk_rows_per_wave<TYPE, MODE>() / 16> &L,
-                                        int wave, int lane, int tid, int e, int j0, int n_rows, int row_base) {
-    constexpr int R = sk_rows_per_wave<TYPE, MODE>() / 16;
-    constexpr int H = R / 2;  // SwiGLU: gate tiles 0 .. H-1, up tiles H .. 2H-1
-    constexpr int W = sk_waves<TYPE>();
-    constexpr int P = sk_passes<NB, W>();
-    const int q = lane >> 4, c = lane & 15;
-    const int K = g.K, nkb = K / 256;
-    const int bbytes = TYPE == kTypeQ4K ? kQ4KBytes : kQ6KBytes;
-    const size_t wrow_bytes = (size_t)nkb * bbytes;
-    const uint8_t *Wm = g.W + (size_t)e * g.expert_stride + g.w_off;
-    const uint8_t *Wm2 = g.W + (size_t)e * g.expert_stride + g.w_off2;
-
-    // weight row r of tile a (rows past M re-read the last)
-    int base;  // SwiGLU: first feature of the wave; grouped: first row
-    if (MODE == 1) base = (blockIdx.x * W + wave) * (16 * H);
-    else base = (blockIdx.x * W + wave) * (16 * R);
-    auto row_ptr = [&](int a, int r) {
-        if (MODE == 1) return (a < H ? Wm : Wm2) + (size_t)min(base + 16 * (a % H) + r, g.M - 1) * wrow_bytes;
-        return Wm + (size_t)min(base + 16 * a + r, g.M - 1) * wrow_bytes;
-    };
-    const uint8_t *wrow[R];  // the lane's own A row c of each tile
-    // Q4_K copy sources: chunk ch of a tile is row ch/9, bytes 16(ch%9) .. of the block
-    const uint8_t *tile_src[sk_q4_copies<R>()];
-    auto chunk_ptr = [&](int a, int ch) { return row_ptr(a, ch / 9) + 16 * (ch % 9); };
-#pragma unroll
-    for (int a = 0; a < R; a++) {
-        wrow[a] = row_ptr(a, c);
-#pragma unroll
-        for (int i = 0; i < 2; i++) tile_src[2 * a + i] = chunk_ptr(a, 64 * i + lane);
-    }
-    tile_src[2 * R] = lane < 16 * R ? chunk_ptr(lane >> 4, 128 + (lane & 15)) : chunk_ptr(R - 1, 143);
-    // Q6_K copies (one tile of 16 consecutive rows): offsets from the 4-byte aligned address
-    // at or below the first (clamped) row, tb its misalignment
-    Sk6 st;
-    if constexpr (TYPE == kTypeQ6K) {
-        const int r0 = min(base, g.M - 1);
-        const uint8_t *t0 = Wm + (size_t)r0 * wrow_bytes;
-        const uint32_t tb = (uint32_t)(uintptr_t)t0 & 3u;
-        st.tile = t0 - tb;
-        auto rel = [&](int r) { return (uint32_t)((min(base + r, g.M - 1) - r0) * wrow_bytes) + tb; };
-#pragma unroll
-        for (int i = 0; i < kSk6Copies; i++) {
-            const int t = 64 * i + lane, row = t < 16 * kSk6Slots ? t / kSk6Slots : 15;
-            const int ch = t < 16 * kSk6Slots ? t % kSk6Slots : 12;
-            st.x6[i] = rel(row) + (ch <= 12 ? 16u * (uint32_t)ch : ch == 13 ? 192u + 1u : 192u);
-        }
-        st.roff = rel(c);
-    }
-    // activation staging role: physical slot tid % 32 of rows r = tid/32 + 2W i, which
-    // holds the logical slot (tid % 32) ^ (r % 32); ratio staging: threads below 2 NB 16 copy
-    // 16-byte chunk tid % 2 of row tid / 2
-    const int sr0 = tid >> 5;
-    const _Float16 *arow[P];
-    auto stage_row = [&](int r) {
-        const int j = min(j0 + r, n_rows - 1);
-        return MODE == 1 ? g.perm[row_base + j] : row_base + j;
-    };
-#pragma unroll
-    for (int i = 0; i < P; i++) {
-        const int r = sr0 + 2 * W * i, u = (tid & 31) ^ (r & 31);
-        arow[i] = (const _Float16 *)g.A + (size_t)stage_row(r) * K + 8 * u;
-    }
-    const float *rrow = g.a_rho + (size_t)stage_row(min(tid >> 1, NB * 16 - 1)) * (K / 32) + 4 * (tid & 1);
-    f4 acc[R][NB];
-    float deff[R];  // running d of the lane's A row c of each tile
-#pragma unroll
-    for (int a = 0; a < R; a++) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-        deff[a] = 1.0f;
-    }
-    int tok[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) tok[b] = stage_row(16 * b + c);
-#pragma unroll
-    for (int i = 0; i < P; i++)
-        lds_copy16(arow[i], &L.b[0][(2 * wave + 2 * W * i) * 256]);
-    if (wave < (NB * 32 + 63) / 64)  // whole waves (rows past NB 16 repeat the last)
-        lds_copy16(rrow, &L.rho[0][(tid & ~63) * 4]);
-    if constexpr (TYPE == kTypeQ4K) {
-        sk_copy_q4<R>(tile_src, 0, L.w[0][wave]);
-    } else {
-        sk_copy_q6(st.tile, st.x6, 0, L.w[0][wave]);
-        uint16_t dd;
-        __builtin_memcpy(&dd, st.tile + st.roff + 208, 2);
-        st.dn = dd;
-    }
-    // Q4_K's min term, sum_s -(dmin*m_s)_i * ds_js, first: the accumulator starts as this
-    // absolute value (the running scales start at 1 and their ratios telescope to
-    // 1 / (last d * last d8), which the epilogue multiplies back).  Windows of 32 sub-blocks,
-    // lane group q holding super-block 4w + q of its A row / token; the loads of up to four
-    // windows are issued together, after the copies of the first block (the two round trips
-    // overlap; no measurable change).  Reading the headers here fetches every weight line of
-    // the tile once more before the main loop.
-    // Q4_K with whole windows and at most four of them (K a multiple of 1024, <= 4096) skips
-    // that: lane group q keeps the mins and dmin of the super-blocks it reads from LDS in the
-    // main loop (64 bits per row and window, four windows), and the term is added to the
-    // absolute values after the loop (cfg5 prefill ~1.04 -> ~1.01 ms, 0 spills at 228 VGPRs;
-    // the same ring unpacked to three dwords spilled 44 VGPRs and was slower).
-    const bool late_min = TYPE == kTypeQ4K && (nkb & 3) == 0 && nkb <= 16;  // uniform
-    uint32_t mring[4][R][2] = {};
-    if (TYPE == kTypeQ4K && !late_min) {
-        const int nwin = (nkb + 3) / 4;
-        for (int w0 = 0; w0 < nwin; w0 += 4) {
-            uint4 hdr[4][R], dsv[4][NB];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int sb = 4 * (w0 + u) + q;
-                const bool valid = sb < nkb;
-#pragma unroll
-                for (int a = 0; a < R; a++)
-                    hdr[u][a] = valid ? ld16(wrow[a] + (size_t)sb * kQ4KBytes) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    dsv[u][b] = valid ? ld16((const uint8_t *)(g.a_ds + (size_t)tok[b] * (K / 32) + 8 * sb))
-                                      : make_uint4(0, 0, 0, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int a = 0; a < R; a++) {
-                    h8 hi, lo;
-                    q4k_min_operand(hdr[u][a], hi, lo);
-#pragma unroll
-                    for (int b = 0; b < NB; b++) {
-                        const h8 bd = __builtin_bit_cast(h8, dsv[u][b]);
-                        acc[a][b] = mfma(lo, bd, mfma(hi, bd, acc[a][b]));
-                    }
-                }
-        }
-    }
-    // every wave's copies of the first block have landed before any wave passes
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    // the loop unrolled by two
-    for (int k = 0; k < nkb; k += 2) {
-        sk_block<TYPE, NB, R>(k, nkb, q, c, wave, lane, tid, tile_src, arow, rrow, L, st, deff, acc, late_min, mring);
-        if (k + 1 >= nkb) break;
-        sk_block<TYPE, NB, R>(k + 1, nkb, q, c, wave, lane, tid, tile_src, arow, rrow, L, st, deff, acc, late_min,
-                              mring);
-    }
-    // the copies issued past the last block land before the workgroup's LDS is released
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-
-    // absolute values: the last nonzero d of the rows (from lanes 4q + x) and d8 of the tokens
-    float dt[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) dt[b] = g.a_dlast[tok[b]];
-#pragma unroll
-    for (int a = 0; a < R; a++)
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            const float dr = __shfl(deff[a], 4 * q + x);
-#pragma unroll
-            for (int b = 0; b < NB; b++) acc[a][b][x] *= dr * dt[b];
-        }
-    if (late_min) {
-        // the min term on the absolute values: slot j holds window nwin - 1 - j
-        const int nwin = nkb >> 2;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (j >= nwin) break;  // uniform
-            const int sb = 4 * (nwin - 1 - j) + q;
-            h8 bd[NB];
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-                bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + (size_t)tok[b] * (K / 32) + 8 * sb)));
-#pragma unroll
-            for (int a = 0; a < R; a++) {
-                h8 hi, lo;
-                const uint32_t p0 = mring[j][a][0], p1 = mring[j][a][1];
-                const uint2 mn = make_uint2((p0 & 0x3Fu) | ((p0 << 2) & 0x3F00u) | ((p0 << 4) & 0x3F0000u) |
-                                                ((p0 << 6) & 0x3F000000u),
-                                            ((p0 >> 24) & 0x3Fu) | ((p0 >> 22) & 0x300u) | ((p1 << 10) & 0x3C00u) |
-                                                ((p1 << 12) & 0x3F0000u) | ((p1 << 14) & 0x3F000000u));
-                q4k_min_operand_m(mn, p1 >> 16, hi, lo);
-#pragma unroll
-                for (int b = 0; b < NB; b++) acc[a][b] = mfma(lo, bd[b], mfma(hi, bd[b], acc[a][b]));
-            }
-        }
-    }
-
-    // D layout: lane holds weight rows 4q + x of each 16-row tile, token column c
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const int j = j0 + 16 * b + c;
-        if (j >= n_rows) continue;
-        float *orow = g.out + (size_t)(row_base + j) * g.out_ld;
-        if (MODE == 1) {
-#pragma unroll
-            for (int a = 0; a < H; a++) {
-                const int f = base + 16 * a + 4 * q;
-#pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    const float gt = acc[a][b][x], up = acc[a + H][b][x];
-                    if (f + x < g.M) orow[f + x] = gt / (1.0f + expf(-gt)) * up;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < R; a++) {
-                const int i = base + 16 * a + 4 * q;
-#pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (i + x < g.M) orow[i + x] = acc[a][b][x];
-            }
-        }
-    }
-}
-
-// MODE 1: SwiGLU (gate and up rows of the same features, activation rows gathered through
-// perm[], out[q*ld + f] = silu(gate) * up); MODE 2: the expert-sorted rows themselves.
-// The Q6_K kernel's 16 waves (124 KB of LDS, one workgroup per CU) run four per SIMD within
-// 128 registers (a few spill).  The Q4_K kernels' 150 KB of LDS allow one 8-wave workgroup
-// per CU whatever the registers.
-template <int TYPE, int MODE>
-__global__ void __launch_bounds__(TYPE == kTypeQ6K ? 1024 : 512)
-    __attribute__((amdgpu_waves_per_eu(TYPE == kTypeQ6K ? 4 : 1, 8)))
-gemm_skinny_kernel(GemmArgs g) {
-    __shared__ __align__(16) SkLds<TYPE, sk_rows_per_wave<TYPE, MODE>() / 16> L;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if ((int)blockIdx.y >= g.tiles[-1]) return;
-    const int tl = g.tiles[blockIdx.y];
-    const int e = tl >> 16, nt = tl & 0xFFFF;
-    const int n_rows = g.counts[e], row_base = g.offsets[e], j0 = nt * kGroupTile;
-    const int nvalid = min(kGroupTile, n_rows - j0);
-    // one instantiation per count of 16-row column tiles, so every MFMA is unconditional
-    switch ((nvalid + 15) >> 4) {
-    case 1: sk_tile<TYPE, MODE, 1>(g, L, wave, lane, tid, e, j0, n_rows, row_base); break;
-    case 2: sk_tile<TYPE, MODE, 2>(g, L, wave, lane, tid, e, j0, n_rows, row_base); break;
-    case 3: sk_tile<TYPE, MODE, 3>(g, L, wave, lane, tid, e, j0, n_rows, row_base); break;
-    default: sk_tile<TYPE, MODE, 4>(g, L, wave, lane, tid, e, j0, n_rows, row_base); break;
-    }
-}
-
-// Grouped launches used by the MoE prefill path (moe.hip): tiles[] and the routing arrays
-// live in device memory, the grid covers max_tiles tile-list entries.
-int launch_gemm_grouped(int type, int swiglu, const void *experts, size_t expert_stride, size_t w_off,
-                        size_t w_off2, StagedAct act, const int *counts, const int *offsets, const int *perm,
-                        const int *tiles, int max_tiles, float *out, int out_ld, int M, int K, hipStream_t stream) {
-    GemmArgs g{};
-    g.W = (const uint8_t *)experts;
-    g.A = act.q8;
-    g.a_rho = act.rho;
-    g.a_ds = act.ds;
-    g.a_dlast = act.dlast;
-    g.out = out;
-    g.M = M;
-    g.K = K;
-    g.N = 0;
-    g.splits = 1;
-    g.out_ld = out_ld;
-    g.expert_stride = expert_stride;
-    g.w_off = w_off;
-    g.w_off2 = w_off2;
-    g.counts = counts;
-    g.offsets = offsets;
-    g.perm = perm;
-    g.tiles = tiles;
-    if (swiglu && type != kTypeQ4K)
-        return set_error(kErrUnsupportedType, "grouped gate/up GEMM: Q4_K only (type %d)", type);
-#define MNEMO_SKINNY(T_, M_)                                                                                    \
-    do {                                                                                                        \
-        const int rows = sk_rows_per_wave<T_, M_>() / (M_ == 1 ? 2 : 1) * sk_waves<T_>();                      \
-        hipLaunchKernelGGL((gemm_skinny_kernel<T_, M_>), dim3((M + rows - 1) / rows, max_tiles, 1),            \
-                           dim3(64 * sk_waves<T_>()),                                                          \
-                           0, stream, g);                                                                       \
-    } while (0)
-    if (swiglu) MNEMO_SKINNY(kTypeQ4K, 1);
-    else if (type == kTypeQ4K) MNEMO_SKINNY(kTypeQ4K, 2);
-    else MNEMO_SKINNY(kTypeQ6K, 2);
-#undef MNEMO_SKINNY
-    return check_launch("gemm_grouped");
 }
 
 }  // namespace mnemo

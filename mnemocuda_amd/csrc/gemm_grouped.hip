@@ -1,0 +1,550 @@
+// gemm_grouped.hip -- grouped expert GEMMs of the MoE prefill (Q4_K / Q6_K x staged Q8_1 rows).
+//
+// An expert receives from one to a few hundred tokens, so its tokens are cut into tiles of at
+// most kGroupTile (128) rows and a workgroup multiplies one token tile with a strip of weight
+// rows.  Every wave owns R row tiles of 16 and converts its own A operands in registers; the
+// tile's staged activation rows are shared through LDS.  Each MFMA covers one sub-block (the
+// running scale needs the exact per-sub-block sums, gemm.hip): lane group q = lane/16 holds
+// values 8q .. 8q+7 of the sub-block, i.e.
+//   Q4_K sub-block j = 2g + h: qs bytes 32g + 8q .. +7, nibble h;
+//   Q6_K sub-block j = 4H + grp: ql bytes 64H + 32(grp%2) + 8q .. +7 (nibble grp/2), qh bytes
+//        32H + 8q .. +7 (bits 2grp), scale 8H + 2grp + q/2;
+// and the activation fragment is the staged row's values 32j + 8q .. +7 (natural order).
+//
+// What bounds it: up to ~32 tokens per expert the weights' bytes; above, the VALU (per 16 x 32
+// weights ~12 operations to form the operand, and 4 per 16 x 16 outputs for the running
+// scale, against one 16-cycle MFMA).  Both need work in flight from phases that do not
+// coincide, so the kernel runs as several small workgroups per CU (Q4_K: three of 4 waves,
+// 52 KB of LDS and 168 registers each; Q6_K: two of 8 waves, 128 registers): one workgroup's
+// copies, barriers, first loads and final stores pass while the others multiply.
+#include <cstddef>
+
+#include "gemm_ops.hpp"
+#include "mnemo_common.hpp"
+#include "mnemo_internal.hpp"
+
+namespace mnemo {
+
+struct GroupedArgs {
+    const uint8_t *W;        // expert table base
+    const _Float16 *A;       // staged q8 rows, f16 integers [rows][K]
+    const float *a_rho;      // [rows][K/32] token scale ratios
+    const uint16_t *a_ds;    // [rows][K/32] f16 ds
+    const float *a_dlast;    // [rows][ceil(K/1024)] d8 unit at the end of each window
+    float *out;
+    int M, K, out_ld;        // M, K multiples of 256
+    size_t expert_stride, w_off, w_off2;  // expert e's matrix at W + e*stride + w_off (up: w_off2)
+    const int *counts;       // [n_experts] rows per expert
+    const int *offsets;      // [n_experts] first expert-sorted row
+    const int *perm;         // [rows] expert-sorted row -> token (SwiGLU gather)
+    const int *tiles;        // [max_tiles] (expert << 16) | n_tile; tiles[-1] = count
+};
+
+// Shape of a launch by weight type: waves per workgroup, 16-row tiles per wave, bytes of a
+// wave's weight area.  SwiGLU (MODE 1): the wave's tiles are the gate and up rows of the same
+// 16 features.
+template <int TYPE>
+struct Gw;
+template <>
+struct Gw<kTypeQ4K> {
+    static constexpr int kWaves = 4, kR = 2, kArea = 2 * 16 * kQ4KBytes, kCopies = 6, kPerEu = 3;
+};
+// Q6_K blocks (210 B, every other one at 2 mod 4) are copied from the dword that holds their
+// first byte (sh = block offset & 2 bytes before it), 15 chunk slots of 16 B per row (240 B:
+// the 16 rows' reads fall in distinct banks).  Chunks 0-12 are window bytes 16 ch ..; chunk 13
+// is window bytes 196-211 when sh = 2 (block bytes 194-209) and a repeat of chunk 12 when
+// sh = 0; chunk 14 repeats chunk 12.  So no copy reads past its block, and the block's bytes
+// 0-207 are in the area; d (bytes 208-209) is loaded by the lanes themselves.  Slot
+// t = 64 i + lane is written by copy i; slots past 239 repeat row 15's chunk 12.
+constexpr int kSlots6 = 15;
+template <>
+struct Gw<kTypeQ6K> {
+    static constexpr int kWaves = 8, kR = 1, kArea = 4096, kCopies = 4, kPerEu = 4;
+};
+
+// Activations of one stage in LDS: 64 token rows x 128 K values, or 128 rows x 64 values
+// (tiles of more than 64 tokens), double-buffered.
+template <int NB>
+constexpr int gw_stage_k() { return NB <= 4 ? 128 : 64; }
+
+template <int TYPE>
+struct GwLds {
+    _Float16 b[2][64 * 128];
+    float rho[2][256];  // the rows' scale ratios of the stage's 4 (2) sub-blocks
+    uint8_t w[Gw<TYPE>::kWaves][Gw<TYPE>::kArea];  // each wave's row tiles of one block
+};
+
+// element offset of staged chunk u (8 values) of row r; the chunk index is XOR-ed by the row
+// so that the 16 rows of a fragment read cover the banks once
+template <int SK>
+__device__ __forceinline__ int gw_slot(int r, int u) {
+    return SK == 128 ? r * 128 + ((u ^ (r & 15)) << 3) : r * 64 + ((u ^ ((r >> 1) & 7)) << 3);
+}
+template <int SK>
+__device__ __forceinline__ int gw_unslot(int r, int pc) {  // the chunk stored at position pc
+    return SK == 128 ? pc ^ (r & 15) : pc ^ ((r >> 1) & 7);
+}
+
+// Q4_K lane view of a tile's block: the header (d, dmin, scales) and the lane's qs bytes
+struct Raw4 {
+    uint4 h;
+    uint2 a[4];  // qs bytes 32g + 8q .. +7
+};
+__device__ __forceinline__ Raw4 read4(const uint8_t *tile, int c, int q) {
+    Raw4 r;
+    const uint8_t *row = tile + c * kQ4KBytes;
+    r.h = *(const uint4 *)row;
+#pragma unroll
+    for (int g = 0; g < 4; g++) r.a[g] = *(const uint2 *)(row + 16 + 32 * g + 8 * q);
+    return r;
+}
+// the 8 six-bit scales of a Q4_K block as bytes (get_scale_min_k4, kernels.cu:45-53): sub-blocks
+// 0-3 are the low 6 bits of bytes 0-3, 4-7 the low nibbles of bytes 8-11 with bits 6-7 of
+// bytes 0-3 above them (the packed form of gemm_q4k.cu:53-56)
+__device__ __forceinline__ uint32_t scales4(const uint4 &h, int half) {
+    return half == 0 ? h.y & 0x3F3F3F3Fu : (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+}
+// the scales of sub-blocks 4H + g as f16 pairs (g = 0, 1 | 2, 3) and their products with -1024
+// (odd sub-blocks, the high nibbles, are taken in place as bytes 16 q: their pair is
+// (sc / 16, -64 sc), and (1024 + 16 q) * sc / 16 - 64 sc = q * sc in the same exact fma)
+struct Scales4 {
+    h2 s[2], n[2];
+};
+__device__ __forceinline__ Scales4 scale_pairs4(uint32_t sc4) {
+    Scales4 o;
+    const h2 m = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+    const h2 f = {(_Float16)1.0f, (_Float16)0.0625f};
+    o.s[0] = (magic_pair(sc4, kSelLo) + m) * f;
+    o.s[1] = (magic_pair(sc4, kSelHi) + m) * f;
+    o.n[0] = o.s[0] * m;
+    o.n[1] = o.s[1] * m;
+    return o;
+}
+// sub-block j's A operand: sc * q for the lane's 8 values
+__device__ __forceinline__ h8 operand4(const Raw4 &r, const Scales4 &T, int j) {
+    const _Float16 sj = T.s[(j & 3) >> 1][j & 1], nj = T.n[(j & 3) >> 1][j & 1];
+    const h2 S = {sj, sj}, N = {nj, nj};
+    const uint2 c = r.a[j >> 1];
+    const uint32_t msk = (j & 1) ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
+    const uint32_t w0 = c.x & msk, w1 = c.y & msk;
+    return __builtin_bit_cast(h8, make_uint4(q4_scaled(w0, kSelLo, S, N), q4_scaled(w0, kSelHi, S, N),
+                                             q4_scaled(w1, kSelLo, S, N), q4_scaled(w1, kSelHi, S, N)));
+}
+
+// Q6_K raw bytes of one row tile's lane values for one block
+struct Raw6 {
+    uint2 ql[4];     // ql bytes 64H + 32p + 8q .. +7 (index 2H + p)
+    uint2 qh[2];     // qh bytes 32H + 8q .. +7
+    uint32_t sc[2];  // the lane's scale bytes of halves 0 / 1 (byte grp: scale 8H + 2grp + q/2)
+};
+// the lane's raw values of row c's block from the wave's LDS area (sh: the block's
+// misalignment, 0 or 2 bytes)
+__device__ __forceinline__ Raw6 read6(const uint8_t *area, int c, int q, uint32_t sh) {
+    Raw6 r;
+    const uint32_t *a = (const uint32_t *)area + 4 * kSlots6 * c;
+    auto rd8 = [&](int o) {  // block bytes o .. o + 7, o a multiple of 8
+        const uint32_t w0 = a[o >> 2], w1 = a[(o >> 2) + 1], w2 = a[(o >> 2) + 2];
+        return make_uint2(__builtin_amdgcn_alignbyte(w1, w0, sh), __builtin_amdgcn_alignbyte(w2, w1, sh));
+    };
+#pragma unroll
+    for (int i = 0; i < 4; i++) r.ql[i] = rd8(64 * (i >> 1) + 32 * (i & 1) + 8 * q);
+#pragma unroll
+    for (int H = 0; H < 2; H++) r.qh[H] = rd8(128 + 32 * H + 8 * q);
+    // of the 16 scale bytes the lane needs 8H + 2grp + q/2: bytes q/2, 2 + q/2, .. of each
+    // dword, packed per half; window dword 52 (sh = 2 only) is the last of chunk 13
+    uint32_t w[5];
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = a[48 + i];
+    w[4] = a[sh ? 55 : 52];
+    uint4 sc;
+    sc.x = __builtin_amdgcn_alignbyte(w[1], w[0], sh);
+    sc.y = __builtin_amdgcn_alignbyte(w[2], w[1], sh);
+    sc.z = __builtin_amdgcn_alignbyte(w[3], w[2], sh);
+    sc.w = __builtin_amdgcn_alignbyte(w[4], w[3], sh);
+    const uint32_t sel = 0x06040200u + 0x01010101u * (uint32_t)(q >> 1);
+    r.sc[0] = __builtin_amdgcn_perm(sc.y, sc.x, sel);
+    r.sc[1] = __builtin_amdgcn_perm(sc.w, sc.z, sel);
+    return r;
+}
+// the two factors of the lane's 4 scales of half H (sc - b and b, b = sc & 1) as f16 pairs,
+// for the half's four sub-blocks at once: e6[g/2] / b6[g/2] hold those of sub-blocks 4H + g (g
+// even, g + 1); zero when d is zero
+struct Scales6 {
+    uint32_t e6[2], b6[2];
+};
+__device__ __forceinline__ Scales6 scale_pairs6(uint32_t sc) {
+    Scales6 o;
+    const h2 off = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+    q8x4_exact(sc & 0xFEFEFEFEu, o.e6[0], o.e6[1]);  // the even parts of the signed bytes
+    const uint32_t b = sc & 0x01010101u;
+    o.b6[0] = h2u(magic_pair(b, kSelLo) + off);
+    o.b6[1] = h2u(magic_pair(b, kSelHi) + off);
+    return o;
+}
+// the planes (sc - b)(q - 32) and b(q - 32) of sub-block j (S: its half's scales)
+__device__ __forceinline__ void operand6(const Raw6 &r, const Scales6 &S, int j, h8 &a1, h8 &a2) {
+    const int H = j >> 2, grp = j & 3;
+    const h2 ep = __builtin_bit_cast(h2, S.e6[grp >> 1]);
+    const h2 bp = __builtin_bit_cast(h2, S.b6[grp >> 1]);
+    const h2 E = {ep[grp & 1], ep[grp & 1]}, B = {bp[grp & 1], bp[grp & 1]};
+    const uint2 l = r.ql[2 * H + (grp & 1)], hq = r.qh[H];
+    const int shl = 4 * (grp >> 1), shh = 2 * grp;
+    const uint32_t v0 = ((l.x >> shl) & 0x0F0F0F0Fu) | (((hq.x >> shh) & 0x03030303u) << 4);
+    const uint32_t v1 = ((l.y >> shl) & 0x0F0F0F0Fu) | (((hq.y >> shh) & 0x03030303u) << 4);
+    const h2 c0 = q6_centered(v0, kSelLo), c1 = q6_centered(v0, kSelHi), c2 = q6_centered(v1, kSelLo),
+             c3 = q6_centered(v1, kSelHi);
+    a1 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * E), h2u(c1 * E), h2u(c2 * E), h2u(c3 * E)));
+    a2 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * B), h2u(c1 * B), h2u(c2 * B), h2u(c3 * B)));
+}
+
+// One token tile of NB 16-row columns against the workgroup's weight rows.
+template <int TYPE, int MODE, int NB>
+__device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int wave, int lane, int tid, int e,
+                                        int j0, int n_rows, int row_base) {
+    using T = Gw<TYPE>;
+    constexpr int W = T::kWaves, R = T::kR;
+    constexpr bool Q4 = TYPE == kTypeQ4K;
+    constexpr int SK = gw_stage_k<NB>(), NS = 256 / SK, SJ = SK / 32;  // stages per block, sub-blocks per stage
+    constexpr int CH = SK / 8;                                         // 16-byte chunks per staged row
+    constexpr int P = (NB * 16 * CH + 64 * W - 1) / (64 * W);          // copies per wave and stage
+    const int q = lane >> 4, c = lane & 15;
+    const int K = g.K, nkb = K / 256;
+    const uint32_t wrow_bytes = (uint32_t)nkb * (Q4 ? kQ4KBytes : kQ6KBytes);
+    const uint8_t *Wm = g.W + (size_t)e * g.expert_stride + g.w_off;
+    // first weight row of the wave's tiles (SwiGLU: first feature)
+    const int base = (blockIdx.x * W + wave) * (MODE == 1 ? 16 : 16 * R);
+    // the wave's tiles: 16 consecutive rows each
+    const uint8_t *tp[R];
+    tp[0] = Wm + (size_t)base * wrow_bytes;
+    if constexpr (R == 2)
+        tp[1] = MODE == 1 ? g.W + (size_t)e * g.expert_stride + g.w_off2 + (size_t)base * wrow_bytes
+                          : tp[0] + (size_t)16 * wrow_bytes;
+
+    // weight copies.  Q4_K: a tile's block is 144 chunks of 16 B, row ch/9, bytes 16(ch%9);
+    // chunks 0-127 in two copies, 128-143 as 64 dwords in a third.
+    uint32_t wo[Q4 ? 3 : 4];
+    uint32_t tb = 0, roff = 0;
+    if constexpr (Q4) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) wo[i] = ((64 * i + lane) / 9) * wrow_bytes + 16 * ((64 * i + lane) % 9);
+        wo[2] = ((128 + lane / 4) / 9) * wrow_bytes + 16 * ((128 + lane / 4) % 9) + 4 * (lane & 3);
+    } else {
+        // offsets from the 4-byte aligned address at or below the tile's first byte (tb: its
+        // misalignment); bit 0 set for chunk 13, which moves 4 bytes on when sh = 2
+        tb = (uint32_t)(uintptr_t)tp[0] & 3u;
+        tp[0] -= tb;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int t = 64 * i + lane, row = t < 16 * kSlots6 ? t / kSlots6 : 15;
+            const int ch = t < 16 * kSlots6 ? t % kSlots6 : 12;
+            wo[i] = row * wrow_bytes + tb + (ch <= 12 ? 16u * (uint32_t)ch : ch == 13 ? 192u + 1u : 192u);
+        }
+        roff = c * wrow_bytes + tb;
+    }
+    const uint8_t *area = L.w[wave];
+    // LDS addresses of the copies' targets (scalars)
+    const uint32_t lds_w = lds + (uint32_t)offsetof(GwLds<TYPE>, w) + wave * T::kArea;
+    const uint32_t lds_b = lds + wave * 1024, lds_r = lds + (uint32_t)offsetof(GwLds<TYPE>, rho) + wave * 256;
+    auto copy_w = [&](int k) {
+        if constexpr (Q4) {
+#pragma unroll
+            for (int a = 0; a < R; a++) {
+                const uint8_t *s = tp[a] + (size_t)k * kQ4KBytes;
+                lds_copy16(s, wo[0], lds_w + 2304 * a);
+                lds_copy16(s, wo[1], lds_w + 2304 * a + 1024);
+                lds_copy4(s, wo[2], lds_w + 2304 * a + 2048);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t a = wo[i] + (uint32_t)(kQ6KBytes * k);
+                lds_copy16(tp[0], (a & ~3u) + ((a & 1u) ? (a & 2u) << 1 : 0u), lds_w + 1024 * i);
+            }
+        }
+    };
+    // activation copies: LDS chunk slot s = 64 W i + tid holds chunk gw_unslot(s % CH) of row
+    // s / CH; rows past the tile's last repeat it
+    auto stage_row = [&](int r) {
+        const int j = min(j0 + r, n_rows - 1);
+        return MODE == 1 ? g.perm[row_base + j] : row_base + j;
+    };
+    const _Float16 *ap[P];
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        const int s = 64 * W * i + tid, r = s / CH;
+        ap[i] = g.A + (size_t)stage_row(r) * K + 8 * gw_unslot<SK>(r, s % CH);
+    }
+    // ratio copies: float tid of the stage's [row][sub-block] array (waves 0-3)
+    const float *rp = g.a_rho + (size_t)stage_row((tid & 255) / SJ) * (K / 32) + tid % SJ;
+    auto copy_b = [&](int t, int buf) {  // stage t (t * SK values into the rows)
+#pragma unroll
+        for (int i = 0; i < P; i++)
+            if (64 * W * (i + 1) <= NB * 16 * CH || 64 * W * i + 64 * wave < NB * 16 * CH)  // wave-uniform
+                lds_copy16(ap[i] + (size_t)t * SK, lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
+        if (W == 4 || wave < 4) lds_copy4(rp + (size_t)t * SJ, lds_r + buf * (uint32_t)sizeof L.rho[0]);
+    };
+
+    f4 acc[R][NB];
+    float deff[R];  // running d of the lane's A row c of each tile
+#pragma unroll
+    for (int a = 0; a < R; a++) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+        deff[a] = 1.0f;
+    }
+    copy_b(0, 0);
+    copy_w(0);
+    uint32_t dn = 0;  // Q6_K: f16 d of row c's next block
+    auto load_d6 = [&](int k) {
+        uint16_t dd;
+        __builtin_memcpy(&dd, tp[0] + roff + (size_t)k * kQ6KBytes + 208, 2);
+        dn = dd;
+    };
+    if constexpr (!Q4) load_d6(0);
+
+    // Q4_K's min term, sum_s -(dmin*m_s)_i * ds_js, is one product over the sub-block index:
+    // two MFMAs (hi + lo operand) per window of 32 sub-blocks (4 blocks).  Lane group q keeps the
+    // packed mins and dmin of the window's block 4 w + q as it reads the headers (K index 8 q + s
+    // of the MFMA = sub-block s of that block); at the window's end the accumulators become
+    // absolute, take the term and start the next window with unit scales, which is what the
+    // staged ratios assume.  (Adding the term before the main loop read every header's weight
+    // line twice: gate/up of 512 tokens ~1.04 against ~1.01 ms in all.)
+    uint2 mins[Q4 ? R : 1];
+    uint32_t dmins[Q4 ? R : 1];
+    const int nwin = (nkb + 3) / 4;
+    // every wave's copies of the first stage and block have landed before any wave passes
+    wait_vm<0>();
+    lds_barrier();
+
+    for (int k = 0; k < nkb; k++) {
+        const int kn = min(k + 1, nkb - 1);  // past the end the last block is copied again
+        // block k's weights into registers; the area is refilled once they are there
+        Raw4 w4[Q4 ? R : 1];
+        Raw6 w6;
+        float d[R];
+        if constexpr (Q4) {
+#pragma unroll
+            for (int a = 0; a < R; a++) w4[a] = read4(area + 2304 * a, c, q);
+        } else {
+            d[0] = h2f(dn);
+            w6 = read6(area, c, q, (roff + (uint32_t)(kQ6KBytes * k)) & 2u);
+            asm volatile("" : "+v"(d[0]));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const int buf = s & 1;
+            // the next stage's activations go first, then (first stage) the next block's
+            // weights: the first stage's barrier leaves the weights in flight
+            copy_b(s + 1 < NS ? k * NS + s + 1 : kn * NS, buf ^ 1);
+            if (s == 0) {
+                copy_w(kn);
+                if constexpr (!Q4) load_d6(kn);
+                if constexpr (Q4) {
+#pragma unroll
+                    for (int a = 0; a < R; a++) {
+                        d[a] = h2f(w4[a].h.x & 0xFFFFu);
+                        const bool cap = (k & 3) == q;
+                        const uint2 mn = q4k_mins(w4[a].h);
+                        mins[a].x = cap ? mn.x : mins[a].x;
+                        mins[a].y = cap ? mn.y : mins[a].y;
+                        dmins[a] = cap ? w4[a].h.x >> 16 : dmins[a];
+                        if (d[a] == 0.0f) w4[a].h.y = w4[a].h.w = 0u;  // scales 0: the block's products are zero
+                    }
+                } else if (d[0] == 0.0f) {
+                    w6.sc[0] = w6.sc[1] = 0u;
+                }
+                // the running row scales: lane c owns A row c of each tile; the lane's outputs are
+                // rows 4q + x, whose ratios come from lanes 4q + x
+#pragma unroll
+                for (int a = 0; a < R; a++) {
+                    const float nd = d[a] == 0.0f ? deff[a] : d[a];
+                    const float sg = deff[a] * __builtin_amdgcn_rcpf(nd);
+                    deff[a] = nd;
+#pragma unroll
+                    for (int x = 0; x < 4; x++) {
+                        const float se = __shfl(sg, 4 * q + x);
+#pragma unroll
+                        for (int b = 0; b < NB; b++) acc[a][b][x] *= se;
+                    }
+                }
+            }
+            const _Float16 *bb = L.b[buf];
+            const float *rb = L.rho[buf];
+            Scales4 s4[Q4 ? R : 1];
+            Scales6 s6;
+#pragma unroll
+            for (int jj = 0; jj < SJ; jj++) {
+                const int j = SJ * s + jj;  // sub-block of the block
+                float rr[NB];  // the token columns' ratios
+#pragma unroll
+                for (int b = 0; b < NB; b++) rr[b] = rb[(16 * b + c) * SJ + jj];
+                h8 a1[R], a2[Q4 ? 1 : R];
+#pragma unroll
+                for (int a = 0; a < R; a++) {
+                    if constexpr (Q4) {
+                        if (jj == 0) s4[a] = scale_pairs4(scales4(w4[a].h, j >> 2));
+                        a1[a] = operand4(w4[a], s4[a], j);
+                    } else {
+                        if (jj == 0) s6 = scale_pairs6(w6.sc[j >> 2]);
+                        operand6(w6, s6, j, a1[a], a2[a]);
+                    }
+                }
+                constexpr int NG = NB > 4 ? 2 : 1, NC = NB / NG;  // columns in groups of at most 4
+#pragma unroll
+                for (int gr = 0; gr < NG; gr++) {
+                    h8 bf[NC];
+#pragma unroll
+                    for (int b = 0; b < NC; b++)
+                        bf[b] = *(const h8 *)(bb + gw_slot<SK>(16 * (NC * gr + b) + c, 4 * jj + q));
+#pragma unroll
+                    for (int a = 0; a < R; a++)
+#pragma unroll
+                        for (int b = 0; b < NC; b++) {
+                            f4 &ac = acc[a][NC * gr + b];
+                            ac *= rr[NC * gr + b];
+                            ac = mfma(a1[a], bf[b], ac);
+                            if constexpr (!Q4) ac = mfma(a2[a], bf[b], ac);
+                        }
+                    if constexpr (NB >= 6) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (s == NS - 1 && ((k & 3) == 3 || k == nkb - 1)) {  // uniform: the window's end
+                const int w = k >> 2;
+                // the window's last blocks: lane groups past the row's end add nothing
+                const bool valid = 4 * w + q < nkb;
+                const int sb = min(4 * w + q, nkb - 1);
+                int cw = c;  // not known to be loop-invariant: the rows' addresses are formed here, once
+                asm volatile("" : "+v"(cw));  // per window, instead of in registers held through the loop
+                float dr[R][4];
+#pragma unroll
+                for (int a = 0; a < R; a++) {
+#pragma unroll
+                    for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
+                    deff[a] = 1.0f;
+                }
+                constexpr int NC = NB > 4 ? NB / 2 : NB;
+#pragma unroll
+                for (int b0 = 0; b0 < NB; b0 += NC) {
+                    float dt[NC];
+                    h8 bd[Q4 ? NC : 1];
+#pragma unroll
+                    for (int b = 0; b < NC; b++) {
+                        const size_t tok = stage_row(16 * (b0 + b) + cw);
+                        dt[b] = g.a_dlast[tok * nwin + w];
+                        if constexpr (Q4) {
+                            bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
+                            if (!valid) bd[b] = h8{};
+                        }
+                    }
+#pragma unroll
+                    for (int a = 0; a < R; a++) {
+                        h8 hi, lo;
+                        if constexpr (Q4) q4k_min_operand_m(mins[a], valid ? dmins[a] : 0u, hi, lo);
+#pragma unroll
+                        for (int b = 0; b < NC; b++) {
+                            f4 &ac = acc[a][b0 + b];
+#pragma unroll
+                            for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
+                            if constexpr (Q4) ac = mfma(lo, bd[b], mfma(hi, bd[b], ac));
+                        }
+                    }
+                    if constexpr (NB >= 6) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // the next stage's activations have landed for every wave (and, from the second
+            // stage on, the next block's weights)
+            if (s == 0) wait_vm<T::kCopies + (Q4 ? 0 : 1)>();
+            else wait_vm<0>();
+            lds_barrier();
+        }
+    }
+
+    // D layout: lane holds weight rows 4q + x of each 16-row tile, token column c
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int j = j0 + 16 * b + c;
+        if (j >= n_rows) continue;
+        float *orow = g.out + (size_t)(row_base + j) * g.out_ld + base + 4 * q;
+        if constexpr (MODE == 1) {
+            f4 v;
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const float gt = acc[0][b][x], up = acc[R - 1][b][x];
+                v[x] = gt / (1.0f + expf(-gt)) * up;
+            }
+            *(f4 *)orow = v;
+        } else {
+#pragma unroll
+            for (int a = 0; a < R; a++) *(f4 *)(orow + 16 * a) = acc[a][b];
+        }
+    }
+}
+
+// MODE 1: SwiGLU (gate and up rows of the same features, activation rows gathered through
+// perm[], out[q*ld + f] = silu(gate) * up); MODE 2: the expert-sorted rows themselves.
+template <int TYPE, int MODE>
+__global__ void __launch_bounds__(64 * Gw<TYPE>::kWaves)
+    __attribute__((amdgpu_waves_per_eu(Gw<TYPE>::kPerEu, Gw<TYPE>::kPerEu))) gemm_grouped_kernel(GroupedArgs g) {
+    __shared__ __align__(16) GwLds<TYPE> L;
+    const uint32_t lds = lds_addr(&L);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.y >= g.tiles[-1]) return;
+    const int tl = g.tiles[blockIdx.y];
+    const int e = tl >> 16, nt = tl & 0xFFFF;
+    const int n_rows = g.counts[e], row_base = g.offsets[e], j0 = nt * kGroupTile;
+    const int nvalid = min(kGroupTile, n_rows - j0);
+#define MNEMO_GW(NB_) gw_tile<TYPE, MODE, NB_>(g, L, lds, wave, lane, tid, e, j0, n_rows, row_base)
+    // one instantiation per count of 16-row column tiles, so every MFMA is unconditional (5
+    // and 7 run padded to 6 and 8)
+    switch ((nvalid + 15) >> 4) {
+    case 1: MNEMO_GW(1); break;
+    case 2: MNEMO_GW(2); break;
+    case 3: MNEMO_GW(3); break;
+    case 4: MNEMO_GW(4); break;
+    case 5:
+    case 6: MNEMO_GW(6); break;
+    default: MNEMO_GW(8); break;
+    }
+#undef MNEMO_GW
+}
+
+// Grouped launches used by the MoE prefill path (moe.hip): tiles[] and the routing arrays
+// live in device memory, the grid covers max_tiles tile-list entries.  M and K are multiples of
+// 256, so every wave's rows exist.
+int launch_gemm_grouped(int type, int swiglu, const void *experts, size_t expert_stride, size_t w_off,
+                        size_t w_off2, StagedAct act, const int *counts, const int *offsets, const int *perm,
+                        const int *tiles, int max_tiles, float *out, int out_ld, int M, int K, hipStream_t stream) {
+    GroupedArgs g{};
+    g.W = (const uint8_t *)experts;
+    g.A = act.q8;
+    g.a_rho = act.rho;
+    g.a_ds = act.ds;
+    g.a_dlast = act.dlast;
+    g.out = out;
+    g.M = M;
+    g.K = K;
+    g.out_ld = out_ld;
+    g.expert_stride = expert_stride;
+    g.w_off = w_off;
+    g.w_off2 = w_off2;
+    g.counts = counts;
+    g.offsets = offsets;
+    g.perm = perm;
+    g.tiles = tiles;
+    if (swiglu && type != kTypeQ4K)
+        return set_error(kErrUnsupportedType, "grouped gate/up GEMM: Q4_K only (type %d)", type);
+#define MNEMO_GROUPED(T_, M_)                                                                              \
+    do {                                                                                                   \
+        const int rows = (M_ == 1 ? 16 : 16 * Gw<T_>::kR) * Gw<T_>::kWaves;                                \
+        hipLaunchKernelGGL((gemm_grouped_kernel<T_, M_>), dim3(M / rows, max_tiles), dim3(64 * Gw<T_>::kWaves), 0, \
+                           stream, g);                                                                     \
+    } while (0)
+    if (swiglu) MNEMO_GROUPED(kTypeQ4K, 1);
+    else if (type == kTypeQ4K) MNEMO_GROUPED(kTypeQ4K, 2);
+    else MNEMO_GROUPED(kTypeQ6K, 2);
+#undef MNEMO_GROUPED
+    return check_launch("gemm_grouped");
+}
+
+}  // namespace mnemo

@@ -7,12 +7,13 @@
 namespace mnemo {
 
 // Token rows per tile of a grouped (MoE prefill) GEMM launch, the unit of the tile list the
-// routing writes (up to four 16-token MFMA columns of the grouped kernel).
-constexpr int kGroupTile = 64;
+// routing writes (up to eight 16-token MFMA columns of the grouped kernel).
+constexpr int kGroupTile = 128;
 
 // Activation rows staged for the grouped GEMM (gemm.hip, stage_f32_kernel): the Q8_1 values
 // of each row as f16 integers [rows][K], the f16 ds of each 32-value sub-block [rows][K/32],
-// the running-scale ratio of each sub-block [rows][K/32] and the row's last nonzero d8 [rows].
+// the running-scale ratio of each sub-block [rows][K/32] and the d8 unit at the end of every
+// 1024-value window [rows][ceil(K/1024)].
 struct StagedAct {
     _Float16 *q8;
     float *rho;
