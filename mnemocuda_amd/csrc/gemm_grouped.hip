@@ -32,7 +32,8 @@ struct GroupedArgs {
     const uint16_t *a_ds;    // [rows][K/32] f16 ds
     const float *a_dlast;    // [rows][ceil(K/1024)] d8 unit at the end of each window
     float *out;
-    int M, K, out_ld;        // M, K multiples of 256
+    int K, out_ld;           // K a multiple of 256
+    int row_blocks;          // workgroups per token tile
     size_t expert_stride, w_off, w_off2;  // expert e's matrix at W + e*stride + w_off (up: w_off2)
     const int *counts;       // [n_experts] rows per expert
     const int *offsets;      // [n_experts] first expert-sorted row
@@ -199,8 +200,8 @@ __device__ __forceinline__ void operand6(const Raw6 &r, const Scales6 &S, int j,
 
 // One token tile of NB 16-row columns against the workgroup's weight rows.
 template <int TYPE, int MODE, int NB>
-__device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int wave, int lane, int tid, int e,
-                                        int j0, int n_rows, int row_base) {
+__device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int rb,
+                                        int wave, int lane, int tid, int e, int j0, int n_rows, int row_base) {
     using T = Gw<TYPE>;
     constexpr int W = T::kWaves, R = T::kR;
     constexpr bool Q4 = TYPE == kTypeQ4K;
@@ -212,7 +213,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     const uint32_t wrow_bytes = (uint32_t)nkb * (Q4 ? kQ4KBytes : kQ6KBytes);
     const uint8_t *Wm = g.W + (size_t)e * g.expert_stride + g.w_off;
     // first weight row of the wave's tiles (SwiGLU: first feature)
-    const int base = (blockIdx.x * W + wave) * (MODE == 1 ? 16 : 16 * R);
+    const int base = (rb * W + wave) * (MODE == 1 ? 16 : 16 * R);
     // the wave's tiles: 16 consecutive rows each
     const uint8_t *tp[R];
     tp[0] = Wm + (size_t)base * wrow_bytes;
@@ -489,12 +490,28 @@ __global__ void __launch_bounds__(64 * Gw<TYPE>::kWaves)
     __shared__ __align__(16) GwLds<TYPE> L;
     const uint32_t lds = lds_addr(&L);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if ((int)blockIdx.y >= g.tiles[-1]) return;
-    const int tl = g.tiles[blockIdx.y];
+    // Workgroups go to the 8 XCDs in turn.  The row blocks of one tile share its activation rows, so
+    // they run on one XCD (tiles are dealt to the XCDs in turn, heaviest first) and read them from
+    // its L2; the last n % 8 tiles are spread over all XCDs.  With every tile spread, the rows came
+    // from beyond the L2 for each XCD (512 tokens, gate/up: 1.44 GB fetched for 0.91 GB of weights).
+    const int n = g.tiles[-1], nb = g.row_blocks;
+    int id = blockIdx.x, tile, rb;
+    const int even = (n & ~7) * nb;
+    if (id < even) {
+        const int l = id >> 3;
+        tile = (l / nb) * 8 + (id & 7);
+        rb = l % nb;
+    } else {
+        id -= even;
+        tile = (n & ~7) + id / nb;
+        rb = id % nb;
+    }
+    if (tile >= n) return;
+    const int tl = g.tiles[tile];
     const int e = tl >> 16, nt = tl & 0xFFFF;
     const int n_rows = g.counts[e], row_base = g.offsets[e], j0 = nt * kGroupTile;
     const int nvalid = min(kGroupTile, n_rows - j0);
-#define MNEMO_GW(NB_) gw_tile<TYPE, MODE, NB_>(g, L, lds, wave, lane, tid, e, j0, n_rows, row_base)
+#define MNEMO_GW(NB_) gw_tile<TYPE, MODE, NB_>(g, L, lds, rb, wave, lane, tid, e, j0, n_rows, row_base)
     // one instantiation per count of 16-row column tiles, so every MFMA is unconditional (5
     // and 7 run padded to 6 and 8)
     switch ((nvalid + 15) >> 4) {
@@ -522,7 +539,6 @@ int launch_gemm_grouped(int type, int swiglu, const void *experts, size_t expert
     g.a_ds = act.ds;
     g.a_dlast = act.dlast;
     g.out = out;
-    g.M = M;
     g.K = K;
     g.out_ld = out_ld;
     g.expert_stride = expert_stride;
@@ -537,8 +553,9 @@ int launch_gemm_grouped(int type, int swiglu, const void *experts, size_t expert
 #define MNEMO_GROUPED(T_, M_)                                                                              \
     do {                                                                                                   \
         const int rows = (M_ == 1 ? 16 : 16 * Gw<T_>::kR) * Gw<T_>::kWaves;                                \
-        hipLaunchKernelGGL((gemm_grouped_kernel<T_, M_>), dim3(M / rows, max_tiles), dim3(64 * Gw<T_>::kWaves), 0, \
-                           stream, g);                                                                     \
+        g.row_blocks = M / rows;                                                                           \
+        hipLaunchKernelGGL((gemm_grouped_kernel<T_, M_>), dim3(g.row_blocks * max_tiles),                  \
+                           dim3(64 * Gw<T_>::kWaves), 0, stream, g);                                       \
     } while (0)
     if (swiglu) MNEMO_GROUPED(kTypeQ4K, 1);
     else if (type == kTypeQ4K) MNEMO_GROUPED(kTypeQ4K, 2);

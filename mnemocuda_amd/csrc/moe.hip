@@ -142,40 +142,50 @@ __global__ void __launch_bounds__(kRouteThreads) moe_route_kernel(const int *__r
         running[ex] = acc;
     }
     __syncthreads();
-    // exclusive scans of the counts and of the tiles per expert: thread ex holds expert ex
-    // (E <= 512), a wave-wide scan (DPP shuffles), then the wave totals in wave order
-    __shared__ int wsum[2][kRouteWaves];
+    // exclusive scan of the counts: thread ex holds expert ex (E <= 512), a wave-wide scan
+    // (shuffles), then the wave totals in wave order
+    __shared__ int wsum[kRouteWaves];
     __shared__ int s_off[kMaxMoeExperts];
+    // tiles by their count of 16-row columns, heaviest first: the grouped launches deal them to
+    // the XCDs in turn, so that each gets the same work, and end on the lightest
+    constexpr int kCols = kMoeTileRows / 16;
+    __shared__ int s_cls[kCols + 1];
+    if (tid <= kCols) s_cls[tid] = 0;
     const int c = tid < E ? running[tid] : 0;
-    const int nt = (c + kMoeTileRows - 1) / kMoeTileRows;
-    int ic = c, it = nt;
+    const int full = c / kMoeTileRows, part = (c % kMoeTileRows + 15) / 16;  // part: columns of the last tile
+    int ic = c;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(ic, o), b = __shfl_up(it, o);
-        if (lane >= o) {
-            ic += a;
-            it += b;
-        }
+        const int a = __shfl_up(ic, o);
+        if (lane >= o) ic += a;
     }
-    if (lane == 63) {
-        wsum[0][wave] = ic;
-        wsum[1][wave] = it;
-    }
+    if (lane == 63) wsum[wave] = ic;
     __syncthreads();
-    int bc = 0, bt = 0;
-    for (int w = 0; w < wave; w++) {
-        bc += wsum[0][w];
-        bt += wsum[1][w];
-    }
+    if (full) atomicAdd(&s_cls[kCols], full);
+    if (part) atomicAdd(&s_cls[part], 1);
+    int bc = 0;
+    for (int w = 0; w < wave; w++) bc += wsum[w];
     if (tid < E) {
-        const int oc = bc + ic - c, ot = bt + it - nt;
         counts[tid] = c;
-        offsets[tid] = oc;
-        s_off[tid] = oc;
-        for (int j = 0; j < nt; j++) tiles[1 + ot + j] = (tid << 16) | j;  // expert order
-        if (tid == E - 1) tiles[0] = ot + nt;
+        offsets[tid] = bc + ic - c;
+        s_off[tid] = bc + ic - c;
     }
     __syncthreads();
+    if (tid == 0) {
+        int at = 0;
+        for (int v = kCols; v > 0; v--) {
+            const int n = s_cls[v];
+            s_cls[v] = at;
+            at += n;
+        }
+        tiles[0] = at;
+    }
+    __syncthreads();
+    if (full) {
+        const int at = atomicAdd(&s_cls[kCols], full);
+        for (int j = 0; j < full; j++) tiles[1 + at + j] = (tid << 16) | j;
+    }
+    if (part) tiles[1 + atomicAdd(&s_cls[part], 1)] = (tid << 16) | full;
     // place the pairs (loads of four pairs per thread in flight at a time)
     for (int p0 = 0; p0 < pairs; p0 += 4 * kRouteThreads) {
         int r[4], e[4];
