@@ -42,13 +42,18 @@ struct GroupedArgs {
 };
 
 // Shape of a launch by weight type: waves per workgroup, 16-row tiles per wave, bytes of a
-// wave's weight area.  SwiGLU (MODE 1): the wave's tiles are the gate and up rows of the same
+// wave's weight area, and kLast, the 16-byte copies that end a block's weight copies.  The first
+// stage of a block waits until at most kLast operations are outstanding: 16-byte copies complete
+// in order, so the stage's activations, which went before, have landed.  Nothing else is
+// counted on: loads into registers (Q6_K's d) and 4-byte copies may complete in another order
+// (a wait that counted d among the younger operations let a stage read stale ratios about
+// once in 10^5 workgroups).  SwiGLU (MODE 1): the wave's tiles are the gate and up rows of the same
 // 16 features.
 template <int TYPE>
 struct Gw;
 template <>
 struct Gw<kTypeQ4K> {
-    static constexpr int kWaves = 4, kR = 2, kArea = 2 * 16 * kQ4KBytes, kCopies = 6, kPerEu = 3;
+    static constexpr int kWaves = 4, kR = 2, kArea = 2 * 16 * kQ4KBytes, kLast = 4, kPerEu = 3;
 };
 // Q6_K blocks (210 B, every other one at 2 mod 4) are copied from the dword that holds their
 // first byte (sh = block offset & 2 bytes before it), 15 chunk slots of 16 B per row (240 B:
@@ -60,7 +65,7 @@ struct Gw<kTypeQ4K> {
 constexpr int kSlots6 = 15;
 template <>
 struct Gw<kTypeQ6K> {
-    static constexpr int kWaves = 8, kR = 1, kArea = 4096, kCopies = 4, kPerEu = 4;
+    static constexpr int kWaves = 8, kR = 1, kArea = 4096, kLast = 4, kPerEu = 4;
 };
 
 // Activations of one stage in LDS: 64 token rows x 128 K values, or 128 rows x 64 values
@@ -250,10 +255,13 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         if constexpr (Q4) {
 #pragma unroll
             for (int a = 0; a < R; a++) {
+                lds_copy4(tp[a] + (size_t)k * kQ4KBytes, wo[2], lds_w + 2304 * a + 2048);
+            }
+#pragma unroll
+            for (int a = 0; a < R; a++) {
                 const uint8_t *s = tp[a] + (size_t)k * kQ4KBytes;
                 lds_copy16(s, wo[0], lds_w + 2304 * a);
                 lds_copy16(s, wo[1], lds_w + 2304 * a + 1024);
-                lds_copy4(s, wo[2], lds_w + 2304 * a + 2048);
             }
         } else {
 #pragma unroll
@@ -278,11 +286,11 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     // ratio copies: float tid of the stage's [row][sub-block] array (waves 0-3)
     const float *rp = g.a_rho + (size_t)stage_row((tid & 255) / SJ) * (K / 32) + tid % SJ;
     auto copy_b = [&](int t, int buf) {  // stage t (t * SK values into the rows)
+        if (W == 4 || wave < 4) lds_copy4(rp + (size_t)t * SJ, lds_r + buf * (uint32_t)sizeof L.rho[0]);
 #pragma unroll
         for (int i = 0; i < P; i++)
             if (64 * W * (i + 1) <= NB * 16 * CH || 64 * W * i + 64 * wave < NB * 16 * CH)  // wave-uniform
                 lds_copy16(ap[i] + (size_t)t * SK, lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
-        if (W == 4 || wave < 4) lds_copy4(rp + (size_t)t * SJ, lds_r + buf * (uint32_t)sizeof L.rho[0]);
     };
 
     f4 acc[R][NB];
@@ -455,7 +463,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
             }
             // the next stage's activations have landed for every wave (and, from the second
             // stage on, the next block's weights)
-            if (s == 0) wait_vm<T::kCopies + (Q4 ? 0 : 1)>();
+            if (s == 0) wait_vm<T::kLast>();
             else wait_vm<0>();
             lds_barrier();
         }
