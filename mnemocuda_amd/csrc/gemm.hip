@@ -38,7 +38,7 @@
 // at the f16 MFMA's rate (16 cycles for 16x16x32, measured) while needing three VALU
 // operations per output per sub-block (int -> float, the product of the row and token
 // scales, the fma) where the exact f16 form needs one.
-#include <algorithm>
+#include <cstddef>
 
 #include "gemm_ops.hpp"
 #include "mnemo_common.hpp"
@@ -47,502 +47,438 @@
 namespace mnemo {
 
 // ------------------------------------------------------------------ tiled kernel
-// A workgroup computes a 128 x 128 tile (weight rows x tokens) over one K slice (blockIdx.z
-// of `splits`, whole super-blocks).  Its waves form a 2 (rows: 64 each) x kWC (tokens) x 2
-// (sub-block parity) grid: wave (wi, wj, kh) multiplies rows wi .. wi+63 with tokens
-// wj .. wj+kWTok-1 over sub-block kh of every 64-wide K step (the step's sub-blocks 2ks and
-// 2ks + 1); the two parities are summed through LDS at the end.  All threads load and
-// convert the step's weights and activations once into LDS: thread t owns weight row /
-// token t / kParts and part t % kParts (kVP values) of the step.
-#ifndef MNEMO_GEMM_THREADS
-#define MNEMO_GEMM_THREADS 512
-#endif
-constexpr int kThreads = MNEMO_GEMM_THREADS;  // 512 or 1024
-constexpr int kWaves = kThreads / 64;
-constexpr int kBM = 128, kBN = 128;
-constexpr int kKS = 64;                // K per step
-constexpr int kWC = kWaves / 4;        // token groups
-constexpr int kWTok = kBN / kWC;       // tokens per wave
-constexpr int kNB = kWTok / 16;        // 16-token MFMA columns per wave
-constexpr int kParts = kThreads / 128; // loader parts per row and step
-constexpr int kVP = kKS / kParts;      // values per part (16 or 8)
-static_assert(kVP == 8 || kVP == 16, "loader parts of 8 or 16 values");
-// raw ring slots: loads run kPF-2 steps ahead of their conversion
-#ifndef MNEMO_GEMM_PF
-#define MNEMO_GEMM_PF 3
-#endif
-constexpr int kPF = MNEMO_GEMM_PF;
-// lcm(kPF, 3 LDS stages, 4 steps per super-block): every ring slot, stage and super-block
-// boundary of the unrolled loop is a compile-time constant
-constexpr int kUnroll = 12;
-static_assert(kUnroll % kPF == 0, "ring size must divide the unroll");
+// A workgroup is RG x KS waves.  Wave (rg, ks) multiplies R 16-row weight tiles (their operands
+// converted in its own registers) with the workgroup's 16 NB tokens over slice ks of K (whole
+// super-blocks); the slices meet through LDS at the end.  So a weight is converted once per
+// token tile, no wave waits for another's weights, and the only shared operand is the
+// activation tile: the RG waves of a slice turn the Q8_1 rows of a 64-value stage into f16 in
+// LDS, one stage ahead of the multiplication (double-buffered; the raw bytes one stage
+// earlier still, in registers).
+//
+// What bounds it: the issue rate of a wave (one instruction per ~4.8 cycles, two waves per SIMD)
+// and what a stage serialises: per stage of the 256 x 128 shape ~1900 of ~3300 cycles multiply
+// (30 per MFMA with its four rescales), the rest is the conversion and the barrier.  Everything
+// that a stage or window waited for was moved out of it: the Q4_K min term's operands come from
+// LDS (read from memory at each window's end they cost 8 400 cycles per window), the conversion
+// of the next stage sits in front of the multiplication in the same basic block (so the two
+// interleave), addresses are scalars plus constants.  M = 8192, K = 4096, N = 512: 81.4 -> 64 us
+// (540 TOPS); M = 4096, K = 8192, N = 1999: 319 -> 200 us (670 TOPS); N = 7: 25.5 -> 12 us, with
+// the tiled kernel before (128 x 128 tiles, operands of both sides through LDS, K split over
+// workgroups by atomics) on the left.
+constexpr int kStageK = 64;  // K per stage
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
-// kVP raw bytes as dwords
-struct PartBytes {
-    uint32_t w[kVP / 4];
-};
-__device__ __forceinline__ PartBytes ld_part(const uint8_t *p) {
-    PartBytes r;
-    if constexpr (kVP == 16) {
-        const uint4 v = ld16(p);
-        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
-    } else {
-        const uint2 v = ld8(p);
-        r.w[0] = v.x; r.w[1] = v.y;
-    }
-    return r;
-}
-__device__ __forceinline__ PartBytes ld_part_a2(const uint8_t *p) {
-    PartBytes r;
-    if constexpr (kVP == 16) {
-        const uint4 v = ld16_a2(p);
-        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
-    } else {
-        const uint2 v = ld8_a2(p);
-        r.w[0] = v.x; r.w[1] = v.y;
-    }
-    return r;
-}
-
-struct RawW {
-    uint4 h;         // Q4_K: the super-block header (d, dmin, 12 scale bytes)
-    PartBytes a, b;  // Q4_K: a = qs bytes;  Q6_K: a = ql bytes, b = qh bytes
-    uint32_t s, dd;  // Q6_K: the int8 scale of the values, f16 d
-};
-struct RawA {
-    PartBytes q;  // int8 quants
-    uint32_t ds;  // half2 (d8, ds) of their 32-value sub-block
+template <int TYPE, int R, int RG, int KS, int NB>
+struct GemmLds {
+    static constexpr int kPer = R * NB * 4 * 64;  // floats of a wave's accumulators
+    union {
+        _Float16 b[KS][2][NB * 16 * kStageK];  // q8 of a stage's tokens, chunks XOR-swizzled (b_off)
+        float red[KS > 1 ? kPer * RG : 1];  // after the loop: a slice's sums, lane-minor
+    };
+    float rho[KS][2][2][NB * 16];  // token scale ratios of the stage's sub-blocks
+    float unit[KS][2][NB * 16];    // the tokens' d8 units at the end of the window (two windows)
+    // Q4_K: the f16 ds of the tokens' sub-blocks in the current window and the next
+    uint16_t ds[TYPE == kTypeQ4K ? KS : 1][2][NB * 16][32];
+    // .. and a lane's packed mins and dmin of the window's block 4 w + q, by row tile
+    u4v mins[TYPE == kTypeQ4K ? RG * KS : 1][R][64];
 };
 
-// Part p of step ks covers K columns kVP*p .. +kVP-1 of the step: sub-block 2(ks%4) + c/32 of
-// super-block ks/4, positions c%32 .. (c = kVP*p).
-// Q4_K: qs bytes 32(ks%4) + c%32 .., the low (c < 32) or high nibbles.
-__device__ __forceinline__ void load_w_q4k(const uint8_t *__restrict__ wrow, int ks, int p, RawW &r) {
-    const uint8_t *blk = wrow + (size_t)(ks >> 2) * kQ4KBytes;
-    r.h = ld16(blk);
-    r.a = ld_part(blk + 16 + 32 * (ks & 3) + ((kVP * p) & 31));
-}
-// Q6_K: values v0 = 64(ks%4) + c of the super-block: half hh = (ks%4)/2, group
-// grp = 2(ks%2) + c/32, positions l0 = c%32: ql bytes 64hh + 32(grp%2) + l0 (high nibbles if
-// grp >= 2), qh bytes 32hh + l0 at bit 2grp, scale byte 8hh + 2grp + l0/16.
-__device__ __forceinline__ void load_w_q6k(const uint8_t *__restrict__ wrow, int ks, int p, RawW &r) {
-    const uint8_t *blk = wrow + (size_t)(ks >> 2) * kQ6KBytes;
-    const int c = kVP * p, hh = (ks & 3) >> 1, grp = 2 * (ks & 1) + (c >> 5), l0 = c & 31;
-    r.a = ld_part_a2(blk + 64 * hh + 32 * (grp & 1) + l0);
-    r.b = ld_part_a2(blk + 128 + 32 * hh + l0);
-    uint8_t sc;
-    uint16_t dd;
-    __builtin_memcpy(&sc, blk + 192 + 8 * hh + 2 * grp + (l0 >> 4), 1);
-    __builtin_memcpy(&dd, blk + 208, 2);
-    r.s = sc;
-    r.dd = dd;
-}
-// Activations of step ks, part p: values 64ks + kVP*p .. of the token's Q8_1 MMQ row
-// (block v/128, sub-block (v/32)%4).
-__device__ __forceinline__ void load_a(const uint8_t *__restrict__ arow, int ks, int p, RawA &r) {
-    const int v0 = ks * kKS + kVP * p;
-    const uint8_t *blk = arow + (size_t)(v0 >> 7) * kQ81Bytes;
-    __builtin_memcpy(&r.ds, blk + 4 * ((v0 >> 5) & 3), 4);
-    r.q = ld_part(blk + 16 + (v0 & 127));
-}
+// f16 rows of 64 K-columns = 8 chunks of 16 B (a row is 128 B, half of the 64 x 4 B LDS banks),
+// stored without padding with the chunk index XOR-ed by (row / 2) % 8: the 16 rows of an MFMA
+// fragment read (one chunk each) cover the 64 banks once
+__device__ __forceinline__ int b_off(int row, int chunk) { return row * kStageK + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
-// f16 tiles of 64 K-columns per row = 8 chunks of 16 B (a row is 128 B, half of the 64 x 4 B
-// LDS banks), stored without padding with the chunk index XOR-ed by (row / 2) % 8: the 16
-// rows of an MFMA fragment read (one chunk each) cover the 64 banks once, and so do the
-// lanes of a conversion store.
-__device__ __forceinline__ int tile_off(int row, int chunk) { return row * kKS + ((chunk ^ ((row >> 1) & 7)) << 3); }
-// the part's converted values (kVP / 2 dwords of f16 pairs) into its chunks
-__device__ __forceinline__ void put_part(_Float16 *tile, int row, int p, const uint32_t (&o)[kVP / 2]) {
-#pragma unroll
-    for (int c = 0; c < kVP / 8; c++)
-        *(uint4 *)(tile + tile_off(row, (kVP / 8) * p + c)) = make_uint4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);
-}
-
-// One LDS stage: the step's operand tiles and the running-scale factors.
-template <int TYPE>
-struct Stage {
-    static constexpr int kPlanes = TYPE == kTypeQ4K ? 1 : 2;
-    _Float16 a[kPlanes][kBM * kKS];  // weights: sc*q (Q4_K) or the two Q6_K planes
-    _Float16 b[kBN * kKS];           // q8
-    float rho[2][kBN];               // token scale ratio of sub-block 2ks + p
-    float sig[kBM];                  // row scale ratio (written at super-block starts)
-};
-
-// Running scales of a loader thread: the last nonzero d of its weight row (part 0 threads)
-// and the last nonzero d8 of its token for the sub-block parity of its part (the first part
-// of each sub-block).  Both start at 1.
-struct LoaderState {
-    float deff, d8eff;
-};
-
-__device__ __forceinline__ void row_scale_step(float d, int ks, int p, float *sig, int row, LoaderState &ls, bool live) {
-    if (p == 0 && (ks & 3) == 0 && live) {  // super-block start: the row scale changes
-        const float dn = d != 0.0f ? d : ls.deff;
-        sig[row] = ls.deff * __builtin_amdgcn_rcpf(dn);
-        ls.deff = dn;
-    }
-}
-
-__device__ __forceinline__ void store_w_q4k(const RawW &r, int ks, int p, Stage<kTypeQ4K> &st, int row,
-                                            LoaderState &ls, bool live) {
-    const int c = kVP * p;
-    const int j = 2 * (ks & 3) + (c >> 5);
-    uint32_t sc, m;
-    q4k_scale_min(r.h.y, r.h.z, r.h.w, j, sc, m);
-    const float d = h2f(r.h.x & 0xFFFFu);
-    if (d == 0.0f) sc = 0;  // the block's products are zero
-    // the pair (sc, -1024 sc) from sc under the 0x64 exponent; high nibbles are taken in
-    // place as the bytes 16 q with (sc / 16, -64 sc): (1024 + 16 q) sc / 16 - 64 sc = q sc
-    const bool hi = (c >> 5) != 0;
-    const h2 F = hi ? h2{(_Float16)0.0625f, (_Float16)0.0625f} : h2{(_Float16)1.0f, (_Float16)1.0f};
-    const h2 mk = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const h2 S = __builtin_elementwise_fma(magic_pair(sc, 0x04000400u), F, F * mk);
-    const h2 N = S * mk;
-    const uint32_t msk = hi ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-    uint32_t o[kVP / 2];
-#pragma unroll
-    for (int k = 0; k < kVP / 4; k++) {
-        const uint32_t w = r.a.w[k] & msk;
-        o[2 * k] = q4_scaled(w, kSelLo, S, N);
-        o[2 * k + 1] = q4_scaled(w, kSelHi, S, N);
-    }
-    put_part(st.a[0], row, p, o);
-    row_scale_step(d, ks, p, st.sig, row, ls, live);
-}
-
-// Q6_K planes (sc - b)(q - 32) and b(q - 32), b = sc & 1
-__device__ __forceinline__ void store_w_q6k(const RawW &r, int ks, int p, Stage<kTypeQ6K> &st, int row,
-                                            LoaderState &ls, bool live) {
-    const int c = kVP * p, grp = 2 * (ks & 1) + (c >> 5);
-    const float d = h2f(r.dd);
-    int sc = (int)(int8_t)(r.s & 0xFF);
-    if (d == 0.0f) sc = 0;
-    const int b1 = sc & 1;
-    const _Float16 e = (_Float16)(float)(sc - b1), bb = (_Float16)(float)b1;
-    const h2 E = {e, e}, B = {bb, bb};
-    const int shl = grp >= 2 ? 4 : 0;
-    uint32_t o1[kVP / 2], o2[kVP / 2];
-#pragma unroll
-    for (int k = 0; k < kVP / 4; k++) {
-        const uint32_t lo = (r.a.w[k] >> shl) & 0x0F0F0F0Fu;
-        const uint32_t qh = r.b.w[k];
-        const uint32_t hi = (2 * grp <= 4 ? (qh << (4 - 2 * grp)) : (qh >> (2 * grp - 4))) & 0x30303030u;
-        const uint32_t v = lo | hi;
-        const h2 c0 = q6_centered(v, kSelLo), c1 = q6_centered(v, kSelHi);
-        o1[2 * k] = h2u(c0 * E);
-        o1[2 * k + 1] = h2u(c1 * E);
-        o2[2 * k] = h2u(c0 * B);
-        o2[2 * k + 1] = h2u(c1 * B);
-    }
-    put_part(st.a[0], row, p, o1);
-    put_part(st.a[1], row, p, o2);
-    row_scale_step(d, ks, p, st.sig, row, ls, live);
-}
-
-template <int TYPE>
-__device__ __forceinline__ void store_a(const RawA &r, int p, Stage<TYPE> &st, int row, LoaderState &ls, bool live) {
-    const float d8 = h2f(r.ds & 0xFFFFu);
-    const bool zero = d8 == 0.0f;  // x = 0 * q8 = 0 whatever the quants hold (a block whose d
-                                   // rounds to f16 zero keeps quants up to +-127)
-    uint32_t o[kVP / 2];
-#pragma unroll
-    for (int k = 0; k < kVP / 4; k++) q8x4_exact(zero ? 0u : r.q.w[k], o[2 * k], o[2 * k + 1]);
-    put_part(st.b, row, p, o);
-    const int c = kVP * p;
-    if ((c & 31) == 0 && live) {  // first part of a sub-block: its token scale ratio
-        const float dn = zero ? ls.d8eff : d8;
-        st.rho[c >> 5][row] = ls.d8eff * __builtin_amdgcn_rcpf(dn);
-        ls.d8eff = dn;
-    }
-}
-
-template <int TYPE>
-__device__ __forceinline__ void load_step(const uint8_t *wrow, const uint8_t *arow, int ks, int p, RawW &rw,
-                                          RawA &ra) {
-    if (TYPE == kTypeQ4K) load_w_q4k(wrow, ks, p, rw);
-    else load_w_q6k(wrow, ks, p, rw);
-    load_a(arow, ks, p, ra);
-}
-template <int TYPE>
-__device__ __forceinline__ void store_step(const RawW &rw, const RawA &ra, int ks, int p, Stage<TYPE> &st, int row,
-                                           LoaderState &ls, bool live) {
-    if constexpr (TYPE == kTypeQ4K) store_w_q4k(rw, ks, p, st, row, ls, live);
-    else store_w_q6k(rw, ks, p, st, row, ls, live);
-    store_a<TYPE>(ra, p, st, row, ls, live);
-}
-
-// A wave's operands of one step: fragments of its sub-block (kh) for 4 x kNB MFMA tiles, the
-// token scale ratios of its 16-token columns, and (at super-block starts) the row ratios of
-// the rows its accumulators hold.
-template <int TYPE>
-struct Frags {
-    h8 a[Stage<TYPE>::kPlanes][4];
-    h8 b[kNB];
-    float rho[kNB];
-};
-template <int TYPE>
-__device__ __forceinline__ void read_frags(const Stage<TYPE> &st, int wi, int wj, int kh, int lane, Frags<TYPE> &f) {
-    const int chunk = 4 * kh + (lane >> 4);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const int ra = wi + 16 * t + (lane & 15);
-#pragma unroll
-        for (int p = 0; p < Stage<TYPE>::kPlanes; p++) f.a[p][t] = *(const h8 *)(st.a[p] + tile_off(ra, chunk));
-    }
-#pragma unroll
-    for (int t = 0; t < kNB; t++) {
-        const int rb = wj + 16 * t + (lane & 15);
-        f.b[t] = *(const h8 *)(st.b + tile_off(rb, chunk));
-        f.rho[t] = st.rho[kh][rb];
-    }
-}
-
-// acc = acc * rho, then the MFMA adds the step's exact products to the rescaled accumulator
-// (rounded as fp32 sums onto it)
-// (at a super-block start the row ratios come first, read from the step's own stage, which
-// no thread writes during the step)
-template <int TYPE>
-__device__ __forceinline__ void mfma_step(const Frags<TYPE> &f, const Stage<TYPE> &st, int wi, int lane,
-                                          f4 (&acc)[4][kNB], bool sb_start) {
-    if (sb_start) {
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const f4 sg = *(const f4 *)(st.sig + wi + 16 * a + 4 * (lane >> 4));
-#pragma unroll
-            for (int b = 0; b < kNB; b++) acc[a][b] *= sg;
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < kNB; b++) {
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            acc[a][b] *= f.rho[b];
-            acc[a][b] = mfma(f.a[0][a], f.b[b], acc[a][b]);
-            if constexpr (TYPE == kTypeQ6K) acc[a][b] = mfma(f.a[1][a], f.b[b], acc[a][b]);
-        }
-    }
+// a / b to within an ulp of the quotient (the plain product with the reciprocal where that is
+// not finite)
+__device__ __forceinline__ float ratio(float a, float b) {
+    const float r = __builtin_amdgcn_rcpf(b), q = a * r;
+    const float e = __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+    return e == e ? e : q;
 }
 
 struct GemmArgs {
     const uint8_t *W;  // weights [M][K]
     const uint8_t *A;  // Q8_1 MMQ rows [N]
     float *out;
-    int M, K, N, splits;
-    int out_ld;
+    int M, K, N;
 };
 
-template <int TYPE, bool ATOMIC>
-__global__ void __launch_bounds__(kThreads) gemm_q8_1_kernel(GemmArgs g) {
-    __shared__ __align__(16) Stage<TYPE> lds[3];
-    __shared__ float dlast[kBM], d8last[2][kBN];
-    // Q4_K min term: the operands of the split's super-blocks (up to kMhSb), kept as the
-    // loaders pass them -- per weight row and super-block the 8 six-bit mins (one byte each)
-    // and dmin, per token and sub-block the f16 ds of its Q8_1 block
-    constexpr int kMhSb = 16;
-    constexpr int kQ4 = TYPE == kTypeQ4K;
-    __shared__ uint2 mhm[kQ4 ? kBM * kMhSb : 1];
-    __shared__ uint16_t mhd[kQ4 ? kBM * kMhSb : 1];
-    __shared__ __align__(16) uint16_t dsk[kQ4 ? kBN * kMhSb * 8 : 8];
-    const int tid = threadIdx.x;
-    // the wave index as a scalar, so that every per-wave decision below is a scalar branch
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int K = g.K;
-    const int wi = (wave & 1) * 64, wj = ((wave >> 1) % kWC) * kWTok, kh = wave / (2 * kWC);
-    const int bbytes = TYPE == kTypeQ4K ? kQ4KBytes : kQ6KBytes;
-    const size_t wrow_bytes = (size_t)(K / 256) * bbytes;
-    // this split's super-blocks [sb0, sb1) = steps [ks0, ks1)
-    const int nsb = K / 256;
-    const int sb0 = (int)((long)nsb * blockIdx.z / g.splits), sb1 = (int)((long)nsb * (blockIdx.z + 1) / g.splits);
-    const int ks0 = 4 * sb0, ks1 = 4 * sb1, last = ks1 - 1;
-    const int i0 = blockIdx.x * kBM, j0 = blockIdx.y * kBN;
+// Loads at a uniform base + a uniform offset + a lane's 32-bit offset (no 64-bit address per
+// lane and load: those took 20 registers and as many VALU operations per stage)
+struct Buf {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ explicit Buf(const uint8_t *p)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 0xFFFFFFFF, 0x00020000)) {}
+    __device__ __forceinline__ uint2 ld8(uint32_t lane, uint32_t uni) const {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, lane, uni, 0));
+    }
+    __device__ __forceinline__ uint4 ld16(uint32_t lane, uint32_t uni) const {
+        return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, lane, uni, 0));
+    }
+    __device__ __forceinline__ uint32_t ld2(uint32_t lane, uint32_t uni) const {
+        return __builtin_amdgcn_raw_buffer_load_b16(r, lane, uni, 0);
+    }
+};
 
-    // loader role: thread -> (row / token lr, part lp); rows past the end re-read the last
-    const int lr = tid / kParts, lp = tid % kParts;
-    const uint8_t *wrow = g.W + (size_t)min(i0 + lr, g.M - 1) * wrow_bytes;
-    const uint8_t *arow = g.A + (size_t)min(j0 + lr, g.N - 1) * (K / 128) * kQ81Bytes;
-    LoaderState ls{1.0f, 1.0f};
+// LDS accesses at a lane's byte address plus a constant (an offset of the instruction): the
+// address is hidden from the compiler, which otherwise keeps one sum per row in registers
+template <typename T>
+__device__ __forceinline__ T lds_get(uint32_t addr, uint32_t off) {
+    return *(__attribute__((address_space(3))) const T *)(uintptr_t)(addr + off);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(uint32_t addr, uint32_t off, T v) {
+    *(__attribute__((address_space(3))) T *)(uintptr_t)(addr + off) = v;
+}
 
-    f4 acc[4][kNB];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < kNB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-
-    // Pipeline: three LDS stages.  In step ks a wave multiplies the fragments of step ks
-    // (read during step ks-1), reads the fragments of step ks+1 (its stage was completed
-    // before the previous barrier), converts step ks+2 into the third stage, then meets
-    // the barrier.  Raw blocks sit in a ring of kPF register slots, loaded kPF-2 steps
-    // before their conversion.  Conversions past the last step fill idle stages and leave
-    // the running scales alone.
-    RawW rw[kPF];
-    RawA ra[kPF];
-#pragma unroll
-    for (int p = 0; p < kPF; p++) load_step<TYPE>(wrow, arow, min(ks0 + p, last), lp, rw[p], ra[p]);
-    const bool keep_min = TYPE == kTypeQ4K && sb1 - sb0 <= kMhSb;  // uniform
-    // step q (relative to ks0) of the split: the loader of a row's first part keeps its mins
-    // and dmin at the super-block's first step, the loader of a sub-block's first values its ds
-    auto keep = [&](const RawW &w, const RawA &a, int q, bool first_step, bool live) {
-        if (!keep_min || !live) return;
-        if (lp == 0 && first_step) {
-            mhm[lr * kMhSb + (q >> 2)] = q4k_mins(w.h);
-            mhd[lr * kMhSb + (q >> 2)] = (uint16_t)(w.h.x >> 16);
+// The lane's raw weights of one super-block of its row: the quants of the four sub-block pairs
+// are replaced by the next block's as soon as a pair's operands are formed, the header is held
+// for this block and the next
+template <int TYPE>
+struct RawW;
+template <>
+struct RawW<kTypeQ4K> {
+    Raw4 r;
+    // u: the block's offset, o: the lane's row
+    __device__ __forceinline__ void load_pair(const Buf &w, uint32_t u, uint32_t o, int q, int p) {
+        r.a[p] = w.ld8(o + 8 * q, u + 16 + 32 * p);
+    }
+    __device__ __forceinline__ void load_head(const Buf &w, uint32_t u, uint32_t o) { r.h = w.ld16(o, u); }
+    // from here on (nothing is formed from the loads before this point: the compiler would wait
+    // for them there)
+    __device__ __forceinline__ void pin_pair(int p) { asm volatile("" : "+v"(r.a[p].x), "+v"(r.a[p].y)); }
+    __device__ __forceinline__ void next_head() {
+        asm volatile("" : "+v"(r.h.x), "+v"(r.h.y), "+v"(r.h.z), "+v"(r.h.w));
+    }
+    __device__ __forceinline__ uint32_t d_bits() const { return r.h.x & 0xFFFFu; }
+};
+template <>
+struct RawW<kTypeQ6K> {
+    Raw6 r;
+    uint4 sc;
+    uint32_t d;
+    // pairs 2H, 2H + 1 share qh; pair p = 2H + u holds the nibbles u of both ql groups
+    __device__ __forceinline__ void load_pair(const Buf &w, uint32_t u, uint32_t o, int q, int p) {
+        if (p & 1) {  // both pairs of half H are formed
+            const int H = p >> 1;
+            r.ql[2 * H] = w.ld8(o + 8 * q, u + 64 * H);
+            r.ql[2 * H + 1] = w.ld8(o + 8 * q, u + 64 * H + 32);
+            r.qh[H] = w.ld8(o + 8 * q, u + 128 + 32 * H);
         }
-        if (((kVP * lp) & 31) == 0)
-            dsk[lr * kMhSb * 8 + (q >> 2) * 8 + 2 * (q & 3) + ((kVP * lp) >> 5)] = (uint16_t)(a.ds >> 16);
-    };
-    store_step<TYPE>(rw[0], ra[0], ks0, lp, lds[0], lr, ls, true);
-    keep(rw[0], ra[0], 0, true, true);
-    store_step<TYPE>(rw[1], ra[1], ks0 + 1, lp, lds[1], lr, ls, ks0 + 1 < ks1);
-    keep(rw[1], ra[1], 1, false, ks0 + 1 < ks1);
-    lds_barrier();
-    Frags<TYPE> fr;
-    read_frags<TYPE>(lds[0], wi, wj, kh, lane, fr);
+    }
+    __device__ __forceinline__ void load_head(const Buf &w, uint32_t u, uint32_t o) {
+        sc = w.ld16(o, u + 192);
+        d = w.ld2(o, u + 208);
+    }
+    __device__ __forceinline__ void pin_pair(int p) {
+        const int H = p >> 1;
+        if (!(p & 1))
+            asm volatile("" : "+v"(r.ql[2 * H].x), "+v"(r.ql[2 * H].y), "+v"(r.ql[2 * H + 1].x), "+v"(r.ql[2 * H + 1].y),
+                         "+v"(r.qh[H].x), "+v"(r.qh[H].y));
+    }
+    uint32_t dc;
+    __device__ __forceinline__ void next_head(int q) {
+        asm volatile("" : "+v"(sc.x), "+v"(sc.y), "+v"(sc.z), "+v"(sc.w), "+v"(d));
+        // of the 16 scale bytes the lane needs 8H + 2grp + q/2
+        const uint32_t sel = 0x06040200u + 0x01010101u * (uint32_t)(q >> 1);
+        r.sc[0] = __builtin_amdgcn_perm(sc.y, sc.x, sel);
+        r.sc[1] = __builtin_amdgcn_perm(sc.w, sc.z, sel);
+        dc = d;
+    }
+    __device__ __forceinline__ uint32_t d_bits() const { return dc; }
+};
 
-    for (int kb = ks0; kb < ks1; kb += kUnroll) {
+template <int TYPE, int R, int RG, int KS, int NB>
+__global__ void __launch_bounds__(64 * RG * KS) __attribute__((amdgpu_waves_per_eu(R * NB <= 4 ? 4 : 2)))
+gemm_q8_1_kernel(GemmArgs g) {
+    using Lds = GemmLds<TYPE, R, RG, KS, NB>;
+    constexpr bool Q4 = TYPE == kTypeQ4K;
+    constexpr int kTok = NB * 16;
+    constexpr int kBlk = Q4 ? kQ4KBytes : kQ6KBytes;
+    __shared__ __align__(16) Lds L;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave % RG, ks = wave / RG, q = lane >> 4, c = lane & 15;
+    const int nsb = g.K / 256;
+    const int sb0 = nsb * ks / KS, n = nsb * (ks + 1) / KS - sb0;  // the slice's super-blocks
+    const int nmax = (nsb + KS - 1) / KS;                          // .. at most this many in any slice
+    const int i0 = (blockIdx.x * RG + rg) * 16 * R, j0 = blockIdx.y * kTok;
+
+    // the lane's weight rows (rows past the end re-read the last): byte offsets from the workgroup's
+    // first row
+    const uint32_t wrow = (uint32_t)nsb * kBlk;
+    const int iw = blockIdx.x * RG * 16 * R;
+    const Buf wb(g.W + (size_t)iw * wrow + (size_t)sb0 * kBlk);
+    uint32_t wo[R];
 #pragma unroll
-        for (int p = 0; p < kUnroll; p++) {
-            const int ks = kb + p;
-            if (ks < ks1) {  // uniform
-                // kb - ks0 is a multiple of kUnroll and ks0 of 4, so these are compile-time
-                // constants
-                const int r = p % kPF, b = p % 3;
-                load_step<TYPE>(wrow, arow, min(ks + kPF, last), lp, rw[r], ra[r]);
-                mfma_step<TYPE>(fr, lds[b], wi, lane, acc, p % 4 == 0);
-                read_frags<TYPE>(lds[(b + 1) % 3], wi, wj, kh, lane, fr);
-                store_step<TYPE>(rw[(r + 2) % kPF], ra[(r + 2) % kPF], ks + 2, lp, lds[(b + 2) % 3], lr, ls,
-                                 ks + 2 < ks1);
-                // (ks + 2 - ks0) % 4 == (p + 2) % 4: a compile-time test
-                keep(rw[(r + 2) % kPF], ra[(r + 2) % kPF], ks + 2 - ks0, ((p + 2) & 3) == 0, ks + 2 < ks1);
+    for (int a = 0; a < R; a++) wo[a] = (uint32_t)(min(i0 + 16 * a + c, g.M - 1) - iw) * wrow;
+    // loader role in the slice: thread -> token lt, values VP lp .. of each stage
+    constexpr int VP = NB * 16 * kStageK / (64 * RG) < 8 ? 8 : NB * 16 * kStageK / (64 * RG);
+    constexpr int PT = kStageK / VP;  // threads per token
+    const int ltid = rg * 64 + lane, lt = ltid / PT, lp = ltid % PT;
+    const bool loader = kTok * PT >= 64 * RG || lt < kTok;
+    const Buf ab(g.A + ((size_t)j0 * (g.K / 128) + 2 * sb0) * kQ81Bytes);  // the tile's first token
+    const uint32_t ao = (uint32_t)(min(j0 + min(lt, kTok - 1), g.N - 1) - j0) * (uint32_t)(g.K / 128) * kQ81Bytes;
+    struct RawA {
+        uint32_t v[VP / 4];
+        uint2 hd;  // (d8, ds) of the stage's two sub-blocks
+    };
+    auto load_a = [&](int t, RawA &r) {  // stage t of the slice
+        const uint32_t u = (uint32_t)(t >> 1) * kQ81Bytes;
+        r.hd = ab.ld8(ao, u + 8 * (t & 1));
+        const uint32_t p = u + 64 * (t & 1);
+        if constexpr (VP == 8) {
+            const uint2 v = ab.ld8(ao + VP * lp, p + 16);
+            r.v[0] = v.x; r.v[1] = v.y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < VP / 16; i++) {
+                const uint4 v = ab.ld16(ao + VP * lp, p + 16 + 16 * i);
+                r.v[4 * i] = v.x; r.v[4 * i + 1] = v.y; r.v[4 * i + 2] = v.z; r.v[4 * i + 3] = v.w;
+            }
+        }
+    };
+    // LDS addresses: the lane's fragment chunks of both sub-blocks of a stage, its token column's
+    // ratios, the chunks and ratios that it writes
+    const uint32_t lds = lds_addr(&L);
+    const uint32_t kRow = kStageK * 2, kBuf = kTok * kRow;  // bytes of a row, of a buffer
+    const uint32_t lb = lds + offsetof(Lds, b) + (uint32_t)ks * 2 * kBuf;
+    const uint32_t lr = lds + offsetof(Lds, rho) + (uint32_t)ks * 4 * kTok * 4;
+    const uint32_t ld = lds + offsetof(Lds, ds) + (uint32_t)ks * 2 * kTok * 64;
+    uint32_t wd = ld + 64 * lt, dq = ld + 64 * c + 16 * q;  // ds: written, and the lane's window operand
+    uint32_t wu = lds + offsetof(Lds, unit) + ((uint32_t)ks * 2 * kTok + lt) * 4;
+    uint32_t mn0 = lds + offsetof(Lds, mins) + (uint32_t)wave * R * 1024 + 16 * lane;
+    uint32_t fr[2], rr0 = lr + 4 * c, wr = lr + 4 * lt, wc[VP / 8 > 0 ? VP / 8 : 1];
+#pragma unroll
+    for (int jj = 0; jj < 2; jj++) fr[jj] = lb + 2 * b_off(c, 4 * jj + q);
+#pragma unroll
+    for (int i = 0; i < VP / 8; i++) wc[i] = lb + 2 * b_off(lt, VP / 8 * lp + i);
+    asm volatile("" : "+v"(fr[0]), "+v"(fr[1]), "+v"(rr0), "+v"(wr), "+v"(mn0), "+v"(wd), "+v"(dq), "+v"(wu));
+#pragma unroll
+    for (int i = 0; i < VP / 8; i++) asm volatile("" : "+v"(wc[i]));
+    float unit = 1.0f;  // the token's running d8 (1 at a window's start, unchanged by d8 = 0)
+    auto convert_a = [&](int t, RawA &r, int buf) {
+#pragma unroll
+        for (int i = 0; i < VP / 4; i++) asm volatile("" : "+v"(r.v[i]));  // pins, as RawW's
+        asm volatile("" : "+v"(r.hd.x), "+v"(r.hd.y));
+        const float d0 = h2f(r.hd.x & 0xFFFFu), d1 = h2f(r.hd.y & 0xFFFFu);
+        if ((t & 15) == 0) unit = 1.0f;
+        const float c0 = d0 != 0.0f ? d0 : unit, c1 = d1 != 0.0f ? d1 : c0;
+        if (loader) {
+            // the PT threads of a token write the same values
+            lds_put<float>(wr, buf * 2 * kTok * 4, ratio(unit, c0));
+            lds_put<float>(wr, (buf * 2 + 1) * kTok * 4, ratio(c0, c1));
+            lds_put<float>(wu, ((t >> 4) & 1) * kTok * 4, c1);
+            if constexpr (Q4)
+                lds_put<uint32_t>(wd, ((t >> 4) & 1) * kTok * 64 + (t & 15) * 4,
+                                  __builtin_amdgcn_perm(r.hd.y, r.hd.x, 0x07060302u));  // the high halves
+#pragma unroll
+            for (int i = 0; i < VP / 8; i++) {
+                const int ch = VP / 8 * lp + i;
+                // a block whose d rounds to f16 zero keeps quants up to +-127: its values are 0 * q8
+                const bool zero = (ch < 4 ? d0 : d1) == 0.0f;
+                uint4 o;
+                q8x4_exact(zero ? 0u : r.v[2 * i], o.x, o.y);
+                q8x4_exact(zero ? 0u : r.v[2 * i + 1], o.z, o.w);
+                lds_put<u4v>(wc[i], buf * kBuf, u4v{o.x, o.y, o.z, o.w});
+            }
+        }
+        unit = c1;
+    };
+
+    f4 acc[R][NB];
+    float deff[R];  // running d of the lane's row of each tile
+#pragma unroll
+    for (int a = 0; a < R; a++) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+        deff[a] = 1.0f;
+    }
+    RawW<TYPE> w[R];
+    RawA ra;
+    if (n > 0) {
+        load_a(0, ra);
+#pragma unroll
+        for (int a = 0; a < R; a++) {
+            w[a].load_head(wb, 0, wo[a]);
+#pragma unroll
+            for (int p = 0; p < 4; p++) w[a].load_pair(wb, 0, wo[a], q, p);
+        }
+        convert_a(0, ra, 0);
+        load_a(1, ra);
+    }
+    lds_barrier();
+
+    for (int k = 0; k < nmax; k++) {
+        if (k < n) {  // wave-uniform (slices differ by one super-block at most)
+            const uint32_t next = (uint32_t)min(k + 1, n - 1) * kBlk;
+#pragma unroll
+            for (int a = 0; a < R; a++) {
+                if constexpr (Q4) w[a].next_head();
+                else w[a].next_head(q);
+                if constexpr (!Q4) w[a].load_head(wb, next, wo[a]);
+                const float d = h2f(w[a].d_bits());
+                if constexpr (Q4) {
+                    if ((k & 3) == q) {
+                        const uint2 mn = q4k_mins(w[a].r.h);
+                        lds_put<u4v>(mn0, a * 1024, u4v{mn.x, mn.y, w[a].r.h.x >> 16, 0u});
+                    }
+                    if (d == 0.0f) w[a].r.h.y = w[a].r.h.w = 0u;  // scales 0: the block's products are zero
+                } else {
+                    if (d == 0.0f) w[a].r.sc[0] = w[a].r.sc[1] = 0u;
+                }
+                // the running row scale: lane c owns row c; the lane's outputs are rows 4q + x
+                const float nd = d == 0.0f ? deff[a] : d;
+                const float sg = ratio(deff[a], nd);
+                deff[a] = nd;
+#pragma unroll
+                for (int x = 0; x < 4; x++) {
+                    const float se = __shfl(sg, 4 * q + x);
+#pragma unroll
+                    for (int b = 0; b < NB; b++) acc[a][b][x] *= se;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const int t = 4 * k + s, buf = s & 1;
+                convert_a(t + 1, ra, buf ^ 1);
+                load_a(min(t + 2, 4 * n - 1), ra);
+                Scales4 s4[R];
+                Scales6 s6[R];
+#pragma unroll
+                for (int jj = 0; jj < 2; jj++) {
+                    h8 bf[NB];
+                    float rr[NB];
+#pragma unroll
+                    for (int b = 0; b < NB; b++) {
+                        rr[b] = lds_get<float>(rr0, ((buf * 2 + jj) * kTok + 16 * b) * 4);
+                        bf[b] = lds_get<h8>(fr[jj], buf * kBuf + 16 * b * kRow);
+                    }
+                    h8 a1[R], a2[R];
+#pragma unroll
+                    for (int a = 0; a < R; a++) {
+                        if (jj == 0) w[a].pin_pair(s);
+                        if constexpr (Q4) {
+                            if (jj == 0) s4[a] = scale_pair4(w[a].r.h, s);
+                            if (jj == 1 && s == 3) w[a].load_head(wb, next, wo[a]);  // the block's last scales are formed
+                            a1[a] = operand4(w[a].r, s4[a], s, jj);
+                        } else {
+                            if (jj == 0) s6[a] = scale_pair6(w[a].r.sc[s >> 1], s);
+                            operand6(w[a].r, s6[a], 2 * s + jj, a1[a], a2[a]);
+                        }
+                        if (jj == 1) w[a].load_pair(wb, next, wo[a], q, s);
+                    }
+#pragma unroll
+                    for (int b = 0; b < NB; b++)
+#pragma unroll
+                        for (int a = 0; a < R; a++) {
+                            acc[a][b] *= rr[b];
+                            acc[a][b] = mfma(a1[a], bf[b], acc[a][b]);
+                            if constexpr (!Q4) acc[a][b] = mfma(a2[a], bf[b], acc[a][b]);
+                        }
+                }
+                if (s == 3 && ((k & 3) == 3 || k == n - 1)) {  // the window's end
+                    // the accumulators become absolute and take the Q4_K min term of the window's 32
+                    // sub-blocks, sum_s -(dmin*m_s)_i * ds_js: lane group q holds super-block 4w + q of its
+                    // row and token (K index 8q + s of the MFMA = sub-block s); groups past the end add
+                    // nothing
+                    const int kw = (k & ~3) + q;
+                    const bool valid = kw < n;
+                    constexpr int NC = NB > 4 ? NB / 2 : NB;  // columns at a time
+                    float dr[R][4];
+#pragma unroll
+                    for (int a = 0; a < R; a++) {
+#pragma unroll
+                        for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
+                        deff[a] = 1.0f;
+                    }
+#pragma unroll
+                    for (int b0 = 0; b0 < NB; b0 += NC) {
+                        float dt[NC];
+                        h8 bd[Q4 ? NC : 1];
+#pragma unroll
+                        for (int b = 0; b < NC; b++) {
+                            dt[b] = L.unit[ks][(k >> 2) & 1][16 * (b0 + b) + c];
+                            if constexpr (Q4) {
+                                bd[b] = lds_get<h8>(dq, ((k >> 2) & 1) * kTok * 64 + 16 * (b0 + b) * 64);
+                                if (!valid) bd[b] = h8{};
+                            }
+                        }
+#pragma unroll
+                        for (int a = 0; a < R; a++) {
+                            h8 hi, lo;
+                            if constexpr (Q4) {
+                                const u4v mn = lds_get<u4v>(mn0, a * 1024);
+                                q4k_min_operand_m(make_uint2(mn.x, mn.y), valid ? mn.z : 0u, hi, lo);
+                            }
+#pragma unroll
+                            for (int b = 0; b < NC; b++) {
+                                f4 &ac = acc[a][b0 + b];
+#pragma unroll
+                                for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
+                                if constexpr (Q4) ac = mfma(lo, bd[b], mfma(hi, bd[b], ac));
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
                 lds_barrier();
             }
-        }
-    }
-    // absolute values: the last nonzero scales of each row and each token (per parity)
-    if (lp == 0) dlast[lr] = ls.deff;
-    if (((kVP * lp) & 31) == 0) d8last[(kVP * lp) >> 5][lr] = ls.d8eff;
-    __syncthreads();
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const f4 dr = *(const f4 *)(dlast + wi + 16 * a + 4 * (lane >> 4));
-#pragma unroll
-        for (int b = 0; b < kNB; b++) {
-            const float dt = d8last[kh][wj + 16 * b + (lane & 15)];
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[a][b][e] *= dr[e] * dt;
+        } else {
+            for (int s = 0; s < 4; s++) lds_barrier();
         }
     }
 
-    // Q4_K min term, sum_s -(dmin*m_s)_i * ds_js, added to the absolute accumulator after
-    // the loop, from the operands the loaders kept in LDS (up to 16 super-blocks per split;
-    // reading the headers and the Q8_1 block heads again from memory touched every weight
-    // line a second time and 4096 activation lines per workgroup).  Windows of 32 sub-blocks
-    // (4 super-blocks), wave parity kh taking windows kh, kh+2, ...; lane group q = lane/16
-    // holds super-block 4w + q of its row / token (K index 8q + s of the MFMA = sub-block s of
-    // that super-block).
-    if constexpr (TYPE == kTypeQ4K) {
-        const int q = lane >> 4;
-        const int nwin = (sb1 - sb0 + 3) / 4;
-        for (int w = kh; w < nwin; w += 2) {
-            const int sb = sb0 + 4 * w + q;
-            const bool valid = sb < sb1;
-            uint4 hdr[4], blk[kNB][2];
-            if (keep_min) {  // the operands the loaders kept: no second pass over weights or activations
-                const int rs = valid ? sb - sb0 : 0;
-                h8 bd[kNB];
+    // the slices' sums meet in slice 0's waves, through the (now idle) stages, lane-minor so that
+    // the accesses are conflict-free
+    if constexpr (KS > 1) {
+        float *red = L.red;
+        constexpr int kPer = Lds::kPer;
+        constexpr int kUnion = sizeof L.b > sizeof L.red ? sizeof L.b : sizeof L.red;
+        constexpr int kFit = kUnion / (int)(sizeof(float) * kPer * RG);  // slices at a time
 #pragma unroll
-                for (int b = 0; b < kNB; b++) {
-                    bd[b] = *(const h8 *)&dsk[(wj + 16 * b + (lane & 15)) * kMhSb * 8 + rs * 8];
-                    if (!valid) bd[b] = h8{};
-                }
+        for (int z0 = 1; z0 < KS; z0 += kFit) {
+            if (z0 > 1) lds_barrier();
+            if (ks >= z0 && ks < z0 + kFit) {
 #pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    const int row = wi + 16 * a + (lane & 15);
-                    h8 hi, lo;
-                    q4k_min_operand_m(mhm[row * kMhSb + rs], valid ? mhd[row * kMhSb + rs] : 0u, hi, lo);
+                for (int a = 0; a < R; a++)
 #pragma unroll
-                    for (int b = 0; b < kNB; b++) acc[a][b] = mfma(lo, bd[b], mfma(hi, bd[b], acc[a][b]));
-                }
-                continue;
+                    for (int b = 0; b < NB; b++)
+#pragma unroll
+                        for (int x = 0; x < 4; x++)
+                            red[((ks - z0) * RG + rg) * kPer + ((a * NB + b) * 4 + x) * 64 + lane] = acc[a][b][x];
             }
+            lds_barrier();
+            if (ks == 0) {
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const uint8_t *rp = g.W + (size_t)min(i0 + wi + 16 * a + (lane & 15), g.M - 1) * wrow_bytes;
-                hdr[a] = valid ? ld16(rp + (size_t)sb * kQ4KBytes) : make_uint4(0, 0, 0, 0);
-            }
+                for (int z = z0; z < KS && z < z0 + kFit; z++)
 #pragma unroll
-            for (int b = 0; b < kNB; b++) {
-                const uint8_t *ap = g.A +
-                                    (size_t)min(j0 + wj + 16 * b + (lane & 15), g.N - 1) * (K / 128) * kQ81Bytes;
-                blk[b][0] = valid ? ld16(ap + (size_t)(2 * sb) * kQ81Bytes) : make_uint4(0, 0, 0, 0);
-                blk[b][1] = valid ? ld16(ap + (size_t)(2 * sb + 1) * kQ81Bytes) : make_uint4(0, 0, 0, 0);
-            }
-            h8 bd[kNB];
+                    for (int a = 0; a < R; a++)
 #pragma unroll
-            for (int b = 0; b < kNB; b++) bd[b] = ds_operand(blk[b][0], blk[b][1]);
+                        for (int b = 0; b < NB; b++)
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                h8 hi, lo;
-                q4k_min_operand(hdr[a], hi, lo);
-#pragma unroll
-                for (int b = 0; b < kNB; b++) acc[a][b] = mfma(lo, bd[b], mfma(hi, bd[b], acc[a][b]));
+                            for (int x = 0; x < 4; x++)
+                                acc[a][b][x] += red[((z - z0) * RG + rg) * kPer + ((a * NB + b) * 4 + x) * 64 + lane];
             }
         }
+        if (ks) return;
     }
-
-    // sum the two parities: the kh = 1 waves hand their tiles to their kh = 0 counterparts
-    // through the (now idle) stages, laid out lane-minor so the accesses are conflict-free
-    __syncthreads();
-    float *red = (float *)&lds[0] + (size_t)(wave % (kWaves / 2)) * (64 * kWTok);
-    if (kh) {
+    // D layout (16x16 f32): lane l holds rows 4*(l/16)+x, column l%16.  Rows index weights (A
+    // operand), columns tokens (B operand).
 #pragma unroll
-        for (int a = 0; a < 4; a++)
+    for (int b = 0; b < NB; b++) {
+        const int j = j0 + 16 * b + c;
+        if (j >= g.N) continue;
+        float *o = g.out + (size_t)j * g.M + i0 + 4 * q;
 #pragma unroll
-            for (int b = 0; b < kNB; b++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) red[((a * kNB + b) * 4 + e) * 64 + lane] = acc[a][b][e];
-    }
-    __syncthreads();
-    if (kh) return;
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < kNB; b++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[a][b][e] += red[((a * kNB + b) * 4 + e) * 64 + lane];
-    // D layout (16x16 f32): lane l holds rows 4*(l/16)+e, column l%16.  Rows index
-    // weights (A operand), columns tokens (B operand).
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < kNB; b++) {
-            const int j = j0 + wj + 16 * b + (lane & 15);
-            const int ib = i0 + wi + 16 * a + 4 * (lane >> 4);
-            if (j >= g.N) continue;
-            float *o = g.out + (size_t)j * g.out_ld + ib;
-            if (ATOMIC) {
-                // to the wave's own (idle) reduction buffer, token-major, 16-byte groups
-                // XOR-swizzled by token so that the row-wise reads below are conflict-free
-                *(f4 *)(red + (16 * b + (lane & 15)) * 64 + (((4 * a + (lane >> 4)) ^ (lane & 15)) << 2)) = acc[a][b];
-            } else if (ib + 3 < g.M && ((g.out_ld & 3) == 0)) {
-                *(f4 *)o = acc[a][b];
+        for (int a = 0; a < R; a++) {
+            const int i = i0 + 16 * a + 4 * q;
+            if (i + 3 < g.M && (g.M & 3) == 0) {
+                *(f4 *)(o + 16 * a) = acc[a][b];
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (ib + e < g.M) o[e] = acc[a][b][e];
+                for (int x = 0; x < 4; x++)
+                    if (i + x < g.M) o[16 * a + x] = acc[a][b][x];
             }
-        }
-    if (ATOMIC) {
-        // one atomic instruction per token covers 64 consecutive outputs (two cache lines);
-        // the MFMA layout would spread each instruction over 16 token rows, which measured
-        // twice as slow in the L2 atomic units
-        const int ib = i0 + wi + lane;
-        for (int t = 0; t < kWTok; t++) {
-            const int j = j0 + wj + t;
-            if (j >= g.N) break;
-            if (ib < g.M)
-                __hip_atomic_fetch_add(g.out + (size_t)j * g.out_ld + ib,
-                                       red[t * 64 + ((((lane >> 2) ^ (t & 15)) << 2) | (lane & 3))], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -550,7 +486,8 @@ __global__ void __launch_bounds__(kThreads) gemm_q8_1_kernel(GemmArgs g) {
 // ------------------------------------------------------------------ activation staging
 // fp32 rows [N][K] -> the grouped kernel's operand form of cuda_quantize_mmq_q8_1's output
 // (per 32 values d = amax/127, q = rint(x*127/amax) clamped to +-127, ds = f16(d * sum x);
-// gemm_q4k.cu:327-358): q8 as f16 integers [N][K], the f16 ds [N][K/32], the running-scale
+// gemm_q4k.cu:327-358): q8 as f16 integers [N][K] in the operands' element order
+// (gemm_ops.hpp), the f16 ds [N][K/32], the running-scale
 // ratio rho_s = d8eff_{s-1} / d8eff_s [N][K/32] and d8eff at the end of every window of 32
 // sub-blocks (1024 values) [N][ceil(K/1024)].  d8eff is the last nonzero f16 d8 at or before s
 // in s's window, 1 before the window's first.  One wave per row.
@@ -588,12 +525,13 @@ __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *_
             float sum = 0.0f;
             uint32_t o[16];
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                float r0 = rintf(xv[2 * i] * id), r1 = rintf(xv[2 * i + 1] * id);
+            for (int i = 0; i < 32; i++) sum += xv[i];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {  // the operands' element order: values 0 2 | 1 3 of each four
+                const int v = 4 * (i / 2) + (i & 1);
+                float r0 = rintf(xv[v] * id), r1 = rintf(xv[v + 2] * id);
                 r0 = fminf(fmaxf(r0, -127.0f), 127.0f);
                 r1 = fminf(fmaxf(r1, -127.0f), 127.0f);
-                sum += xv[2 * i];
-                sum += xv[2 * i + 1];
                 o[i] = h2u(h2{(_Float16)r0, (_Float16)r1});
             }
             float dsum = d * sum;
@@ -628,11 +566,6 @@ int launch_stage_f32(const float *x, int K, int N, StagedAct sa, hipStream_t s) 
     return check_launch("stage_f32");
 }
 
-__global__ void zero_kernel(float4 *__restrict__ p, long n4) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x)
-        p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
 static int device_cus_gemm() {
     static int cus = 0;
     if (!cus) {
@@ -646,6 +579,32 @@ static int device_cus_gemm() {
     return cus;
 }
 
+// The workgroup shapes and what each costs.  A launch of t tiles runs in ceil(t / CUs) rounds (one
+// workgroup per CU: the workgroups are latency-bound, a second one per CU gains nothing), and a
+// round takes c1 us per super-block of a K slice plus c2 us (first loads, the slices' sums,
+// the stores); c0: the launch.  Fitted to 520 sizes (M 512-8192, K 512-8192, N 1-2048, both
+// types; rms 6 %): the choice with the least cost is within 1.3 % of the fastest shape on
+// average and 29 % at worst (Q6_K, K = 1536, a slice per block).
+// Large products take the wide tiles (fewest conversions and LDS reads per MFMA), small ones
+// narrow tiles with K in up to 8 slices, so that the launch still covers the chip.
+struct GemmShape {
+    int r, rg, ks, nb;
+    double q4[3], q6[3];
+};
+#define MNEMO_GEMM_SHAPES(X)                                                      \
+    X(0, 2, 8, 1, 8, {-7.7, 5.82, 14.7}, {-8.3, 9.14, 16.2}) /* 256 x 128 */      \
+    X(1, 2, 4, 2, 8, {-2.5, 6.46, 9.3}, {-3.0, 10.3, 10.5})  /* 128 x 128 */      \
+    X(2, 2, 4, 2, 4, {0.8, 4.46, 4.6}, {0.6, 7.39, 5.5})     /* 128 x 64 */       \
+    X(3, 1, 4, 2, 4, {5.1, 2.84, 0.4}, {4.2, 3.96, 0.9})     /* 64 x 64 */        \
+    X(4, 1, 4, 4, 4, {1.5, 5.40, 1.6}, {1.0, 8.34, 0.1})     /* 64 x 64 */        \
+    X(5, 1, 4, 4, 2, {3.3, 3.96, 0.4}, {2.6, 6.96, -1.0})    /* 64 x 32 */        \
+    X(6, 1, 2, 8, 2, {3.2, 5.40, -0.2}, {3.9, 9.15, -3.6})   /* 32 x 32 */        \
+    X(7, 2, 1, 8, 1, {5.4, 4.16, -1.7}, {5.4, 7.99, -4.5})   /* 32 x 16 */
+#define MNEMO_GEMM_SHAPE(I_, R_, RG_, KS_, NB_, ...) {R_, RG_, KS_, NB_, __VA_ARGS__},
+static const GemmShape kShapes[] = {MNEMO_GEMM_SHAPES(MNEMO_GEMM_SHAPE)};
+
+static int gemm_tiles(int n, int tile) { return (int)(((long)n + tile - 1) / tile); }
+
 int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M, int K, int N,
                      hipStream_t stream) {
     if (!w || !act || !out || M <= 0 || N <= 0 || K <= 0 || K % 256 != 0)
@@ -653,39 +612,35 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
     if (type != kTypeQ4K && type != kTypeQ6K) return set_error(kErrUnsupportedType, "gemm: unsupported type %d", type);
     if (((uintptr_t)out & 15) != 0) return set_error(kErrBadArg, "gemm: output must be 16-byte aligned");
     if (((uintptr_t)act & 3) != 0) return set_error(kErrBadArg, "gemm: activation blocks must be 4-byte aligned");
-    const int tm = (M + kBM - 1) / kBM, tn = (N + kBN - 1) / kBN;
-    // split K (whole super-blocks) while the split grid still fits the CUs once, keeping
-    // at least 2 super-blocks per split
-    const int nsb = K / 256;
-    int splits = 1;
-    while (2 * tm * tn * splits <= device_cus_gemm() && nsb / (splits * 2) >= 2) splits *= 2;
-    if (((long)M * N) % 4 != 0) splits = 1;  // the fill kernel clears float4s
     // activations are read as Q8_1 blocks and converted per tile: nothing is allocated, so
     // the call may sit inside a graph capture
-    GemmArgs g{};
-    g.W = (const uint8_t *)w;
-    g.A = (const uint8_t *)act;
-    g.out = out;
-    g.M = M;
-    g.K = K;
-    g.N = N;
-    g.splits = splits;
-    g.out_ld = M;
-    if (splits > 1) {
-        const long n = (long)M * N;
-        hipLaunchKernelGGL(zero_kernel, dim3((unsigned)std::min<long>((n / 4 + 255) / 256, 4096)), dim3(256), 0,
-                           stream, (float4 *)out, n / 4);
+    const GemmArgs g{(const uint8_t *)w, (const uint8_t *)act, out, M, K, N};
+    const int cus = device_cus_gemm(), nsb = K / 256;
+    int best = 0;
+    double least = 0;
+    for (int i = 0; i < (int)(sizeof kShapes / sizeof kShapes[0]); i++) {
+        const GemmShape &h = kShapes[i];
+        const double *c = type == kTypeQ4K ? h.q4 : h.q6;
+        if (i && gemm_tiles(N, 16 * h.nb) > 65535) continue;  // the grid's second dimension
+        const long tiles = (long)gemm_tiles(M, 16 * h.r * h.rg) * gemm_tiles(N, 16 * h.nb);
+        const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]);
+        if (i == 0 || t < least) {
+            best = i;
+            least = t;
+        }
     }
-    const dim3 grid(tm, tn, splits);
-#define MNEMO_GEMM_LAUNCH(T_, A_) hipLaunchKernelGGL((gemm_q8_1_kernel<T_, A_>), grid, dim3(kThreads), 0, stream, g)
-    if (type == kTypeQ4K) {
-        if (splits > 1) MNEMO_GEMM_LAUNCH(kTypeQ4K, true);
-        else MNEMO_GEMM_LAUNCH(kTypeQ4K, false);
-    } else {
-        if (splits > 1) MNEMO_GEMM_LAUNCH(kTypeQ6K, true);
-        else MNEMO_GEMM_LAUNCH(kTypeQ6K, false);
-    }
-#undef MNEMO_GEMM_LAUNCH
+    const dim3 grid(gemm_tiles(M, 16 * kShapes[best].r * kShapes[best].rg), gemm_tiles(N, 16 * kShapes[best].nb));
+#define MNEMO_GEMM(I_, R_, RG_, KS_, NB_, ...)                                                                   \
+    case I_:                                                                                                     \
+        if (type == kTypeQ4K)                                                                                    \
+            hipLaunchKernelGGL((gemm_q8_1_kernel<kTypeQ4K, R_, RG_, KS_, NB_>), grid, dim3(64 * RG_ * KS_), 0,   \
+                               stream, g);                                                                       \
+        else                                                                                                     \
+            hipLaunchKernelGGL((gemm_q8_1_kernel<kTypeQ6K, R_, RG_, KS_, NB_>), grid, dim3(64 * RG_ * KS_), 0,   \
+                               stream, g);                                                                       \
+        break;
+    switch (best) { MNEMO_GEMM_SHAPES(MNEMO_GEMM) }
+#undef MNEMO_GEMM
     return check_launch("gemm_q8_1");
 }
 

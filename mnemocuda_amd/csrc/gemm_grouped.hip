@@ -91,11 +91,7 @@ __device__ __forceinline__ int gw_unslot(int r, int pc) {  // the chunk stored a
     return SK == 128 ? pc ^ (r & 15) : pc ^ ((r >> 1) & 7);
 }
 
-// Q4_K lane view of a tile's block: the header (d, dmin, scales) and the lane's qs bytes
-struct Raw4 {
-    uint4 h;
-    uint2 a[4];  // qs bytes 32g + 8q .. +7
-};
+// the lane's values of row c of a Q4_K tile in the wave's LDS area
 __device__ __forceinline__ Raw4 read4(const uint8_t *tile, int c, int q) {
     Raw4 r;
     const uint8_t *row = tile + c * kQ4KBytes;
@@ -104,45 +100,6 @@ __device__ __forceinline__ Raw4 read4(const uint8_t *tile, int c, int q) {
     for (int g = 0; g < 4; g++) r.a[g] = *(const uint2 *)(row + 16 + 32 * g + 8 * q);
     return r;
 }
-// the 8 six-bit scales of a Q4_K block as bytes (get_scale_min_k4, kernels.cu:45-53): sub-blocks
-// 0-3 are the low 6 bits of bytes 0-3, 4-7 the low nibbles of bytes 8-11 with bits 6-7 of
-// bytes 0-3 above them (the packed form of gemm_q4k.cu:53-56)
-__device__ __forceinline__ uint32_t scales4(const uint4 &h, int half) {
-    return half == 0 ? h.y & 0x3F3F3F3Fu : (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-}
-// the scales of sub-blocks 4H + g as f16 pairs (g = 0, 1 | 2, 3) and their products with -1024
-// (odd sub-blocks, the high nibbles, are taken in place as bytes 16 q: their pair is
-// (sc / 16, -64 sc), and (1024 + 16 q) * sc / 16 - 64 sc = q * sc in the same exact fma)
-struct Scales4 {
-    h2 s[2], n[2];
-};
-__device__ __forceinline__ Scales4 scale_pairs4(uint32_t sc4) {
-    Scales4 o;
-    const h2 m = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    const h2 f = {(_Float16)1.0f, (_Float16)0.0625f};
-    o.s[0] = (magic_pair(sc4, kSelLo) + m) * f;
-    o.s[1] = (magic_pair(sc4, kSelHi) + m) * f;
-    o.n[0] = o.s[0] * m;
-    o.n[1] = o.s[1] * m;
-    return o;
-}
-// sub-block j's A operand: sc * q for the lane's 8 values
-__device__ __forceinline__ h8 operand4(const Raw4 &r, const Scales4 &T, int j) {
-    const _Float16 sj = T.s[(j & 3) >> 1][j & 1], nj = T.n[(j & 3) >> 1][j & 1];
-    const h2 S = {sj, sj}, N = {nj, nj};
-    const uint2 c = r.a[j >> 1];
-    const uint32_t msk = (j & 1) ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-    const uint32_t w0 = c.x & msk, w1 = c.y & msk;
-    return __builtin_bit_cast(h8, make_uint4(q4_scaled(w0, kSelLo, S, N), q4_scaled(w0, kSelHi, S, N),
-                                             q4_scaled(w1, kSelLo, S, N), q4_scaled(w1, kSelHi, S, N)));
-}
-
-// Q6_K raw bytes of one row tile's lane values for one block
-struct Raw6 {
-    uint2 ql[4];     // ql bytes 64H + 32p + 8q .. +7 (index 2H + p)
-    uint2 qh[2];     // qh bytes 32H + 8q .. +7
-    uint32_t sc[2];  // the lane's scale bytes of halves 0 / 1 (byte grp: scale 8H + 2grp + q/2)
-};
 // the lane's raw values of row c's block from the wave's LDS area (sh: the block's
 // misalignment, 0 or 2 bytes)
 __device__ __forceinline__ Raw6 read6(const uint8_t *area, int c, int q, uint32_t sh) {
@@ -172,37 +129,6 @@ __device__ __forceinline__ Raw6 read6(const uint8_t *area, int c, int q, uint32_
     r.sc[1] = __builtin_amdgcn_perm(sc.w, sc.z, sel);
     return r;
 }
-// the two factors of the lane's 4 scales of half H (sc - b and b, b = sc & 1) as f16 pairs,
-// for the half's four sub-blocks at once: e6[g/2] / b6[g/2] hold those of sub-blocks 4H + g (g
-// even, g + 1); zero when d is zero
-struct Scales6 {
-    uint32_t e6[2], b6[2];
-};
-__device__ __forceinline__ Scales6 scale_pairs6(uint32_t sc) {
-    Scales6 o;
-    const h2 off = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-    q8x4_exact(sc & 0xFEFEFEFEu, o.e6[0], o.e6[1]);  // the even parts of the signed bytes
-    const uint32_t b = sc & 0x01010101u;
-    o.b6[0] = h2u(magic_pair(b, kSelLo) + off);
-    o.b6[1] = h2u(magic_pair(b, kSelHi) + off);
-    return o;
-}
-// the planes (sc - b)(q - 32) and b(q - 32) of sub-block j (S: its half's scales)
-__device__ __forceinline__ void operand6(const Raw6 &r, const Scales6 &S, int j, h8 &a1, h8 &a2) {
-    const int H = j >> 2, grp = j & 3;
-    const h2 ep = __builtin_bit_cast(h2, S.e6[grp >> 1]);
-    const h2 bp = __builtin_bit_cast(h2, S.b6[grp >> 1]);
-    const h2 E = {ep[grp & 1], ep[grp & 1]}, B = {bp[grp & 1], bp[grp & 1]};
-    const uint2 l = r.ql[2 * H + (grp & 1)], hq = r.qh[H];
-    const int shl = 4 * (grp >> 1), shh = 2 * grp;
-    const uint32_t v0 = ((l.x >> shl) & 0x0F0F0F0Fu) | (((hq.x >> shh) & 0x03030303u) << 4);
-    const uint32_t v1 = ((l.y >> shl) & 0x0F0F0F0Fu) | (((hq.y >> shh) & 0x03030303u) << 4);
-    const h2 c0 = q6_centered(v0, kSelLo), c1 = q6_centered(v0, kSelHi), c2 = q6_centered(v1, kSelLo),
-             c3 = q6_centered(v1, kSelHi);
-    a1 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * E), h2u(c1 * E), h2u(c2 * E), h2u(c3 * E)));
-    a2 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * B), h2u(c1 * B), h2u(c2 * B), h2u(c3 * B)));
-}
-
 // One token tile of NB 16-row columns against the workgroup's weight rows.
 template <int TYPE, int MODE, int NB>
 __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int rb,
@@ -392,10 +318,10 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
                 for (int a = 0; a < R; a++) {
                     if constexpr (Q4) {
-                        if (jj == 0) s4[a] = scale_pairs4(scales4(w4[a].h, j >> 2));
-                        a1[a] = operand4(w4[a], s4[a], j);
+                        if ((jj & 1) == 0) s4[a] = scale_pair4(w4[a].h, j >> 1);
+                        a1[a] = operand4(w4[a], s4[a], j >> 1, jj & 1);
                     } else {
-                        if (jj == 0) s6 = scale_pairs6(w6.sc[j >> 2]);
+                        if ((jj & 1) == 0) s6 = scale_pair6(w6.sc[j >> 2], j >> 1);
                         operand6(w6, s6, j, a1[a], a2[a]);
                     }
                 }

@@ -53,6 +53,32 @@ def test_gemm_vs_oracle(gpu, oracle, type_id, M, K, N):
 
 
 @pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("M,K,N", [
+    # each workgroup shape with ragged rows and tokens (an M that is no multiple of 4 stores single
+    # values); K below, at and above its slices (slices of no super-block, of unequal length, of
+    # more than one 1024-value window)
+    (33, 256, 17), (31, 2304, 1), (1001, 1280, 15), (4099, 2304, 16),   # 32 x 16
+    (513, 3328, 65), (1000, 4096, 97),                                  # 32 x 32
+    (1537, 1536, 201), (2801, 4096, 63),                                # 64 x 32
+    (4093, 1280, 130), (1533, 4352, 510),                               # 64 x 64
+    (4095, 2816, 333), (8191, 1024, 201),                               # 128 x 64
+    (6001, 2304, 513), (2047, 4352, 1027),                              # 128 x 128
+    (8190, 1280, 1025), (4093, 5376, 2047),                             # 256 x 128
+])
+def test_gemm_shapes_ragged(gpu, type_id, M, K, N):
+    rng = np.random.default_rng(M + K + N)
+    w = dev(synth.weights(rng, type_id, M, K))
+    x = torch.randn((N, K), device="cuda", generator=torch.Generator("cuda").manual_seed(M))
+    act = torch.zeros(N * (K // 128) * 144, dtype=torch.uint8, device="cuda")
+    case(f"gemm ragged type={type_id} M={M} K={K} N={N}")
+    gpu.ops.quantize_q8_1(x, act, K, N)
+    out = _run(gpu, type_id, w, act, M, K, N)
+    assert torch.equal(out, _run(gpu, type_id, w, act, M, K, N))  # no atomics: the same every time
+    ref = torch_ref.gemm(type_id, w, act, M, K, N)
+    assert rel_l2(host(out), ref.cpu().numpy()) < TOL
+
+
+@pytest.mark.parametrize("type_id", [12, 14])
 def test_gemm_zero_scales_and_range(gpu, oracle, type_id):
     """Zero weight blocks (d = 0 with nonzero quants), zero activation sub-blocks and sub-blocks
     six decades apart inside one row: the running scale carries across them."""
