@@ -88,14 +88,6 @@ struct GemmLds {
 // fragment read (one chunk each) cover the 64 banks once
 __device__ __forceinline__ int b_off(int row, int chunk) { return row * kStageK + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
-// a / b to within an ulp of the quotient (the plain product with the reciprocal where that is
-// not finite)
-__device__ __forceinline__ float ratio(float a, float b) {
-    const float r = __builtin_amdgcn_rcpf(b), q = a * r;
-    const float e = __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
-    return e == e ? e : q;
-}
-
 struct GemmArgs {
     const uint8_t *W;  // weights [M][K]
     const uint8_t *A;  // Q8_1 MMQ rows [N]
@@ -119,17 +111,6 @@ struct Buf {
         return __builtin_amdgcn_raw_buffer_load_b16(r, lane, uni, 0);
     }
 };
-
-// LDS accesses at a lane's byte address plus a constant (an offset of the instruction): the
-// address is hidden from the compiler, which otherwise keeps one sum per row in registers
-template <typename T>
-__device__ __forceinline__ T lds_get(uint32_t addr, uint32_t off) {
-    return *(__attribute__((address_space(3))) const T *)(uintptr_t)(addr + off);
-}
-template <typename T>
-__device__ __forceinline__ void lds_put(uint32_t addr, uint32_t off, T v) {
-    *(__attribute__((address_space(3))) T *)(uintptr_t)(addr + off) = v;
-}
 
 // The lane's raw weights of one super-block of its row: the quants of the four sub-block pairs
 // are replaced by the next block's as soon as a pair's operands are formed, the header is held

@@ -77,6 +77,7 @@ template <int TYPE>
 struct GwLds {
     _Float16 b[2][64 * 128];
     float rho[2][256];  // the rows' scale ratios of the stage's 4 (2) sub-blocks
+    uint32_t row[kGroupTile];  // the tile's token rows
     uint8_t w[Gw<TYPE>::kWaves][Gw<TYPE>::kArea];  // each wave's row tiles of one block
 };
 
@@ -160,6 +161,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
         for (int i = 0; i < 2; i++) wo[i] = ((64 * i + lane) / 9) * wrow_bytes + 16 * ((64 * i + lane) % 9);
         wo[2] = ((128 + lane / 4) / 9) * wrow_bytes + 16 * ((128 + lane / 4) % 9) + 4 * (lane & 3);
+#pragma unroll
+        for (int i = 0; i < 3; i++) asm volatile("" : "+v"(wo[i]));
     } else {
         // offsets from the 4-byte aligned address at or below the tile's first byte (tb: its
         // misalignment); bit 0 set for chunk 13, which moves 4 bytes on when sh = 2
@@ -203,21 +206,32 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         const int j = min(j0 + r, n_rows - 1);
         return MODE == 1 ? g.perm[row_base + j] : row_base + j;
     };
-    const _Float16 *ap[P];
+    uint32_t ao[P];  // in 16-byte units of the activations
 #pragma unroll
     for (int i = 0; i < P; i++) {
         const int s = 64 * W * i + tid, r = s / CH;
-        ap[i] = g.A + (size_t)stage_row(r) * K + 8 * gw_unslot<SK>(r, s % CH);
+        ao[i] = (uint32_t)stage_row(r) * (uint32_t)(K / 8) + gw_unslot<SK>(r, s % CH);
+        asm volatile("" : "+v"(ao[i]));
     }
     // ratio copies: float tid of the stage's [row][sub-block] array (waves 0-3)
-    const float *rp = g.a_rho + (size_t)stage_row((tid & 255) / SJ) * (K / 32) + tid % SJ;
+    uint32_t ro = (uint32_t)stage_row((tid & 255) / SJ) * (uint32_t)(K / 32) + tid % SJ;
+    asm volatile("" : "+v"(ro));
     auto copy_b = [&](int t, int buf) {  // stage t (t * SK values into the rows)
-        if (W == 4 || wave < 4) lds_copy4(rp + (size_t)t * SJ, lds_r + buf * (uint32_t)sizeof L.rho[0]);
+        if (W == 4 || wave < 4) lds_copy4(g.a_rho + (size_t)t * SJ + ro, lds_r + buf * (uint32_t)sizeof L.rho[0]);
 #pragma unroll
         for (int i = 0; i < P; i++)
             if (64 * W * (i + 1) <= NB * 16 * CH || 64 * W * i + 64 * wave < NB * 16 * CH)  // wave-uniform
-                lds_copy16(ap[i] + (size_t)t * SK, lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
+                lds_copy16(g.A + (size_t)t * SK + 8 * (size_t)ao[i], lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
     };
+
+    // the lane's LDS addresses: its fragment chunk of each sub-block of a stage, its column's ratios
+    uint32_t fra[SJ], rra = lds + (uint32_t)offsetof(GwLds<TYPE>, rho) + 4 * SJ * c;
+#pragma unroll
+    for (int jj = 0; jj < SJ; jj++) {
+        fra[jj] = lds + 2 * gw_slot<SK>(c, 4 * jj + q);
+        asm volatile("" : "+v"(fra[jj]));
+    }
+    asm volatile("" : "+v"(rra));
 
     f4 acc[R][NB];
     float deff[R];  // running d of the lane's A row c of each tile
@@ -227,6 +241,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
         deff[a] = 1.0f;
     }
+    if (tid < 16 * NB) lds_put<uint32_t>(lds + (uint32_t)offsetof(GwLds<TYPE>, row), 4 * tid, (uint32_t)stage_row(tid));
     copy_b(0, 0);
     copy_w(0);
     uint32_t dn = 0;  // Q6_K: f16 d of row c's next block
@@ -245,7 +260,6 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     // staged ratios assume.  (Adding the term before the main loop read every header's weight
     // line twice: gate/up of 512 tokens ~1.04 against ~1.01 ms in all.)
     uint2 mins[Q4 ? R : 1];
-    uint32_t dmins[Q4 ? R : 1];
     const int nwin = (nkb + 3) / 4;
     // every wave's copies of the first stage and block have landed before any wave passes
     wait_vm<0>();
@@ -280,10 +294,9 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                     for (int a = 0; a < R; a++) {
                         d[a] = h2f(w4[a].h.x & 0xFFFFu);
                         const bool cap = (k & 3) == q;
-                        const uint2 mn = q4k_mins(w4[a].h);
+                        const uint2 mn = q4k_min_pack(w4[a].h);
                         mins[a].x = cap ? mn.x : mins[a].x;
                         mins[a].y = cap ? mn.y : mins[a].y;
-                        dmins[a] = cap ? w4[a].h.x >> 16 : dmins[a];
                         if (d[a] == 0.0f) w4[a].h.y = w4[a].h.w = 0u;  // scales 0: the block's products are zero
                     }
                 } else if (d[0] == 0.0f) {
@@ -294,7 +307,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
                 for (int a = 0; a < R; a++) {
                     const float nd = d[a] == 0.0f ? deff[a] : d[a];
-                    const float sg = deff[a] * __builtin_amdgcn_rcpf(nd);
+                    const float sg = ratio(deff[a], nd);
                     deff[a] = nd;
 #pragma unroll
                     for (int x = 0; x < 4; x++) {
@@ -304,16 +317,11 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                     }
                 }
             }
-            const _Float16 *bb = L.b[buf];
-            const float *rb = L.rho[buf];
             Scales4 s4[Q4 ? R : 1];
             Scales6 s6;
 #pragma unroll
             for (int jj = 0; jj < SJ; jj++) {
                 const int j = SJ * s + jj;  // sub-block of the block
-                float rr[NB];  // the token columns' ratios
-#pragma unroll
-                for (int b = 0; b < NB; b++) rr[b] = rb[(16 * b + c) * SJ + jj];
                 h8 a1[R], a2[Q4 ? 1 : R];
 #pragma unroll
                 for (int a = 0; a < R; a++) {
@@ -325,19 +333,23 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                         operand6(w6, s6, j, a1[a], a2[a]);
                     }
                 }
-                constexpr int NG = NB > 4 ? 2 : 1, NC = NB / NG;  // columns in groups of at most 4
+                constexpr int NG = NB > 4 ? NB / 2 : 1, NC = NB / NG;  // columns in groups of at most 4
 #pragma unroll
                 for (int gr = 0; gr < NG; gr++) {
                     h8 bf[NC];
+                    float rr[NC];  // the token columns' ratios
 #pragma unroll
                     for (int b = 0; b < NC; b++)
-                        bf[b] = *(const h8 *)(bb + gw_slot<SK>(16 * (NC * gr + b) + c, 4 * jj + q));
+                        rr[b] = lds_get<float>(rra, (buf * 256 + 16 * (NC * gr + b) * SJ + jj) * 4);
+#pragma unroll
+                    for (int b = 0; b < NC; b++)
+                        bf[b] = lds_get<h8>(fra[jj], buf * (uint32_t)sizeof L.b[0] + 16 * (NC * gr + b) * SK * 2);
 #pragma unroll
                     for (int a = 0; a < R; a++)
 #pragma unroll
                         for (int b = 0; b < NC; b++) {
                             f4 &ac = acc[a][NC * gr + b];
-                            ac *= rr[NC * gr + b];
+                            ac *= rr[b];
                             ac = mfma(a1[a], bf[b], ac);
                             if constexpr (!Q4) ac = mfma(a2[a], bf[b], ac);
                         }
@@ -349,8 +361,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                 // the window's last blocks: lane groups past the row's end add nothing
                 const bool valid = 4 * w + q < nkb;
                 const int sb = min(4 * w + q, nkb - 1);
-                int cw = c;  // not known to be loop-invariant: the rows' addresses are formed here, once
-                asm volatile("" : "+v"(cw));  // per window, instead of in registers held through the loop
+                uint32_t rowa = lds + (uint32_t)offsetof(GwLds<TYPE>, row) + 4 * c;
+                asm volatile("" : "+v"(rowa));  // formed here, not held through the loop
                 float dr[R][4];
 #pragma unroll
                 for (int a = 0; a < R; a++) {
@@ -358,33 +370,30 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                     for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
                     deff[a] = 1.0f;
                 }
-                constexpr int NC = NB > 4 ? NB / 2 : NB;
+                // every operand is loaded before the first is used: the lane's weights and
+                // fragments are dead here, and their registers take them
+                float dt[NB];
+                h8 bd[Q4 ? NB : 1];
 #pragma unroll
-                for (int b0 = 0; b0 < NB; b0 += NC) {
-                    float dt[NC];
-                    h8 bd[Q4 ? NC : 1];
+                for (int b = 0; b < NB; b++) {
+                    const size_t tok = lds_get<uint32_t>(rowa, 64 * b);
+                    dt[b] = g.a_dlast[tok * nwin + w];
+                    if constexpr (Q4) bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
+                }
 #pragma unroll
-                    for (int b = 0; b < NC; b++) {
-                        const size_t tok = stage_row(16 * (b0 + b) + cw);
-                        dt[b] = g.a_dlast[tok * nwin + w];
+                for (int a = 0; a < R; a++) {
+                    h8 hi, lo;
+                    if constexpr (Q4) q4k_min_operand(valid ? mins[a] : make_uint2(0u, 0u), hi, lo);
+#pragma unroll
+                    for (int b = 0; b < NB; b++) {
+                        f4 &ac = acc[a][b];
+#pragma unroll
+                        for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
                         if constexpr (Q4) {
-                            bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
-                            if (!valid) bd[b] = h8{};
+                            const h8 bv = valid ? bd[b] : h8{};
+                            ac = mfma(lo, bv, mfma(hi, bv, ac));
                         }
                     }
-#pragma unroll
-                    for (int a = 0; a < R; a++) {
-                        h8 hi, lo;
-                        if constexpr (Q4) q4k_min_operand_m(mins[a], valid ? dmins[a] : 0u, hi, lo);
-#pragma unroll
-                        for (int b = 0; b < NC; b++) {
-                            f4 &ac = acc[a][b0 + b];
-#pragma unroll
-                            for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
-                            if constexpr (Q4) ac = mfma(lo, bd[b], mfma(hi, bd[b], ac));
-                        }
-                    }
-                    if constexpr (NB >= 6) __builtin_amdgcn_sched_barrier(0);
                 }
             }
             // the next stage's activations have landed for every wave (and, from the second

@@ -48,23 +48,6 @@ __device__ __forceinline__ h2 q6_centered(uint32_t v) {
 }
 __device__ __forceinline__ uint32_t h2u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
-// byte i of the 12 packed scale bytes held in three dwords
-__device__ __forceinline__ uint32_t sbyte(uint32_t s0, uint32_t s1, uint32_t s2, int i) {
-    const uint32_t w = i < 4 ? s0 : (i < 8 ? s1 : s2);
-    return (w >> (8 * (i & 3))) & 0xFFu;
-}
-// (sc, m) of sub-block j (get_scale_min_k4, kernels.cu:45-53)
-__device__ __forceinline__ void q4k_scale_min(uint32_t s0, uint32_t s1, uint32_t s2, int j, uint32_t &sc,
-                                              uint32_t &m) {
-    if (j < 4) {
-        sc = sbyte(s0, s1, s2, j) & 63;
-        m = sbyte(s0, s1, s2, j + 4) & 63;
-    } else {
-        sc = (sbyte(s0, s1, s2, j + 4) & 15) | ((sbyte(s0, s1, s2, j - 4) >> 6) << 4);
-        m = (sbyte(s0, s1, s2, j + 4) >> 4) | ((sbyte(s0, s1, s2, j) >> 6) << 4);
-    }
-}
-
 // The 8 six-bit mins of a Q4_K super-block as bytes, sub-blocks 0-3 / 4-7 (the packed form of
 // get_scale_min_k4, kernels.cu:45-53: m_j = scales[j+4] & 63 for j < 4, else
 // (scales[j+4] >> 4) | ((scales[j] >> 6) << 4)); hdr.z, hdr.w hold scale bytes 4-7, 8-11.
@@ -90,15 +73,15 @@ __device__ __forceinline__ void q4k_min_operand_m(uint2 mins, uint32_t dmin_bits
     hi = __builtin_bit_cast(h8, make_uint4(H[0], H[1], H[2], H[3]));
     lo = __builtin_bit_cast(h8, make_uint4(L[0], L[1], L[2], L[3]));
 }
-__device__ __forceinline__ void q4k_min_operand(const uint4 &hdr, h8 &hi, h8 &lo) {
-    q4k_min_operand_m(q4k_mins(hdr), hdr.x >> 16, hi, lo);
+// dmin and the mins of a block header in two registers: dmin's nibbles take the places of the
+// scales' low nibbles in hdr.w
+__device__ __forceinline__ uint2 q4k_min_pack(const uint4 &hdr) {
+    const uint32_t e = ((hdr.x >> 16) & 0x0F0Fu) | ((hdr.x >> 4) & 0x0F0F0000u);
+    return make_uint2(hdr.z, (hdr.w & 0xF0F0F0F0u) | e);
 }
-// the ds halves of the 8 sub-blocks of a super-block: two Q8_1 block headers
-__device__ __forceinline__ h8 ds_operand(const uint4 &b0, const uint4 &b1) {
-    const uint32_t sel = 0x07060302u;  // the high halves of two dwords
-    const uint4 u = make_uint4(__builtin_amdgcn_perm(b0.y, b0.x, sel), __builtin_amdgcn_perm(b0.w, b0.z, sel),
-                               __builtin_amdgcn_perm(b1.y, b1.x, sel), __builtin_amdgcn_perm(b1.w, b1.z, sel));
-    return __builtin_bit_cast(h8, u);
+__device__ __forceinline__ void q4k_min_operand(uint2 p, h8 &hi, h8 &lo) {
+    const uint32_t d = (p.y & 0x0F0Fu) | ((p.y >> 12) & 0xF0F0u);
+    q4k_min_operand_m(q4k_mins(make_uint4(0u, 0u, p.x, p.y)), d, hi, lo);
 }
 
 // ------------------------------------------------------------------ a lane's A operands
@@ -167,6 +150,14 @@ __device__ __forceinline__ void operand6(const Raw6 &r, const Scales6 &S, int j,
     a2 = __builtin_bit_cast(h8, make_uint4(h2u(c0 * B), h2u(c1 * B), h2u(c2 * B), h2u(c3 * B)));
 }
 
+// a / b to within an ulp of the quotient (the plain product with the reciprocal where that is
+// not finite)
+__device__ __forceinline__ float ratio(float a, float b) {
+    const float r = __builtin_amdgcn_rcpf(b), q = a * r;
+    const float e = __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+    return e == e ? e : q;
+}
+
 // ------------------------------------------------------------------ LDS copies and the MFMA
 // Copies 16 (4) bytes per lane from global memory straight into LDS: lane i's bytes land at
 // LDS address dst + 16 i (4 i), dst wave-uniform; the source is a lane's pointer, or a uniform base and a
@@ -192,6 +183,16 @@ __device__ __forceinline__ void lds_copy4(const void *base, uint32_t off, uint32
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base)
                  : "memory");
 }
+// LDS accesses at a lane's byte address plus a constant (an offset of the instruction): the
+// address is hidden from the compiler, which otherwise keeps one sum per row in registers
+template <typename T>
+__device__ __forceinline__ T lds_get(uint32_t addr, uint32_t off) {
+    return *(__attribute__((address_space(3))) const T *)(uintptr_t)(addr + off);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(uint32_t addr, uint32_t off, T v) {
+    *(__attribute__((address_space(3))) T *)(uintptr_t)(addr + off) = v;
+}
 // Waits until at most N of the wave's vector memory operations are outstanding (they complete
 // in the order of their issue).
 template <int N>
@@ -202,9 +203,6 @@ __device__ __forceinline__ void wait_vm() {
 
 __device__ __forceinline__ f4 mfma(const h8 &a, const h8 &b, const f4 &c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4 mfma0(const h8 &a, const h8 &b) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 }
 
 }  // namespace mnemo
