@@ -15,7 +15,7 @@
 //   xs      T staged rows of x (StagedAct: q8 [T][hidden] f16, rho and ds [T][hidden/32],
 //           dlast [T][ceil(hidden/1024)])
 //   counts  E ints, offsets E ints
-//   rank    T*k ints   (rank of a pair within its expert; -1 for dropped slots)
+//   rank    T*k ints   (rank of a pair within its expert and wave range; -1 for dropped slots)
 //   inv     T*k ints   (pair -> expert-sorted row, -1 for dropped slots)
 //   perm    T*k ints   (expert-sorted row -> token)
 //   tiles   1 + E + ceil(T*k/kGroupTile) ints (count, then (expert << 16) | token tile)
@@ -45,6 +45,7 @@ int launch_router_topk(const float *w, const float *x, const float *nw, float ep
 
 constexpr int kRouteThreads = 1024;
 constexpr int kRouteWaves = kRouteThreads / 64;
+constexpr int kRouteAhead = 8;  // steps whose loads are in flight together
 constexpr int kMaxMoeExperts = 512;
 constexpr int kMoeTileRows = kGroupTile;  // token rows per grouped GEMM tile
 
@@ -111,24 +112,36 @@ __global__ void __launch_bounds__(kRouteThreads) moe_route_kernel(const int *__r
     __shared__ int running[kMaxMoeExperts];
     __shared__ int wave_cnt[kRouteWaves][kMaxMoeExperts];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < kRouteWaves * E; i += kRouteThreads) wave_cnt[i / E][i % E] = 0;
+    for (int w = 0; w < kRouteWaves; w++)
+        for (int i = tid; i < E; i += kRouteThreads) wave_cnt[w][i] = 0;
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int per = ((pairs + kRouteWaves - 1) / kRouteWaves + 63) & ~63;  // pairs per wave range
     __syncthreads();
     {
         const int w0 = wave * per, w1 = min(w0 + per, pairs);
-        for (int c = w0; c < w1; c += 64) {  // wave-uniform
-            const int p = c + lane;
-            int e = p < w1 ? topk_idx[p] : -1;
-            if (e >= E) e = -1;  // out-of-range expert ids are dropped like empty slots
-            const int key = e < 0 ? E : e;  // E = "dropped" bucket, matched like any value
-            const uint64_t m = match_mask(key, bits);
-            const int r_in = __popcll(m & lt);
-            if (e >= 0) rank[p] = wave_cnt[wave][e] + r_in;
-            else if (p < w1) rank[p] = -1;
-            // the group's first lane adds the group; the next step's reads come after it
-            // (one wave's LDS operations complete in order)
-            if (e >= 0 && r_in == 0) wave_cnt[wave][e] += __popcll(m);
+        // one workgroup, so a serial chain of load latencies bounds it: the ids of kRouteAhead
+        // steps are loaded at a time, and the placing below divides nothing per pair (16,384 pairs:
+        // 41 us with one load per step and two divisions per pair, 34 so)
+        for (int c0 = w0; c0 < w1; c0 += 64 * kRouteAhead) {  // wave-uniform
+            int ids[kRouteAhead];
+#pragma unroll
+            for (int i = 0; i < kRouteAhead; i++) ids[i] = topk_idx[min(c0 + 64 * i + lane, pairs - 1)];
+#pragma unroll
+            for (int i = 0; i < kRouteAhead; i++) {
+                const int p = c0 + 64 * i + lane;
+                if (c0 + 64 * i >= w1) break;  // wave-uniform
+                int e = p < w1 ? ids[i] : -1;
+                if (e >= E) e = -1;  // out-of-range expert ids are dropped like empty slots
+                const int key = e < 0 ? E : e;  // E = "dropped" bucket, matched like any value
+                const uint64_t m = match_mask(key, bits);
+                const int r_in = __popcll(m & lt);
+                if (e >= 0) rank[p] = wave_cnt[wave][e] + r_in;
+                else if (p < w1) rank[p] = -1;
+                // the group's first lane adds the group; the next step's reads come after it
+                // (one wave's LDS operations complete in order)
+                if (e >= 0 && r_in == 0) wave_cnt[wave][e] += __popcll(m);
+                __builtin_amdgcn_wave_barrier();
+            }
         }
     }
     __syncthreads();
@@ -186,28 +199,32 @@ __global__ void __launch_bounds__(kRouteThreads) moe_route_kernel(const int *__r
         for (int j = 0; j < full; j++) tiles[1 + at + j] = (tid << 16) | j;
     }
     if (part) tiles[1 + atomicAdd(&s_cls[part], 1)] = (tid << 16) | full;
-    // place the pairs (loads of four pairs per thread in flight at a time)
-    for (int p0 = 0; p0 < pairs; p0 += 4 * kRouteThreads) {
-        int r[4], e[4];
+    // place the pairs: each wave its own range again, whose prefix row it knows
+    const int w0 = wave * per, w1 = min(w0 + per, pairs);
+    int t = (w0 + lane) / k, rem = (w0 + lane) % k;  // the pair's token, carried along
+    const int dt = 64 / k, dr = 64 % k;
+    for (int c0 = w0; c0 < w1; c0 += 64 * kRouteAhead) {
+        int r[kRouteAhead], e[kRouteAhead];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int p = min(p0 + tid + i * kRouteThreads, pairs - 1);
+        for (int i = 0; i < kRouteAhead; i++) {
+            const int p = min(c0 + 64 * i + lane, pairs - 1);
             r[i] = rank[p];
             e[i] = topk_idx[p];
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int p = p0 + tid + i * kRouteThreads;
-            if (p >= pairs) break;
-            if (r[i] < 0) {
-                inv[p] = -1;
-                continue;
+        for (int i = 0; i < kRouteAhead; i++) {
+            const int p = c0 + 64 * i + lane;
+            if (p < w1) {
+                const int q = r[i] < 0 ? -1 : s_off[e[i]] + wave_cnt[wave][e[i]] + r[i];
+                inv[p] = q;
+                if (q >= 0) perm[q] = t;
             }
-            const int rr = r[i] + wave_cnt[p / per][e[i]];
-            rank[p] = rr;
-            const int q = s_off[e[i]] + rr;
-            inv[p] = q;
-            perm[q] = p / k;
+            t += dt;
+            rem += dr;
+            if (rem >= k) {
+                rem -= k;
+                t++;
+            }
         }
     }
 }

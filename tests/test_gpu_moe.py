@@ -107,6 +107,41 @@ def test_moe_prefill_vs_oracle(gpu, oracle, T, H, EFF, E, k, down_type, skew):
     assert err_o < TOL_ORACLE
 
 
+# Tiles of every width: 1 .. 8 columns of 16 rows (5 and 7 run as 6 and 8), one row over and under,
+# second tiles, an empty expert, a tile count that is no multiple of 8; K = 1280 ends a 1024-value
+# window early.  9000 pairs: more than one batch of loads per wave in the routing, with a k
+# that does not divide 64.
+@pytest.mark.parametrize("counts,H,EFF,k,down_type", [
+    ((1, 16, 17, 48, 0, 49, 64, 65, 96, 97, 112, 113, 128, 129, 200), 1280, 768, 1, 12),
+    ((1, 16, 17, 48, 0, 49, 64, 65, 96, 97, 112, 113, 128, 129, 200), 1280, 768, 1, 14),
+    ((375,) * 24, 256, 256, 6, 14),
+])
+def test_moe_prefill_tile_widths(gpu, counts, H, EFF, k, down_type):
+    E = len(counts)
+    rng = np.random.default_rng(sum(counts) + H)
+    table = synth.expert_table(rng, E, H, EFF, down_type)
+    lay = synth.expert_layout(H, EFF, down_type)
+    if k == 1:
+        idx = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(-1, 1)
+    else:  # every token k different experts
+        T = sum(counts) // k
+        idx = ((np.arange(T)[:, None] * 5 + np.arange(k)[None, :] * 3) % E).astype(np.int32)
+    T = idx.shape[0]
+    w = rng.random((T, k)).astype(np.float32)
+    x = (0.05 * rng.standard_normal((T, H))).astype(np.float32)
+    out0 = np.zeros((T, H), dtype=np.float32)
+    case(f"moe_prefill widths T={T} H={H} EFF={EFF} E={E} k={k} down={down_type}")
+    args = (gpu, dev(table), lay, down_type, dev(x), dev(idx), dev(w), T, H, EFF, E, k, dev(out0))
+    got = host(_run(*args))
+    assert np.array_equal(got, host(_run(*args)))
+    comp = host(_compose_plain(gpu, dev(table), lay, down_type, dev(x), idx, w, T, H, EFF, dev(out0)))
+    got, comp = got.reshape(T, H).astype(np.float64), comp.reshape(T, H)
+    assert rel_l2(got, comp) < TOL
+    # no token is lost among the others: each within ten times the bar
+    err = np.linalg.norm(got - comp, axis=1) / np.linalg.norm(comp, axis=1)
+    assert err.max() < 10 * TOL
+
+
 @pytest.mark.parametrize("H", [512, 2048])
 def test_moe_prefill_zero_d_blocks(gpu, oracle, H):
     """Gate/up Q4_K blocks with d = 0 (dmin kept, so only the min term survives), scattered
