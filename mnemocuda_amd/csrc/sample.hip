@@ -38,13 +38,12 @@ __device__ __forceinline__ bool before(float pa, int ia, float pb, int ib) {
 }
 
 // ------------------------------------------------------------------ top-p selection
-// The 2048 candidates are sorted by (p desc, id asc) on 256 threads, 8 per thread: thread t
-// holds sorted positions 8t .. 8t+7 in registers.  A candidate's order is that of one 64-bit
-// key, {p bits, ~id} (p >= 0 orders like its bits); an empty slot (p < 0, NaN) is key 0 and
-// sorts last.  Bitonic network: strides below 8 inside a thread, 8 .. 256 between the lanes
-// of a wave (DPP up to 64, permutes at 128 and 256), 512 and 1024 through LDS.  Then the running sums (inclusive, in
-// sorted order: sequential within a thread, a scan over the threads), the nucleus and the
-// draw.
+// The 2048 candidates are sorted by (p desc, id asc) on 1024 threads, 2 per thread.  A
+// candidate's order is that of one 64-bit key, {p bits, ~id} (p >= 0 orders like its bits); an
+// empty slot (p < 0, NaN) is key 0 and sorts last.  Bitonic network: stride 1 inside a thread,
+// 2 .. 64 between the lanes of a wave (DPP, lane swaps at 32 and 64), 128 .. 1024 through LDS.
+// Then, on 256 threads of 8 sorted positions, the running sums (inclusive, in sorted order:
+// sequential within a thread, a scan over the threads), the nucleus and the draw.
 constexpr int kSelThreads = kCands / 8;  // 256
 constexpr int kSelWaves = kSelThreads / 64;
 
@@ -59,7 +58,7 @@ __device__ __forceinline__ uint64_t keep(uint64_t a, uint64_t b, bool better_her
 }
 
 // v of lane ^ M: DPP within rows of 16 lanes (quad permutes; row rotations, where lane i
-// reads lane (i - n) mod 16), a cross-lane permute beyond
+// reads lane (i - n) mod 16), row and half swaps of the vector unit beyond
 template <int M>
 __device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
     if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kDppXor1, 0xF, 0xF, false);
@@ -69,81 +68,80 @@ __device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
         const uint32_t up = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x12C, 0xF, 0xF, false);  // i + 4
         return (lane_id() & 4) ? dn : up;
     } else if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);
-    else return (uint32_t)__shfl_xor((int)v, M);
+    else if constexpr (M == 16) {  // rows 1, 3 of the first operand trade places with rows 0, 2 of the second
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (lane_id() & 16) ? r[0] : r[1];
+    } else {
+        static_assert(M == 32, "strides within a wave");
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (lane_id() & 32) ? r[0] : r[1];
+    }
 }
 
-// a bitonic pass between lanes t and t ^ M (strides 8M): every key's partner first, then
-// the choices (one wait for the exchanged values, not one per key)
+// a bitonic pass between lanes t and t ^ M (strides 2M)
 template <int M>
-__device__ __forceinline__ void lane_pass(uint64_t (&k)[8], bool better_here) {
-    uint64_t o[8];
+__device__ __forceinline__ void lane_pass(uint64_t (&k)[2], bool better_here) {
 #pragma unroll
-    for (int r = 0; r < 8; r++)
-        o[r] = ((uint64_t)xor_lane<M>((uint32_t)(k[r] >> 32)) << 32) | xor_lane<M>((uint32_t)k[r]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; r++) k[r] = keep(k[r], o[r], better_here);
-}
-
-// a bitonic pass of stride J < 8: pairs inside the thread's 8 keys (sorted positions 8t + r)
-template <int J>
-__device__ __forceinline__ void reg_pass(uint64_t (&k)[8], int t, int kk) {
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-        if (r & J) continue;
-        const bool up = ((8 * t + r) & kk) == 0;
-        const uint64_t a = k[r], b = k[r | J];
-        k[r] = keep(a, b, up);
-        k[r | J] = keep(a, b, !up);
+    for (int r = 0; r < 2; r++) {
+        const uint64_t o = ((uint64_t)xor_lane<M>((uint32_t)(k[r] >> 32)) << 32) | xor_lane<M>((uint32_t)k[r]);
+        k[r] = keep(k[r], o, better_here);
     }
 }
 
 struct SelLds {
-    uint64_t xch[kCands];
+    alignas(16) uint64_t xch[2][kCands];
     float wsum[kSelWaves];
     int wmin[2][kSelWaves];
     float cs_last;
 };
 
-// Every thread of the NT-thread workgroup calls this (it holds barriers); threads
-// t < kSelThreads hold candidates 8t .. 8t+7 in k (any order).  total = the sum of all p.
-template <int NT>
-__device__ void select_sorted(uint64_t (&k)[8], float total, float top_p, unsigned long long seed, SelLds &L,
+// Every thread of the workgroup calls this (it holds barriers) with two candidates in any
+// order.  total = the sum of all p.
+// One workgroup, so the sort's instructions bound it: 66 passes of the network over 2048 keys.
+// On 1024 threads a SIMD has four waves to issue from (with 8 keys on each of 256 threads it
+// had one, which issues at half the rate and waits out every exchange): the workspace form's
+// second launch 23.4 us, from 26.5 (vocabulary 151,936); both launches 35.3 -> 32.1, the
+// one-launch form 136.8 -> 126.7.
+__device__ void select_sorted(uint64_t (&kk2)[2], float total, float top_p, unsigned long long seed, SelLds &L,
                               int *__restrict__ out) {
-    static_assert(NT % 64 == 0 && NT >= kSelThreads, "the selection needs 256 threads");
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const bool act = t < kSelThreads;
     // bitonic sort, best first: at level kk the pair (e, e ^ j), e < e ^ j, puts the better
-    // key at e when (e & kk) == 0
+    // key at e when (e & kk) == 0; thread t holds positions 2t, 2t + 1
+    int buf = 0;
     for (int kk = 2; kk <= kCands; kk <<= 1) {
-        for (int j = kk >> 1; j >= 8; j >>= 1) {
-            const int m = j >> 3;  // partner thread t ^ m
-            const bool up = ((8 * t) & kk) == 0, lower = (t & m) == 0;
-            if (j < 512) {  // partner in the same wave (m is uniform)
-                const bool b = up == lower;
-                switch (m) {
-                case 1: lane_pass<1>(k, b); break;
-                case 2: lane_pass<2>(k, b); break;
-                case 4: lane_pass<4>(k, b); break;
-                case 8: lane_pass<8>(k, b); break;
-                case 16: lane_pass<16>(k, b); break;
-                default: lane_pass<32>(k, b); break;
-                }
-            } else {
-                if (act)
-#pragma unroll
-                    for (int r = 0; r < 8; r++) L.xch[8 * t + r] = k[r];
+        const bool up = ((2 * t) & kk) == 0;
+        for (int m = kk >> 2; m >= 1; m >>= 1) {  // partner thread t ^ m (uniform)
+            const bool b = up == ((t & m) == 0);
+            switch (m) {
+            case 1: lane_pass<1>(kk2, b); break;
+            case 2: lane_pass<2>(kk2, b); break;
+            case 4: lane_pass<4>(kk2, b); break;
+            case 8: lane_pass<8>(kk2, b); break;
+            case 16: lane_pass<16>(kk2, b); break;
+            case 32: lane_pass<32>(kk2, b); break;
+            default:  // between waves; the buffers alternate, so one barrier orders both their uses
+                *(ulonglong2 *)&L.xch[buf][2 * t] = make_ulonglong2(kk2[0], kk2[1]);
                 __syncthreads();
-                if (act)
-#pragma unroll
-                    for (int r = 0; r < 8; r++) k[r] = keep(k[r], L.xch[8 * (t ^ m) + r], up == lower);
-                __syncthreads();
+                const ulonglong2 o = *(const ulonglong2 *)&L.xch[buf][2 * (t ^ m)];
+                kk2[0] = keep(kk2[0], o.x, b);
+                kk2[1] = keep(kk2[1], o.y, b);
+                buf ^= 1;
             }
         }
-        // strides 4, 2, 1 inside the thread
-        if (kk > 4) reg_pass<4>(k, t, kk);
-        if (kk > 2) reg_pass<2>(k, t, kk);
-        reg_pass<1>(k, t, kk);
+        const uint64_t x = kk2[0], y = kk2[1];
+        kk2[0] = keep(x, y, up);
+        kk2[1] = keep(x, y, !up);
+    }
+    *(ulonglong2 *)&L.xch[buf][2 * t] = make_ulonglong2(kk2[0], kk2[1]);
+    __syncthreads();
+    // from here on 256 threads hold 8 sorted positions each, 8t .. 8t + 7
+    const bool act = t < kSelThreads;
+    uint64_t k[8];
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) {
+        const ulonglong2 v = act ? *(const ulonglong2 *)&L.xch[buf][8 * t + r] : make_ulonglong2(0, 0);
+        k[r] = v.x;
+        k[r + 1] = v.y;
     }
     // inclusive running sums of the positive p in sorted order
     float p[8], c[8];
@@ -338,10 +336,10 @@ __global__ void __launch_bounds__(kSampleThreads) sample_token_kernel(const floa
     const float total = red_f[0];
 
     __shared__ SelLds sel;
-    uint64_t key[8];
+    uint64_t key[2];
 #pragma unroll
-    for (int r = 0; r < 8; r++) key[r] = tid < kSelThreads ? cand_key(cp[8 * tid + r], ci[8 * tid + r]) : 0ull;
-    select_sorted<kSampleThreads>(key, total, top_p, seed, sel, out);
+    for (int r = 0; r < 2; r++) key[r] = cand_key(cp[2 * tid + r], ci[2 * tid + r]);
+    select_sorted(key, total, top_p, seed, sel, out);
 }
 
 // ------------------------------------------------------------------ workspace form
@@ -353,8 +351,8 @@ __global__ void __launch_bounds__(kSampleThreads) sample_token_kernel(const floa
 //     largest logit m_w and S_w = sum exp((z - m_w) / T) over its classes;
 //  2. sample_finish_kernel, one workgroup: M = max m_w, total = sum_w S_w exp((m_w - M) / T),
 //     p of the 2048 winners from their logits as the one-launch form computes them, then the
-//     same sort, nucleus and draw (temperature <= 0: the first winner in (z desc, id asc)
-//     order, the argmax).
+//     same sort, nucleus and draw; temperature <= 0: sample_argmax_kernel, the first winner in
+//     (z desc, id asc) order.
 // Differences to the one-launch form: the total is summed per class group first (fp32 sums
 // in another order); a class's 8th and 9th largest p can only be exchanged when their
 // logits differ but round to the same p.
@@ -473,15 +471,50 @@ __global__ void __launch_bounds__(kClsThreads) sample_classes_kernel(const float
     }
 }
 
-__global__ void __launch_bounds__(kSelThreads) sample_finish_kernel(const SampleWs *__restrict__ ws,
+// temperature <= 0: the best class winner (ties to the lower id).  Thread c holds class c's first
+// winner; the groups' sums are not needed (both launches 12.6 -> 11.7 us; 13.5 with this as a
+// branch of the sampling kernel's 1024 threads).
+__global__ void __launch_bounds__(kClasses) sample_argmax_kernel(const SampleWs *__restrict__ ws, int *__restrict__ out) {
+    __shared__ float wv[kClasses / 64];
+    __shared__ int wi[kClasses / 64];
+    const int tid = threadIdx.x;
+    float bv = ws->z[tid * kPerClass];
+    int bi = ws->id[tid * kPerClass];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(bv, o);
+        const int oi = __shfl_xor(bi, o);
+        if (ov > bv || (ov == bv && oi < bi)) {
+            bv = ov;
+            bi = oi;
+        }
+    }
+    if ((tid & 63) == 0) {
+        wv[tid >> 6] = bv;
+        wi[tid >> 6] = bi;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kClasses / 64; w++)
+            if (wv[w] > bv || (wv[w] == bv && wi[w] < bi)) {
+                bv = wv[w];
+                bi = wi[w];
+            }
+        *out = bi == 0x7FFFFFFF ? 0 : bi;
+    }
+}
+
+__global__ void __launch_bounds__(kSampleThreads) sample_finish_kernel(const SampleWs *__restrict__ ws,
                                                                     float temperature, float top_p,
                                                                     unsigned long long seed, int *__restrict__ out) {
     __shared__ SelLds sel;
-    __shared__ float wv[kSelWaves];
-    __shared__ int wi[kSelWaves];
     __shared__ float tot;
     __shared__ float Ms;
     const int tid = threadIdx.x;
+    // winners 2 tid, 2 tid + 1 of the 2048 (8 per class), loaded with the groups' values
+    static_assert(kCands == 2 * kSampleThreads, "two candidates per thread");
+    const float2 cz = *(const float2 *)(ws->z + 2 * tid);
+    const int2 ci = *(const int2 *)(ws->id + 2 * tid);
     if (tid < 64) {
         // one group per lane: the common max and the rescaled total as wave reductions
         // (one round trip to the workspace, a fixed summation order)
@@ -496,44 +529,11 @@ __global__ void __launch_bounds__(kSelThreads) sample_finish_kernel(const Sample
     }
     __syncthreads();
     const float M = Ms;
-    if (temperature <= 0.0f) {  // argmax: the best class winner (ties to the lower id)
-        static_assert(kClasses == kSelThreads, "thread c holds class c's first winner");
-        float bv = ws->z[tid * kPerClass];
-        int bi = ws->id[tid * kPerClass];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(bv, o);
-            const int oi = __shfl_xor(bi, o);
-            if (ov > bv || (ov == bv && oi < bi)) {
-                bv = ov;
-                bi = oi;
-            }
-        }
-        if ((tid & 63) == 0) {
-            wv[tid >> 6] = bv;
-            wi[tid >> 6] = bi;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            bv = wv[0];
-            bi = wi[0];
-            for (int w = 1; w < kSelWaves; w++)
-                if (wv[w] > bv || (wv[w] == bv && wi[w] < bi)) {
-                    bv = wv[w];
-                    bi = wi[w];
-                }
-            *out = bi == 0x7FFFFFFF ? 0 : bi;
-        }
-        return;
-    }
-    // thread t: class t's 8 winners, p as the one-launch form computes it
-    uint64_t key[8];
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int id = ws->id[8 * tid + r];
-        key[r] = cand_key(id == 0x7FFFFFFF ? -1.0f : expf((ws->z[8 * tid + r] - M) / temperature), id);
-    }
-    select_sorted<kSelThreads>(key, tot, top_p, seed, sel, out);
+    // p as the one-launch form computes it
+    uint64_t key[2];
+    key[0] = cand_key(ci.x == 0x7FFFFFFF ? -1.0f : expf((cz.x - M) / temperature), ci.x);
+    key[1] = cand_key(ci.y == 0x7FFFFFFF ? -1.0f : expf((cz.y - M) / temperature), ci.y);
+    select_sorted(key, tot, top_p, seed, sel, out);
 }
 
 int launch_sample_token_ws(const float *logits, int V, float temperature, float top_p, unsigned long long seed,
@@ -547,7 +547,10 @@ int launch_sample_token_ws(const float *logits, int V, float temperature, float 
     SampleWs *w = (SampleWs *)ws;
     hipLaunchKernelGGL(sample_classes_kernel, dim3(kClsGroups), dim3(kClsThreads), 0, stream, logits, V,
                        temperature > 0.0f ? temperature : 1.0f, w);
-    hipLaunchKernelGGL(sample_finish_kernel, dim3(1), dim3(kSelThreads), 0, stream, w, temperature, top_p, seed, out);
+    if (temperature <= 0.0f) hipLaunchKernelGGL(sample_argmax_kernel, dim3(1), dim3(kClasses), 0, stream, w, out);
+    else
+        hipLaunchKernelGGL(sample_finish_kernel, dim3(1), dim3(kSampleThreads), 0, stream, w, temperature, top_p, seed,
+                           out);
     return check_launch("sample_token_ws");
 }
 
