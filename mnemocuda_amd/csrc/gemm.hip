@@ -22,13 +22,14 @@
 //     rho = d8_prev / d8 of the token (one multiply per output per sub-block) and the MFMA
 //     then adds the sub-block's products straight into that rescaled accumulator, so t is
 //     never formed on its own: each step rounds like an fp32 sum of the exact products onto
-//     acc * rho.  At a super-block boundary the rows' acc is multiplied by d_prev / d once.  The epilogue
-//     multiplies by the last d8 * d.  A zero scale leaves the running scale unchanged and
-//     zeroes its block's operand (its products are zero).
+//     acc * rho.  At a super-block boundary the rows' acc is multiplied by d_prev / d once.  After
+//     every window of 1024 values acc is multiplied by the current d8 * d, so that it is
+//     absolute, and the scales start again from 1.  A zero scale leaves the running scale
+//     unchanged and zeroes its block's operand (its products are zero).
 //   * Q4_K's min term, sum_s -(dmin*m_s) * ds_js, is one more product over the sub-block
 //     index: -dmin*m (an f16 times a 6-bit integer, 17 significant bits) is split into an
-//     f16 hi + lo pair that is exact, ds is an f16 already, and two MFMAs per 32 sub-blocks
-//     add it to the finished absolute accumulator.
+//     f16 hi + lo pair that is exact, ds is an f16 already, and two MFMAs per window (32
+//     sub-blocks) add it to the absolute accumulator.
 //   Against the fp64 value the roundings are the rescale multiply and the MFMA's fp32
 //   accumulation per output per sub-block, and the rho quotients (measured ~1e-7 relative
 //   L2).
@@ -431,14 +432,23 @@ gemm_q8_1_kernel(GemmArgs g) {
             lds_barrier();
             if (ks == 0) {
 #pragma unroll
-                for (int z = z0; z < KS && z < z0 + kFit; z++)
+                for (int a = 0; a < R; a++)
 #pragma unroll
-                    for (int a = 0; a < R; a++)
+                    for (int b = 0; b < NB; b++)
 #pragma unroll
-                        for (int b = 0; b < NB; b++)
+                        for (int x = 0; x < 4; x++) {
+                            // summed as a tree: fewer roundings at the full sum's magnitude
+                            float v[kFit];
+                            const int n = KS - z0 < kFit ? KS - z0 : kFit;
 #pragma unroll
-                            for (int x = 0; x < 4; x++)
-                                acc[a][b][x] += red[((z - z0) * RG + rg) * kPer + ((a * NB + b) * 4 + x) * 64 + lane];
+                            for (int z = 0; z < n; z++)
+                                v[z] = red[(z * RG + rg) * kPer + ((a * NB + b) * 4 + x) * 64 + lane];
+#pragma unroll
+                            for (int st = 1; st < n; st <<= 1)
+#pragma unroll
+                                for (int z = 0; z + st < n; z += 2 * st) v[z] += v[z + st];
+                            acc[a][b][x] += v[0];
+                        }
             }
         }
         if (ks) return;
