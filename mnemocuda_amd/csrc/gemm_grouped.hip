@@ -9,14 +9,20 @@
 //   Q4_K sub-block j = 2g + h: qs bytes 32g + 8q .. +7, nibble h;
 //   Q6_K sub-block j = 4H + grp: ql bytes 64H + 32(grp%2) + 8q .. +7 (nibble grp/2), qh bytes
 //        32H + 8q .. +7 (bits 2grp), scale 8H + 2grp + q/2;
-// and the activation fragment is the staged row's values 32j + 8q .. +7 (natural order).
+// and the activation fragment is the staged row's values 32j + 8q .. +7, in the
+// same order of elements as the weights' (gemm_ops.hpp).
 //
 // What bounds it: up to ~32 tokens per expert the weights' bytes; above, the VALU (per 16 x 32
 // weights ~12 operations to form the operand, and 4 per 16 x 16 outputs for the running
 // scale, against one 16-cycle MFMA).  Both need work in flight from phases that do not
 // coincide, so the kernel runs as several small workgroups per CU (Q4_K: three of 4 waves,
 // 52 KB of LDS and 168 registers each; Q6_K: two of 8 waves, 128 registers): one workgroup's
-// copies, barriers, first loads and final stores pass while the others multiply.
+// copies, barriers, first loads and final stores pass while the others multiply.  No
+// instantiation spills: a reload in the loop waits for every copy issued before it (14 spilled
+// registers in the 128-token tiles: 423 against 398 us, below).
+// MoE prefill of 512 tokens (128 experts of 4096 -> 1536, top-8, Q6_K down): 830 -> 618 us; of 37
+// tokens 363 -> 275; of 2048 (64 experts of 2048 -> 768, Q4_K down) 654 -> 382; before: one
+// workgroup of 8 or 16 waves per CU, 64-token tiles.
 #include <cstddef>
 
 #include "gemm_ops.hpp"
@@ -206,22 +212,27 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         const int j = min(j0 + r, n_rows - 1);
         return MODE == 1 ? g.perm[row_base + j] : row_base + j;
     };
-    uint32_t ao[P];  // in 16-byte units of the activations
+    // offsets from the tile's first row (gathered rows: from the first of all, which 16-byte units
+    // reach for every staged x that fits the memory beside its fp32 source)
+    const int row0 = MODE == 1 ? 0 : row_base + j0;
+    const _Float16 *A0 = g.A + (size_t)row0 * K;
+    const float *rho0 = g.a_rho + (size_t)row0 * (K / 32);
+    uint32_t ao[P];  // in 16-byte units
 #pragma unroll
     for (int i = 0; i < P; i++) {
         const int s = 64 * W * i + tid, r = s / CH;
-        ao[i] = (uint32_t)stage_row(r) * (uint32_t)(K / 8) + gw_unslot<SK>(r, s % CH);
+        ao[i] = (uint32_t)(stage_row(r) - row0) * (uint32_t)(K / 8) + gw_unslot<SK>(r, s % CH);
         asm volatile("" : "+v"(ao[i]));
     }
     // ratio copies: float tid of the stage's [row][sub-block] array (waves 0-3)
-    uint32_t ro = (uint32_t)stage_row((tid & 255) / SJ) * (uint32_t)(K / 32) + tid % SJ;
+    uint32_t ro = (uint32_t)(stage_row((tid & 255) / SJ) - row0) * (uint32_t)(K / 32) + tid % SJ;
     asm volatile("" : "+v"(ro));
     auto copy_b = [&](int t, int buf) {  // stage t (t * SK values into the rows)
-        if (W == 4 || wave < 4) lds_copy4(g.a_rho + (size_t)t * SJ + ro, lds_r + buf * (uint32_t)sizeof L.rho[0]);
+        if (W == 4 || wave < 4) lds_copy4(rho0 + (size_t)t * SJ + ro, lds_r + buf * (uint32_t)sizeof L.rho[0]);
 #pragma unroll
         for (int i = 0; i < P; i++)
             if (64 * W * (i + 1) <= NB * 16 * CH || 64 * W * i + 64 * wave < NB * 16 * CH)  // wave-uniform
-                lds_copy16(g.A + (size_t)t * SK + 8 * (size_t)ao[i], lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
+                lds_copy16(A0 + (size_t)t * SK + 8 * (size_t)ao[i], lds_b + buf * (uint32_t)sizeof L.b[0] + 1024 * W * i);
     };
 
     // the lane's LDS addresses: its fragment chunk of each sub-block of a stage, its column's ratios
@@ -370,8 +381,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                     for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
                     deff[a] = 1.0f;
                 }
-                // every operand is loaded before the first is used: the lane's weights and
-                // fragments are dead here, and their registers take them
+                // every operand is loaded before the first is used: the lane's fragments are dead
+                // here, and their registers take them
                 float dt[NB];
                 h8 bd[Q4 ? NB : 1];
 #pragma unroll
