@@ -17,22 +17,25 @@
 //     sc * (q - 32) reaches 4096 in magnitude, where f16 holds only even integers: it is
 //     split into two exact planes, (sc - b) * (q - 32) (even) and b * (q - 32) with
 //     b = sc & 1, and the two MFMAs chain into t (|t| < 2^24, still exact).
-//   * The fp32 rescale is a running scale: the accumulator holds the sum in units of the
-//     current (row scale d) x (token scale d8).  Every sub-block multiplies acc by
-//     rho = d8_prev / d8 of the token (one multiply per output per sub-block) and the MFMA
-//     then adds the sub-block's products straight into that rescaled accumulator, so t is
-//     never formed on its own: each step rounds like an fp32 sum of the exact products onto
-//     acc * rho.  At a super-block boundary the rows' acc is multiplied by d_prev / d once.  After
-//     every window of 1024 values acc is multiplied by the current d8 * d, so that it is
-//     absolute, and the scales start again from 1.  A zero scale leaves the running scale
-//     unchanged and zeroes its block's operand (its products are zero).
+//   * The fp32 rescale is a running scale: the accumulator holds the sum of a span of K in units of
+//     the current (row scale d) x (token scale d8).  Each sub-block is one fma, acc = acc * rho + t
+//     with rho = d8_prev / d8 of the token: one rounding per sub-block.  A span is a super-block
+//     where a wave holds at most 8 output tiles (R NB <= 8): its sum, times d * d8 (exact, two f16
+//     factors), joins an absolute total by one more fma, so that the roundings at the full sum's
+//     magnitude are one per super-block.  Wider tiles have no registers for the totals: their span
+//     is a window of 1024 values, acc is also multiplied by d_prev / d of the rows at super-block
+//     boundaries, becomes absolute at the window's end, and the scales start again from 1.  Q4_K's
+//     wide tiles form acc * rho and let the MFMA add the products to it (two roundings): forming t
+//     first costs them 5 % (M = 4096, K = 4096, N = 1024: 69.0 against 73.2 us).  A zero scale
+//     leaves the running scale unchanged and zeroes its block's operand (its products are zero).
 //   * Q4_K's min term, sum_s -(dmin*m_s) * ds_js, is one more product over the sub-block
 //     index: -dmin*m (an f16 times a 6-bit integer, 17 significant bits) is split into an
 //     f16 hi + lo pair that is exact, ds is an f16 already, and two MFMAs per window (32
-//     sub-blocks) add it to the absolute accumulator.
-//   Against the fp64 value the roundings are the rescale multiply and the MFMA's fp32
-//   accumulation per output per sub-block, and the rho quotients (measured ~1e-7 relative
-//   L2).
+//     sub-blocks) form it.
+//   Relative L2 against the fp64 value, N(0, 1) activations: K = 256 7.5e-8, K = 4096 9.5e-8 (wide tiles
+//   2.5e-7 and 2.2e-7, Q4_K and Q6_K), K = 16384 1.0e-7 to 1.2e-7 (wide 5.0e-7 and 4.4e-7).  With
+//   one running sum per slice of K and two (Q6_K: three) roundings per sub-block: 9.1e-8, 1.4e-7
+//   (2.5e-7), 2.5e-7 (5.2e-7).
 //
 // An int8 MFMA does not fit this product on gfx950: v_mfma_i32_16x16x64_i8 sums 64 values,
 // two sub-blocks with different token scales, and the 32-deep v_mfma_i32_16x16x32_i8 runs
@@ -72,12 +75,13 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 template <int TYPE, int R, int RG, int KS, int NB>
 struct GemmLds {
     static constexpr int kPer = R * NB * 4 * 64;  // floats of a wave's accumulators
+    static constexpr bool kTotals = R * NB <= 8;  // a total per output beside the super-block's sum
     union {
         _Float16 b[KS][2][NB * 16 * kStageK];  // q8 of a stage's tokens, chunks XOR-swizzled (b_off)
         float red[KS > 1 ? kPer * RG : 1];  // after the loop: a slice's sums, lane-minor
     };
     float rho[KS][2][2][NB * 16];  // token scale ratios of the stage's sub-blocks
-    float unit[KS][2][NB * 16];    // the tokens' d8 units at the end of the window (two windows)
+    float unit[KS][2][NB * 16];    // the tokens' d8 units at the end of the span (two spans)
     // Q4_K: the f16 ds of the tokens' sub-blocks in the current window and the next
     uint16_t ds[TYPE == kTypeQ4K ? KS : 1][2][NB * 16][32];
     // .. and a lane's packed mins and dmin of the window's block 4 w + q, by row tile
@@ -170,7 +174,7 @@ struct RawW<kTypeQ6K> {
     __device__ __forceinline__ uint32_t d_bits() const { return dc; }
 };
 
-template <int TYPE, int R, int RG, int KS, int NB>
+template <int TYPE, int R, int RG, int KS, int NB, bool ONCE>
 __global__ void __launch_bounds__(64 * RG * KS) __attribute__((amdgpu_waves_per_eu(R * NB <= 4 ? 4 : 2)))
 gemm_q8_1_kernel(GemmArgs g) {
     using Lds = GemmLds<TYPE, R, RG, KS, NB>;
@@ -194,12 +198,12 @@ gemm_q8_1_kernel(GemmArgs g) {
 #pragma unroll
     for (int a = 0; a < R; a++) wo[a] = (uint32_t)(min(i0 + 16 * a + c, g.M - 1) - iw) * wrow;
     // loader role in the slice: thread -> token lt, values VP lp .. of each stage
-    constexpr int VP = NB * 16 * kStageK / (64 * RG) < 8 ? 8 : NB * 16 * kStageK / (64 * RG);
+    constexpr int VP = kTok * kStageK / (64 * RG);
     constexpr int PT = kStageK / VP;  // threads per token
+    static_assert(VP >= 8 && kTok * PT == 64 * RG, "every thread of a slice loads whole chunks of one token");
     const int ltid = rg * 64 + lane, lt = ltid / PT, lp = ltid % PT;
-    const bool loader = kTok * PT >= 64 * RG || lt < kTok;
     const Buf ab(g.A + ((size_t)j0 * (g.K / 128) + 2 * sb0) * kQ81Bytes);  // the tile's first token
-    const uint32_t ao = (uint32_t)(min(j0 + min(lt, kTok - 1), g.N - 1) - j0) * (uint32_t)(g.K / 128) * kQ81Bytes;
+    const uint32_t ao = (uint32_t)(min(j0 + lt, g.N - 1) - j0) * (uint32_t)(g.K / 128) * kQ81Bytes;
     struct RawA {
         uint32_t v[VP / 4];
         uint2 hd;  // (d8, ds) of the stage's two sub-blocks
@@ -229,7 +233,7 @@ gemm_q8_1_kernel(GemmArgs g) {
     uint32_t wd = ld + 64 * lt, dq = ld + 64 * c + 16 * q;  // ds: written, and the lane's window operand
     uint32_t wu = lds + offsetof(Lds, unit) + ((uint32_t)ks * 2 * kTok + lt) * 4;
     uint32_t mn0 = lds + offsetof(Lds, mins) + (uint32_t)wave * R * 1024 + 16 * lane;
-    uint32_t fr[2], rr0 = lr + 4 * c, wr = lr + 4 * lt, wc[VP / 8 > 0 ? VP / 8 : 1];
+    uint32_t fr[2], rr0 = lr + 4 * c, wr = lr + 4 * lt, wc[VP / 8];
 #pragma unroll
     for (int jj = 0; jj < 2; jj++) fr[jj] = lb + 2 * b_off(c, 4 * jj + q);
 #pragma unroll
@@ -237,42 +241,49 @@ gemm_q8_1_kernel(GemmArgs g) {
     asm volatile("" : "+v"(fr[0]), "+v"(fr[1]), "+v"(rr0), "+v"(wr), "+v"(mn0), "+v"(wd), "+v"(dq), "+v"(wu));
 #pragma unroll
     for (int i = 0; i < VP / 8; i++) asm volatile("" : "+v"(wc[i]));
-    float unit = 1.0f;  // the token's running d8 (1 at a window's start, unchanged by d8 = 0)
+    // the token's running d8: 1 at a span's start, unchanged by d8 = 0.  A span is a super-block
+    // (kTotals) or a window of four
+    constexpr bool kTotals = Lds::kTotals;
+    constexpr int kSpan = kTotals ? 2 : 4;  // log2 of its stages
+    float unit = 1.0f;
     auto convert_a = [&](int t, RawA &r, int buf) {
 #pragma unroll
         for (int i = 0; i < VP / 4; i++) asm volatile("" : "+v"(r.v[i]));  // pins, as RawW's
         asm volatile("" : "+v"(r.hd.x), "+v"(r.hd.y));
         const float d0 = h2f(r.hd.x & 0xFFFFu), d1 = h2f(r.hd.y & 0xFFFFu);
-        if ((t & 15) == 0) unit = 1.0f;
+        if ((t & ((1 << kSpan) - 1)) == 0) unit = 1.0f;
         const float c0 = d0 != 0.0f ? d0 : unit, c1 = d1 != 0.0f ? d1 : c0;
-        if (loader) {
-            // the PT threads of a token write the same values
-            lds_put<float>(wr, buf * 2 * kTok * 4, ratio(unit, c0));
-            lds_put<float>(wr, (buf * 2 + 1) * kTok * 4, ratio(c0, c1));
-            lds_put<float>(wu, ((t >> 4) & 1) * kTok * 4, c1);
-            if constexpr (Q4)
-                lds_put<uint32_t>(wd, ((t >> 4) & 1) * kTok * 64 + (t & 15) * 4,
-                                  __builtin_amdgcn_perm(r.hd.y, r.hd.x, 0x07060302u));  // the high halves
+        // the PT threads of a token write the same values
+        lds_put<float>(wr, buf * 2 * kTok * 4, ratio(unit, c0));
+        lds_put<float>(wr, (buf * 2 + 1) * kTok * 4, ratio(c0, c1));
+        lds_put<float>(wu, ((t >> kSpan) & 1) * kTok * 4, c1);
+        if constexpr (Q4)
+            lds_put<uint32_t>(wd, ((t >> 4) & 1) * kTok * 64 + (t & 15) * 4,
+                              __builtin_amdgcn_perm(r.hd.y, r.hd.x, 0x07060302u));  // the high halves
 #pragma unroll
-            for (int i = 0; i < VP / 8; i++) {
-                const int ch = VP / 8 * lp + i;
-                // a block whose d rounds to f16 zero keeps quants up to +-127: its values are 0 * q8
-                const bool zero = (ch < 4 ? d0 : d1) == 0.0f;
-                uint4 o;
-                q8x4_exact(zero ? 0u : r.v[2 * i], o.x, o.y);
-                q8x4_exact(zero ? 0u : r.v[2 * i + 1], o.z, o.w);
-                lds_put<u4v>(wc[i], buf * kBuf, u4v{o.x, o.y, o.z, o.w});
-            }
+        for (int i = 0; i < VP / 8; i++) {
+            const int ch = VP / 8 * lp + i;
+            // a block whose d rounds to f16 zero keeps quants up to +-127: its values are 0 * q8
+            const bool zero = (ch < 4 ? d0 : d1) == 0.0f;
+            uint4 o;
+            q8x4_exact(zero ? 0u : r.v[2 * i], o.x, o.y);
+            q8x4_exact(zero ? 0u : r.v[2 * i + 1], o.z, o.w);
+            lds_put<u4v>(wc[i], buf * kBuf, u4v{o.x, o.y, o.z, o.w});
         }
         unit = c1;
     };
 
-    f4 acc[R][NB];
-    float deff[R];  // running d of the lane's row of each tile
+    constexpr f4 kZero = {0.f, 0.f, 0.f, 0.f};
+    f4 acc[R][NB];                                // the span's sum
+    f4 tot[kTotals ? R : 1][kTotals ? NB : 1];  // the absolute sum of the spans before
+    float deff[R];  // d of the lane's row of each tile (a window's: its last nonzero d, 1 before)
 #pragma unroll
     for (int a = 0; a < R; a++) {
 #pragma unroll
-        for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < NB; b++) {
+            acc[a][b] = kZero;
+            if constexpr (kTotals) tot[a][b] = kZero;
+        }
         deff[a] = 1.0f;
     }
     RawW<TYPE> w[R];
@@ -307,6 +318,10 @@ gemm_q8_1_kernel(GemmArgs g) {
                     if (d == 0.0f) w[a].r.h.y = w[a].r.h.w = 0u;  // scales 0: the block's products are zero
                 } else {
                     if (d == 0.0f) w[a].r.sc[0] = w[a].r.sc[1] = 0u;
+                }
+                if constexpr (kTotals) {
+                    deff[a] = d;
+                    continue;
                 }
                 // the running row scale: lane c owns row c; the lane's outputs are rows 4q + x
                 const float nd = d == 0.0f ? deff[a] : d;
@@ -353,55 +368,87 @@ gemm_q8_1_kernel(GemmArgs g) {
                     for (int b = 0; b < NB; b++)
 #pragma unroll
                         for (int a = 0; a < R; a++) {
-                            acc[a][b] *= rr[b];
-                            acc[a][b] = mfma(a1[a], bf[b], acc[a][b]);
-                            if constexpr (!Q4) acc[a][b] = mfma(a2[a], bf[b], acc[a][b]);
+                            f4 &ac = acc[a][b];
+                            if constexpr (!ONCE) {
+                                ac *= rr[b];
+                                ac = mfma(a1[a], bf[b], ac);
+                            } else {
+                                f4 t = mfma(a1[a], bf[b], kZero);
+                                if constexpr (!Q4) t = mfma(a2[a], bf[b], t);
+                                if (kTotals && s == 0 && jj == 0) ac = t;
+                                else ac = __builtin_elementwise_fma(ac, f4{rr[b], rr[b], rr[b], rr[b]}, t);
+                            }
                         }
                 }
-                if (s == 3 && ((k & 3) == 3 || k == n - 1)) {  // the window's end
-                    // the accumulators become absolute and take the Q4_K min term of the window's 32
-                    // sub-blocks, sum_s -(dmin*m_s)_i * ds_js: lane group q holds super-block 4w + q of its
-                    // row and token (K index 8q + s of the MFMA = sub-block s); groups past the end add
-                    // nothing
+                const bool wend = (k & 3) == 3 || k == n - 1;  // the window's last super-block
+                if (s == 3 && (kTotals || wend)) {             // the span's end
+                    // The sum becomes absolute, and the Q4_K min term of the window's 32 sub-blocks,
+                    // sum_s -(dmin*m_s)_i * ds_js, joins: lane group q holds super-block 4w + q of its row
+                    // and token (K index 8q + s of the MFMA = sub-block s); groups past the end add
+                    // nothing.  With totals the term goes to the total first, so that the span's sum is
+                    // the only addition at the new magnitude.
                     const int kw = (k & ~3) + q;
                     const bool valid = kw < n;
                     constexpr int NC = NB > 4 ? NB / 2 : NB;  // columns at a time
-                    float dr[R][4];
+                    const int wp = (k >> 2) & 1, up = kTotals ? k & 1 : wp;
+                    // the term of column b, on top of c
+                    auto min_term = [&](const h8 &hi, const h8 &lo, int b, const f4 &c) {
+                        h8 bd = lds_get<h8>(dq, wp * kTok * 64 + 16 * b * 64);
+                        if (!valid) bd = h8{};
+                        return mfma(lo, bd, mfma(hi, bd, c));
+                    };
+                    auto min_rows = [&](int a, h8 &hi, h8 &lo) {
+                        const u4v mn = lds_get<u4v>(mn0, a * 1024);
+                        q4k_min_operand_m(make_uint2(mn.x, mn.y), valid ? mn.z : 0u, hi, lo);
+                    };
+                    if constexpr (kTotals) {
+                        // the sums are formed here: the compiler would sink them past the branch, since
+                        // only the total uses them, and keep every product until then
 #pragma unroll
-                    for (int a = 0; a < R; a++) {
+                        for (int a = 0; a < R; a++)
 #pragma unroll
-                        for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
-                        deff[a] = 1.0f;
+                            for (int b = 0; b < NB; b++) asm volatile("" : "+v"(acc[a][b]));
+                    }
+                    if constexpr (Q4 && kTotals) {
+                        if (wend) {
+#pragma unroll
+                            for (int a = 0; a < R; a++) {
+                                h8 hi, lo;
+                                min_rows(a, hi, lo);
+#pragma unroll
+                                for (int b = 0; b < NB; b++) tot[a][b] = min_term(hi, lo, b, tot[a][b]);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                        }
                     }
 #pragma unroll
                     for (int b0 = 0; b0 < NB; b0 += NC) {
                         float dt[NC];
-                        h8 bd[Q4 ? NC : 1];
 #pragma unroll
-                        for (int b = 0; b < NC; b++) {
-                            dt[b] = L.unit[ks][(k >> 2) & 1][16 * (b0 + b) + c];
-                            if constexpr (Q4) {
-                                bd[b] = lds_get<h8>(dq, ((k >> 2) & 1) * kTok * 64 + 16 * (b0 + b) * 64);
-                                if (!valid) bd[b] = h8{};
-                            }
-                        }
+                        for (int b = 0; b < NC; b++) dt[b] = L.unit[ks][up][16 * (b0 + b) + c];
 #pragma unroll
                         for (int a = 0; a < R; a++) {
+                            float dr[4];
+#pragma unroll
+                            for (int x = 0; x < 4; x++) dr[x] = __shfl(deff[a], 4 * q + x);
                             h8 hi, lo;
-                            if constexpr (Q4) {
-                                const u4v mn = lds_get<u4v>(mn0, a * 1024);
-                                q4k_min_operand_m(make_uint2(mn.x, mn.y), valid ? mn.z : 0u, hi, lo);
-                            }
+                            if constexpr (Q4 && !kTotals) min_rows(a, hi, lo);
 #pragma unroll
                             for (int b = 0; b < NC; b++) {
                                 f4 &ac = acc[a][b0 + b];
+                                f4 to = kZero;
+                                if constexpr (kTotals) to = tot[a][b0 + b];
+                                else if constexpr (Q4) to = min_term(hi, lo, b0 + b, kZero);
 #pragma unroll
-                                for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
-                                if constexpr (Q4) ac = mfma(lo, bd[b], mfma(hi, bd[b], ac));
+                                for (int x = 0; x < 4; x++) to[x] = __builtin_fmaf(ac[x], dr[x] * dt[b], to[x]);
+                                if constexpr (kTotals) tot[a][b0 + b] = to;
+                                else ac = to;
                             }
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
+#pragma unroll
+                    for (int a = 0; a < R; a++) deff[a] = 1.0f;
                 }
                 lds_barrier();
             }
@@ -410,6 +457,12 @@ gemm_q8_1_kernel(GemmArgs g) {
         }
     }
 
+    if constexpr (kTotals) {
+#pragma unroll
+        for (int a = 0; a < R; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = tot[a][b];
+    }
     // the slices' sums meet in slice 0's waves, through the (now idle) stages, lane-minor so that
     // the accesses are conflict-free
     if constexpr (KS > 1) {
@@ -594,6 +647,18 @@ struct GemmShape {
 #define MNEMO_GEMM_SHAPE(I_, R_, RG_, KS_, NB_, ...) {R_, RG_, KS_, NB_, __VA_ARGS__},
 static const GemmShape kShapes[] = {MNEMO_GEMM_SHAPES(MNEMO_GEMM_SHAPE)};
 
+template <int TYPE, int I, int R, int RG, int KS, int NB>
+static void gemm_shape_launch(const GemmArgs &g, dim3 grid, hipStream_t stream) {
+    constexpr bool kOnce = TYPE == kTypeQ6K || GemmLds<TYPE, R, RG, KS, NB>::kTotals;
+    if constexpr (TYPE == kTypeQ4K && I == 0) {
+        if (g.K == 256) {
+            hipLaunchKernelGGL((gemm_q8_1_kernel<TYPE, R, RG, KS, NB, true>), grid, dim3(64 * RG * KS), 0, stream, g);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((gemm_q8_1_kernel<TYPE, R, RG, KS, NB, kOnce>), grid, dim3(64 * RG * KS), 0, stream, g);
+}
+
 static int gemm_tiles(int n, int tile) { return (int)(((long)n + tile - 1) / tile); }
 
 int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M, int K, int N,
@@ -613,6 +678,9 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
         const GemmShape &h = kShapes[i];
         const double *c = type == kTypeQ4K ? h.q4 : h.q6;
         if (i && gemm_tiles(N, 16 * h.nb) > 65535) continue;  // the grid's second dimension
+        // (Q4_K's wide tiles round twice per sub-block, which shows in a sum of one super-block: of them
+        // only shape 0 has a form that rounds once)
+        if (type == kTypeQ4K && nsb == 1 && h.r * h.nb > 8 && i) continue;
         const long tiles = (long)gemm_tiles(M, 16 * h.r * h.rg) * gemm_tiles(N, 16 * h.nb);
         const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]);
         if (i == 0 || t < least) {
@@ -621,14 +689,10 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
         }
     }
     const dim3 grid(gemm_tiles(M, 16 * kShapes[best].r * kShapes[best].rg), gemm_tiles(N, 16 * kShapes[best].nb));
-#define MNEMO_GEMM(I_, R_, RG_, KS_, NB_, ...)                                                                   \
-    case I_:                                                                                                     \
-        if (type == kTypeQ4K)                                                                                    \
-            hipLaunchKernelGGL((gemm_q8_1_kernel<kTypeQ4K, R_, RG_, KS_, NB_>), grid, dim3(64 * RG_ * KS_), 0,   \
-                               stream, g);                                                                       \
-        else                                                                                                     \
-            hipLaunchKernelGGL((gemm_q8_1_kernel<kTypeQ6K, R_, RG_, KS_, NB_>), grid, dim3(64 * RG_ * KS_), 0,   \
-                               stream, g);                                                                       \
+#define MNEMO_GEMM(I_, R_, RG_, KS_, NB_, ...)                                                          \
+    case I_:                                                                                            \
+        if (type == kTypeQ4K) gemm_shape_launch<kTypeQ4K, I_, R_, RG_, KS_, NB_>(g, grid, stream);      \
+        else gemm_shape_launch<kTypeQ6K, I_, R_, RG_, KS_, NB_>(g, grid, stream);                       \
         break;
     switch (best) { MNEMO_GEMM_SHAPES(MNEMO_GEMM) }
 #undef MNEMO_GEMM

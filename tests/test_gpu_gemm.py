@@ -78,6 +78,29 @@ def test_gemm_shapes_ragged(gpu, type_id, M, K, N):
     assert rel_l2(host(out), ref.cpu().numpy()) < TOL
 
 
+# Roundings of a sum: within a super-block one per sub-block at the running sum's magnitude, which
+# grows as the square root of its length (8 / 2 of the block's sum in the mean of squares); then one
+# per super-block of a slice (half of them, likewise), log2 for the tree over the slices, one each for
+# the min term and the store.  A rounding is 2^-24 / sqrt(3) relative in the root mean square, at
+# most (mantissas near 1); a tenth on top for the inputs' draw.
+@pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(64, 256, 300), (512, 4096, 300), (64, 16384, 64), (512, 16384, 300)])
+def test_gemm_rounds_once_per_sub_block(gpu, type_id, M, K, N):
+    case(f"gemm rounding type={type_id} M={M} K={K} N={N}")
+    rng = np.random.default_rng(M + K + N)
+    w = dev(synth.weights(rng, type_id, M, K))
+    x = torch.randn((N, K), device="cuda", generator=torch.Generator("cuda").manual_seed(M))
+    act = torch.zeros(N * (K // 128) * 144, dtype=torch.uint8, device="cuda")
+    gpu.ops.quantize_q8_1(x, act, K, N)
+    out = _run(gpu, type_id, w, act, M, K, N)
+    slices = min(8, K // 256)
+    roundings = 8 / 2 + (K // 256 // slices) / 2 + np.log2(slices) + 2
+    bar = 1.1 * 2.0**-24 * (roundings / 3) ** 0.5
+    err = rel_l2(host(out), torch_ref.gemm(type_id, w, act, M, K, N).cpu().numpy())
+    print(f"rel_l2={err:.3e} bar {bar:.3e}")
+    assert err < bar
+
+
 @pytest.mark.parametrize("type_id", [12, 14])
 def test_gemm_zero_scales_and_range(gpu, oracle, type_id):
     """Zero weight blocks (d = 0 with nonzero quants), zero activation sub-blocks and sub-blocks
