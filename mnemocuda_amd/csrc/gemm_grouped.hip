@@ -49,12 +49,13 @@ struct GroupedArgs {
 
 // Shape of a launch by weight type: waves per workgroup, 16-row tiles per wave, bytes of a
 // wave's weight area, and kLast, the 16-byte copies that end a block's weight copies.  The first
-// stage of a block waits until at most kLast operations are outstanding: 16-byte copies complete
-// in order, so the stage's activations, which went before, have landed.  Nothing else is
-// counted on: loads into registers (Q6_K's d) and 4-byte copies may complete in another order
-// (a wait that counted d among the younger operations let a stage read stale ratios about
-// once in 10^5 workgroups).  SwiGLU (MODE 1): the wave's tiles are the gate and up rows of the same
-// 16 features.
+// stage of a block waits until at most kLast operations are outstanding.  All that relies on is
+// that 16-byte LDS copies complete in order among themselves: everything the next stage reads was
+// either copied in 16-byte units before the last kLast of them or stored by the waves before the
+// barrier (gw_tile's copy_r).  4-byte copies and loads into registers may complete
+// in any order (a wait that counted Q6_K's d among the younger operations let a stage read stale ratios
+// about once in 10^5 workgroups); they are needed only after a wait for all.  SwiGLU (MODE 1): the
+// wave's tiles are the gate and up rows of the same 16 features.
 template <int TYPE>
 struct Gw;
 template <>
@@ -185,7 +186,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     const uint8_t *area = L.w[wave];
     // LDS addresses of the copies' targets (scalars)
     const uint32_t lds_w = lds + (uint32_t)offsetof(GwLds<TYPE>, w) + wave * T::kArea;
-    const uint32_t lds_b = lds + wave * 1024, lds_r = lds + (uint32_t)offsetof(GwLds<TYPE>, rho) + wave * 256;
+    const uint32_t lds_b = lds + wave * 1024, lds_r = lds + (uint32_t)offsetof(GwLds<TYPE>, rho);
     auto copy_w = [&](int k) {
         if constexpr (Q4) {
 #pragma unroll
@@ -224,11 +225,32 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         ao[i] = (uint32_t)(stage_row(r) - row0) * (uint32_t)(K / 8) + gw_unslot<SK>(r, s % CH);
         asm volatile("" : "+v"(ao[i]));
     }
-    // ratio copies: float tid of the stage's [row][sub-block] array (waves 0-3)
-    uint32_t ro = (uint32_t)(stage_row((tid & 255) / SJ) - row0) * (uint32_t)(K / 32) + tid % SJ;
+    // The stage's ratios, [row][sub-block].  128-value stages: a row's four are 16 bytes, one copy of
+    // wave 0 (lane = row).  64-value stages: float tid of the array, a 4-byte copy, which a
+    // block's second stage may not use (the first stage's counted wait does not cover it): its ratios
+    // come through a register, loaded during the last stage before the block, which ends in a wait
+    // for all.  (16-byte copies of two stages' ratios would need 2 KB more LDS, one workgroup per CU
+    // less; the register in 128-value stages too costs 1 % at 37 tokens.)
+    constexpr bool kReg = SK == 64;
+    uint32_t ro = kReg ? (uint32_t)(stage_row((tid & 255) / SJ) - row0) * (uint32_t)(K / 32) + tid % SJ
+                       : (uint32_t)(stage_row(lane) - row0) * (uint32_t)(K / 32);
     asm volatile("" : "+v"(ro));
+    auto copy_r = [&](int t, int buf) {
+        const uint32_t dst = buf * (uint32_t)sizeof L.rho[0];
+        if constexpr (!kReg) {
+            if (wave == 0) lds_copy16(rho0 + (size_t)t * SJ, 4 * ro, lds_r + dst);
+        } else if (W == 4 || wave < 4) {
+            lds_copy4(rho0 + (size_t)t * SJ + ro, lds_r + dst + wave * 256);
+        }
+    };
+    float rn = 0.0f;
+    auto load_r = [&](int k) {
+        if constexpr (kReg) rn = rho0[((size_t)k * NS + 1) * SJ + ro];
+    };
+    auto pin_r = [&] {
+        if constexpr (kReg) asm volatile("" : "+v"(rn));
+    };
     auto copy_b = [&](int t, int buf) {  // stage t (t * SK values into the rows)
-        if (W == 4 || wave < 4) lds_copy4(rho0 + (size_t)t * SJ + ro, lds_r + buf * (uint32_t)sizeof L.rho[0]);
 #pragma unroll
         for (int i = 0; i < P; i++)
             if (64 * W * (i + 1) <= NB * 16 * CH || 64 * W * i + 64 * wave < NB * 16 * CH)  // wave-uniform
@@ -253,7 +275,9 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         deff[a] = 1.0f;
     }
     if (tid < 16 * NB) lds_put<uint32_t>(lds + (uint32_t)offsetof(GwLds<TYPE>, row), 4 * tid, (uint32_t)stage_row(tid));
+    copy_r(0, 0);
     copy_b(0, 0);
+    load_r(0);
     copy_w(0);
     uint32_t dn = 0;  // Q6_K: f16 d of row c's next block
     auto load_d6 = [&](int k) {
@@ -274,6 +298,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     const int nwin = (nkb + 3) / 4;
     // every wave's copies of the first stage and block have landed before any wave passes
     wait_vm<0>();
+    pin_r();
     lds_barrier();
 
     for (int k = 0; k < nkb; k++) {
@@ -296,7 +321,11 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
             const int buf = s & 1;
             // the next stage's activations go first, then (first stage) the next block's
             // weights: the first stage's barrier leaves the weights in flight
-            copy_b(s + 1 < NS ? k * NS + s + 1 : kn * NS, buf ^ 1);
+            const int tn = s + 1 < NS ? k * NS + s + 1 : kn * NS;
+            if (!kReg || s) copy_r(tn, buf ^ 1);
+            else if (W == 4 || wave < 4) lds_put<float>(lds_r + 4 * (uint32_t)tid, sizeof L.rho[0], rn);
+            copy_b(tn, buf ^ 1);
+            if (s == NS - 1) load_r(kn);
             if (s == 0) {
                 copy_w(kn);
                 if constexpr (!Q4) load_d6(kn);
@@ -411,6 +440,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
             // stage on, the next block's weights)
             if (s == 0) wait_vm<T::kLast>();
             else wait_vm<0>();
+            if (s == NS - 1) pin_r();
             lds_barrier();
         }
     }

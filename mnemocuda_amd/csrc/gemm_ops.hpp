@@ -193,8 +193,9 @@ template <typename T>
 __device__ __forceinline__ void lds_put(uint32_t addr, uint32_t off, T v) {
     *(__attribute__((address_space(3))) T *)(uintptr_t)(addr + off) = v;
 }
-// Waits until at most N of the wave's vector memory operations are outstanding (they complete
-// in the order of their issue).
+// Waits until at most N of the wave's vector memory operations are outstanding.  Of the copies above,
+// those of 16 bytes are relied on to complete in the order of their issue; 4-byte copies and loads
+// into registers are not (a load into a register has been seen to overtake the copies), and need N = 0.
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
