@@ -42,6 +42,7 @@
 // at the f16 MFMA's rate (16 cycles for 16x16x32, measured) while needing three VALU
 // operations per output per sub-block (int -> float, the product of the row and token
 // scales, the fma) where the exact f16 form needs one.
+#include <algorithm>
 #include <cstddef>
 
 #include "gemm_ops.hpp"
@@ -98,10 +99,12 @@ struct GemmArgs {
     const uint8_t *A;  // Q8_1 MMQ rows [N]
     float *out;
     int M, K, N;
+    int ld;            // out[j * ld + i]
 };
 
 // Loads at a uniform base + a uniform offset + a lane's 32-bit offset (no 64-bit address per
-// lane and load: those took 20 registers and as many VALU operations per stage)
+// lane and load: those took 20 registers and as many VALU operations per stage).  The base is the
+// workgroup's first row, so its rows span less than 4 GiB (gemm_plan)
 struct Buf {
     __amdgpu_buffer_rsrc_t r;
     __device__ __forceinline__ explicit Buf(const uint8_t *p)
@@ -512,11 +515,11 @@ gemm_q8_1_kernel(GemmArgs g) {
     for (int b = 0; b < NB; b++) {
         const int j = j0 + 16 * b + c;
         if (j >= g.N) continue;
-        float *o = g.out + (size_t)j * g.M + i0 + 4 * q;
+        float *o = g.out + (size_t)j * g.ld + i0 + 4 * q;
 #pragma unroll
         for (int a = 0; a < R; a++) {
             const int i = i0 + 16 * a + 4 * q;
-            if (i + 3 < g.M && (g.M & 3) == 0) {
+            if (i + 3 < g.M && (g.ld & 3) == 0) {
                 *(f4 *)(o + 16 * a) = acc[a][b];
             } else {
 #pragma unroll
@@ -661,6 +664,54 @@ static void gemm_shape_launch(const GemmArgs &g, dim3 grid, hipStream_t stream) 
 
 static int gemm_tiles(int n, int tile) { return (int)(((long)n + tile - 1) / tile); }
 
+// The workgroup shape for a product, and the rows and tokens of one launch: all of them, unless even
+// the smallest tile's rows would span 4 GiB (K above 10^8), where launches of fewer rows take turns.
+struct GemmPlan {
+    int shape, rows, toks;
+};
+
+static GemmPlan gemm_plan(int type, int M, int K, int N, int cus) {
+    constexpr size_t kSpan = 0xFFFFFFFFu;
+    const int nsb = K / 256;
+    const size_t wrow = (size_t)nsb * (type == kTypeQ4K ? kQ4KBytes : kQ6KBytes), arow = (size_t)(K / 128) * kQ81Bytes;
+    // the first pass takes the shapes whose tiles fit, the second, if there was none, any shape
+    // over fewer rows (a multiple of 4 of them where it can be, for the stores' alignment)
+    for (;;) {
+        GemmPlan p{-1, M, N};
+        double least = 0;
+        for (int i = 0; i < (int)(sizeof kShapes / sizeof kShapes[0]); i++) {
+            const GemmShape &h = kShapes[i];
+            const double *c = type == kTypeQ4K ? h.q4 : h.q6;
+            if ((size_t)std::min(M, 16 * h.r * h.rg) * wrow > kSpan || (size_t)std::min(N, 16 * h.nb) * arow > kSpan)
+                continue;
+            if (i && gemm_tiles(N, 16 * h.nb) > 65535) continue;  // the grid's second dimension
+            // (Q4_K's wide tiles round twice per sub-block, which shows in a sum of one super-block: of them
+            // only shape 0 has a form that rounds once)
+            if (type == kTypeQ4K && nsb == 1 && h.r * h.nb > 8 && i) continue;
+            const long tiles = (long)gemm_tiles(M, 16 * h.r * h.rg) * gemm_tiles(N, 16 * h.nb);
+            const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]);
+            if (p.shape < 0 || t < least) {
+                p.shape = i;
+                least = t;
+            }
+        }
+        if (p.shape >= 0) return p;
+        const int rows = (int)std::min<size_t>(M, kSpan / wrow);
+        M = rows > 4 ? rows & ~3 : rows;
+        N = (int)std::min<size_t>(N, kSpan / arow);
+    }
+}
+
+// For the tests: the plan of a product on a device of cus CUs.  Returns the shape's index and writes
+// its tile (rows, tokens, slices of K) and the rows and tokens of one launch.
+extern "C" int mnemo_internal_gemm_plan(int type, int M, int K, int N, int cus, int out[5]) {
+    const GemmPlan p = gemm_plan(type, M, K, N, cus);
+    const GemmShape &h = kShapes[p.shape];
+    const int v[5] = {16 * h.r * h.rg, 16 * h.nb, h.ks, p.rows, p.toks};
+    for (int i = 0; i < 5; i++) out[i] = v[i];
+    return p.shape;
+}
+
 int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M, int K, int N,
                      hipStream_t stream) {
     if (!w || !act || !out || M <= 0 || N <= 0 || K <= 0 || K % 256 != 0)
@@ -670,32 +721,23 @@ int launch_gemm_q8_1(int type, const void *w, const void *act, float *out, int M
     if (((uintptr_t)act & 3) != 0) return set_error(kErrBadArg, "gemm: activation blocks must be 4-byte aligned");
     // activations are read as Q8_1 blocks and converted per tile: nothing is allocated, so
     // the call may sit inside a graph capture
-    const GemmArgs g{(const uint8_t *)w, (const uint8_t *)act, out, M, K, N};
-    const int cus = device_cus_gemm(), nsb = K / 256;
-    int best = 0;
-    double least = 0;
-    for (int i = 0; i < (int)(sizeof kShapes / sizeof kShapes[0]); i++) {
-        const GemmShape &h = kShapes[i];
-        const double *c = type == kTypeQ4K ? h.q4 : h.q6;
-        if (i && gemm_tiles(N, 16 * h.nb) > 65535) continue;  // the grid's second dimension
-        // (Q4_K's wide tiles round twice per sub-block, which shows in a sum of one super-block: of them
-        // only shape 0 has a form that rounds once)
-        if (type == kTypeQ4K && nsb == 1 && h.r * h.nb > 8 && i) continue;
-        const long tiles = (long)gemm_tiles(M, 16 * h.r * h.rg) * gemm_tiles(N, 16 * h.nb);
-        const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]);
-        if (i == 0 || t < least) {
-            best = i;
-            least = t;
-        }
-    }
-    const dim3 grid(gemm_tiles(M, 16 * kShapes[best].r * kShapes[best].rg), gemm_tiles(N, 16 * kShapes[best].nb));
-#define MNEMO_GEMM(I_, R_, RG_, KS_, NB_, ...)                                                          \
-    case I_:                                                                                            \
-        if (type == kTypeQ4K) gemm_shape_launch<kTypeQ4K, I_, R_, RG_, KS_, NB_>(g, grid, stream);      \
-        else gemm_shape_launch<kTypeQ6K, I_, R_, RG_, KS_, NB_>(g, grid, stream);                       \
-        break;
-    switch (best) { MNEMO_GEMM_SHAPES(MNEMO_GEMM) }
+    const GemmPlan plan = gemm_plan(type, M, K, N, device_cus_gemm());
+    const GemmShape &h = kShapes[plan.shape];
+    const size_t wrow = (size_t)(K / 256) * (type == kTypeQ4K ? kQ4KBytes : kQ6KBytes);
+    const size_t arow = (size_t)(K / 128) * kQ81Bytes;
+    for (int r0 = 0; r0 < M; r0 += plan.rows)
+        for (int t0 = 0; t0 < N; t0 += plan.toks) {
+            const GemmArgs g{(const uint8_t *)w + r0 * wrow, (const uint8_t *)act + t0 * arow, out + (size_t)t0 * M + r0,
+                             std::min(M - r0, plan.rows), K, std::min(N - t0, plan.toks), M};
+            const dim3 grid(gemm_tiles(g.M, 16 * h.r * h.rg), gemm_tiles(g.N, 16 * h.nb));
+#define MNEMO_GEMM(I_, R_, RG_, KS_, NB_, ...)                                                              \
+            case I_:                                                                                            \
+                if (type == kTypeQ4K) gemm_shape_launch<kTypeQ4K, I_, R_, RG_, KS_, NB_>(g, grid, stream);      \
+                else gemm_shape_launch<kTypeQ6K, I_, R_, RG_, KS_, NB_>(g, grid, stream);                       \
+                break;
+            switch (plan.shape) { MNEMO_GEMM_SHAPES(MNEMO_GEMM) }
 #undef MNEMO_GEMM
+        }
     return check_launch("gemm_q8_1");
 }
 

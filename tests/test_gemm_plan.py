@@ -1,0 +1,31 @@
+"""The plain GEMM's launch plan (host code only, no GPU)."""
+import ctypes as C
+
+import pytest
+
+from mnemocuda_amd import lib as mlib
+
+BLOCK = {12: 144, 14: 210}
+
+
+def plan(type_id, M, K, N, cus=256):
+    """(shape, rows and tokens of its tile, slices of K, rows and tokens of one launch)"""
+    out = (C.c_int * 5)()
+    shape = mlib.load_library().mnemo_internal_gemm_plan(type_id, M, K, N, cus, out)
+    return (shape, *out)
+
+
+@pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("M", [1, 3, 33, 300, 8192, 1 << 20])
+@pytest.mark.parametrize("K", [256, 16384, 1 << 24, 5 << 22, 1 << 27, 5 << 25, (1 << 31) - 256])
+@pytest.mark.parametrize("N", [1, 17, 2000, 1 << 21])
+def test_a_tile_spans_less_than_4_gib(type_id, M, K, N):
+    # offsets within a workgroup's rows are 32 bits
+    _, rows, toks, _, launch_rows, launch_toks = plan(type_id, M, K, N)
+    assert 1 <= launch_rows <= M and 1 <= launch_toks <= N
+    assert min(rows, launch_rows) * (K // 256) * BLOCK[type_id] < 1 << 32
+    assert min(toks, launch_toks) * (K // 128) * 144 < 1 << 32
+    if launch_rows < M:  # the next launch's output stays 16-byte aligned where the stores are 16 bytes
+        assert launch_rows % 4 == 0 or launch_rows < 4
+    if K <= 1 << 24:
+        assert (launch_rows, launch_toks) == (M, N)

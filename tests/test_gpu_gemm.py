@@ -175,3 +175,26 @@ def test_gemm_large_activations(gpu, oracle, type_id):
     # per token row: rows span 9 decades, so compare each on its own scale
     for j in range(N):
         assert rel_l2(got[j], ref[j]) < TOL, j
+
+
+def test_gemm_rows_over_4_gib(gpu):
+    """33 Q6_K rows of 137.6 MB: one workgroup's rows would span more than a 32-bit offset."""
+    M, K, N = 33, 5 << 25, 1
+    nsb = K // 256
+    gen = torch.Generator("cuda").manual_seed(3)
+    w = torch.randint(0, 256, (M, nsb, 210), dtype=torch.uint8, device="cuda", generator=gen)
+    w[:, :, 208:] = torch.tensor([0.01], dtype=torch.float16).view(torch.uint8).cuda()
+    act = torch.randint(0, 256, (N, K // 128, 144), dtype=torch.uint8, device="cuda", generator=gen)
+    act[:, :, :16] = torch.tensor([0.01, 0.0] * 4, dtype=torch.float16).view(torch.uint8).cuda()
+    case(f"gemm long rows M={M} K={K} N={N}")
+    out = _run(gpu, 14, w.view(-1), act.view(-1), M, K, N)
+    ref = torch.zeros((N, M), dtype=torch.float64, device="cuda")
+    step = 2048  # super-blocks at a time
+    for b in range(0, nsb, step):
+        n = min(step, nsb - b)
+        ref += torch_ref.gemm(14, w[:, b:b + n].reshape(-1), act[:, 2 * b:2 * (b + n)].reshape(-1), M, 256 * n, N).view(N, M)
+    # fp32 sums of 81,920 super-blocks per slice, one rounding each: 1.1 2^-24 sqrt(81,920 / 6); a row
+    # read 4 GiB away is an error of the result's size
+    err = rel_l2(host(out), ref.cpu().numpy())
+    print(f"rel_l2={err:.2e}")
+    assert err < 1.1 * 2.0**-24 * (nsb / 8 / 6) ** 0.5
