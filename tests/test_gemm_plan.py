@@ -4,6 +4,7 @@ import ctypes as C
 import pytest
 
 from mnemocuda_amd import lib as mlib
+from tests.test_gpu_gemm import RAGGED
 
 BLOCK = {12: 144, 14: 210}
 
@@ -29,3 +30,18 @@ def test_a_tile_spans_less_than_4_gib(type_id, M, K, N):
         assert launch_rows % 4 == 0 or launch_rows < 4
     if K <= 1 << 24:
         assert (launch_rows, launch_toks) == (M, N)
+
+
+@pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("shape", range(8))
+def test_gpu_sizes_reach_every_shape(type_id, shape):
+    """Each shape and type runs with ragged rows and tokens, once with slices of at most one super-block
+    and once with unequal slices of more than a window (four)."""
+    short = long = False
+    for M, K, N in RAGGED:
+        got, rows, toks, slices, *_ = plan(type_id, M, K, N)
+        if got == shape and M % rows and M % 4 and N % toks:
+            nsb = K // 256
+            short |= nsb <= slices
+            long |= nsb > 4 * slices and (slices == 1 or nsb % slices != 0)
+    assert short and long

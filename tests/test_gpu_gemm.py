@@ -27,9 +27,9 @@ def _run(gpu, type_id, wd, actd, M, K, N):
 
 @pytest.mark.parametrize("type_id,M,K,N", [(12, 256, 1024, 128), (12, 100, 512, 37), (14, 130, 768, 9),
                                            (12, 1, 256, 1), (14, 64, 1536, 200),
-                                           # ragged tiles with K split 8 ways (summed with atomics)
+                                           # ragged tiles with K in 8 slices
                                            (12, 200, 4096, 100), (14, 36, 2048, 68),
-                                           # 6 tiles of 9 super-blocks: uneven slices of K
+                                           # 9 super-blocks: uneven slices of K
                                            (12, 384, 2304, 130)])
 def test_gemm_vs_oracle(gpu, oracle, type_id, M, K, N):
     rng = np.random.default_rng(M * N + K)
@@ -52,19 +52,24 @@ def test_gemm_vs_oracle(gpu, oracle, type_id, M, K, N):
         assert np.all(np.abs(got - ref) <= bound)
 
 
+# Each workgroup shape with ragged rows and tokens (an M that is no multiple of 4 stores single
+# values), and K below, at and above its slices: slices of no super-block, of unequal length, of more
+# than one 1024-value window.  Which shape a size takes is the launch rule's; tests/test_gemm_plan.py
+# checks that the sizes below reach all of them, for both types.
+RAGGED = [
+    (33, 256, 17), (31, 2304, 1), (1001, 1280, 15), (4099, 2304, 16), (513, 3328, 65), (1000, 4096, 97),
+    (1537, 1536, 201), (2801, 4096, 63), (4093, 1280, 130), (1533, 4352, 510), (4095, 2816, 333), (8191, 1024, 201),
+    (6001, 2304, 513), (2047, 4352, 1027), (8190, 1280, 1025), (4093, 5376, 2047),
+    # at most one super-block per slice
+    (8197, 256, 197), (8263, 512, 195), (8307, 256, 68), (8603, 256, 33), (8201, 768, 33), (4131, 1280, 17),
+    # more than four
+    (33, 8448, 1), (33, 8704, 2070), (8219, 4352, 1), (8455, 4352, 33), (9395, 4864, 34), (8395, 2304, 34),
+    (5409, 2304, 337), (8225, 2304, 65), (8401, 2304, 104),
+]
+
+
 @pytest.mark.parametrize("type_id", [12, 14])
-@pytest.mark.parametrize("M,K,N", [
-    # each workgroup shape with ragged rows and tokens (an M that is no multiple of 4 stores single
-    # values); K below, at and above its slices (slices of no super-block, of unequal length, of
-    # more than one 1024-value window)
-    (33, 256, 17), (31, 2304, 1), (1001, 1280, 15), (4099, 2304, 16),   # 32 x 16
-    (513, 3328, 65), (1000, 4096, 97),                                  # 32 x 32
-    (1537, 1536, 201), (2801, 4096, 63),                                # 64 x 32
-    (4093, 1280, 130), (1533, 4352, 510),                               # 64 x 64
-    (4095, 2816, 333), (8191, 1024, 201),                               # 128 x 64
-    (6001, 2304, 513), (2047, 4352, 1027),                              # 128 x 128
-    (8190, 1280, 1025), (4093, 5376, 2047),                             # 256 x 128
-])
+@pytest.mark.parametrize("M,K,N", RAGGED)
 def test_gemm_shapes_ragged(gpu, type_id, M, K, N):
     rng = np.random.default_rng(M + K + N)
     w = dev(synth.weights(rng, type_id, M, K))
@@ -133,8 +138,8 @@ def test_gemm_zero_scales_and_range(gpu, oracle, type_id):
 
 
 @pytest.mark.parametrize("type_id,M,K,N", [(12, 8192, 4096, 512), (12, 1536, 4096, 512), (14, 4096, 1536, 512),
-                                           # 144 tiles, K unsplit: 18 super-blocks per workgroup, more than
-                                           # the min term keeps in LDS (it reads them from memory)
+                                           # 9 super-blocks per slice: three 1024-value windows, the last
+                                           # of one super-block
                                            (12, 2048, 4608, 1152)])
 def test_gemm_baseline_shapes(gpu, oracle, type_id, M, K, N):
     rng = np.random.default_rng(M + N)
