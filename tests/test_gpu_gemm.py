@@ -193,13 +193,33 @@ def test_gemm_rows_over_4_gib(gpu):
     act[:, :, :16] = torch.tensor([0.01, 0.0] * 4, dtype=torch.float16).view(torch.uint8).cuda()
     case(f"gemm long rows M={M} K={K} N={N}")
     out = _run(gpu, 14, w.view(-1), act.view(-1), M, K, N)
-    ref = torch.zeros((N, M), dtype=torch.float64, device="cuda")
-    step = 2048  # super-blocks at a time
+    rows = [0, 1, 15, 27, 28, 30, 31, 32]  # both launches, the first and last of each among them
+    ref = torch.zeros((N, len(rows)), dtype=torch.float64, device="cuda")
+    w = w[rows]
+    step = 8192  # super-blocks at a time
     for b in range(0, nsb, step):
         n = min(step, nsb - b)
-        ref += torch_ref.gemm(14, w[:, b:b + n].reshape(-1), act[:, 2 * b:2 * (b + n)].reshape(-1), M, 256 * n, N).view(N, M)
+        ref += torch_ref.gemm(14, w[:, b:b + n].reshape(-1), act[:, 2 * b:2 * (b + n)].reshape(-1), len(rows), 256 * n, N)
     # fp32 sums of 81,920 super-blocks per slice, one rounding each: 1.1 2^-24 sqrt(81,920 / 6); a row
     # read 4 GiB away is an error of the result's size
-    err = rel_l2(host(out), ref.cpu().numpy())
+    err = rel_l2(host(out)[:, rows], ref.cpu().numpy())
     print(f"rel_l2={err:.2e}")
     assert err < 1.1 * 2.0**-24 * (nsb / 8 / 6) ** 0.5
+
+
+@pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(33, 2304, 1), (130, 1280, 70), (2047, 2304, 513), (4099, 1280, 1025)])
+def test_gemm_any_weight_address(gpu, type_id, M, K, N):
+    """Weights may start at any byte, activation blocks at any multiple of 4."""
+    rng = np.random.default_rng(M + K)
+    w = dev(synth.weights(rng, type_id, M, K))
+    act = torch.zeros(N * (K // 128) * 144, dtype=torch.uint8, device="cuda")
+    gpu.ops.quantize_q8_1(torch.randn((N, K), device="cuda", generator=torch.Generator("cuda").manual_seed(M)), act, K, N)
+    case(f"gemm alignment type={type_id} M={M} K={K} N={N}")
+    ref = _run(gpu, type_id, w, act, M, K, N)
+    for off, aoff in ((1, 0), (2, 4), (3, 8), (8, 12)):
+        wu = torch.zeros(w.numel() + 16, dtype=torch.uint8, device="cuda")[off:off + w.numel()]
+        au = torch.zeros(act.numel() + 16, dtype=torch.uint8, device="cuda")[aoff:aoff + act.numel()]
+        wu.copy_(w)
+        au.copy_(act)
+        assert torch.equal(_run(gpu, type_id, wu, au, M, K, N), ref), (off, aoff)
