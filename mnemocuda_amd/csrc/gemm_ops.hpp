@@ -165,7 +165,8 @@ __device__ __forceinline__ float ratio(float a, float b) {
 // the copies' LDS targets from other LDS buffers, otherwise puts a wait for all of them in
 // front of the next LDS read, and the copies never overlap anything (MoE prefill 856 -> 772 us
 // at 512 tokens, 376 -> 327 us at 37; 128 experts of 4096 -> 1536, top-8).  Nothing waits for
-// these copies but wait_vm.  (M0 holds their LDS address; the compiler keeps nothing in it.)
+// these copies but wait_vm.  M0 holds their LDS address: a reserved register, which may not be named as a
+// clobber (the compiler warns); nothing else in these kernels uses it, which a test checks.
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {  // of a __shared__ object itself
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
 }

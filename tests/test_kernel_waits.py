@@ -1,4 +1,7 @@
-"""The grouped GEMM's counted wait, read from the compiled kernel's assembly (no GPU).
+"""What the grouped GEMM's hand-written copies rely on, read from its assembly (no GPU).
+
+M0 holds the copies' LDS address.  It is a reserved register, which an asm statement cannot declare as
+clobbered, so the compiler itself must have no use for it in these kernels.
 
 The first stage of a block ends in a wait that leaves the block's last four 16-byte weight copies in
 flight.  Only 16-byte LDS copies are relied on to complete in order, so between the barrier before
@@ -49,3 +52,13 @@ def test_counted_wait_covers_16_byte_copies_only(assembly, type_id, weights4, ke
         assert copies[-left:] == ["global_load_lds_dwordx4"] * left, ops
         assert copies[:-left].count("global_load_lds_dword") == weights4, ops
         assert "global_load_lds_dwordx4" in copies[:-left], ops
+
+
+def test_compiler_leaves_m0_alone(assembly):
+    asm, own = False, 0
+    for line in assembly:
+        asm = (asm or "ASMSTART" in line) and "ASMEND" not in line
+        if re.search(r"\bm0\b", line.split(";")[0]):
+            assert asm, line
+            own += 1
+    assert own
