@@ -163,7 +163,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     // weight copies.  Q4_K: a tile's block is 144 chunks of 16 B, row ch/9, bytes 16(ch%9);
     // chunks 0-127 in two copies, 128-143 as 64 dwords in a third.
     uint32_t wo[Q4 ? 3 : 4];
-    uint32_t tb = 0, roff = 0;
+    uint32_t roff = 0;
     if constexpr (Q4) {
 #pragma unroll
         for (int i = 0; i < 2; i++) wo[i] = ((64 * i + lane) / 9) * wrow_bytes + 16 * ((64 * i + lane) % 9);
@@ -171,17 +171,16 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
         for (int i = 0; i < 3; i++) asm volatile("" : "+v"(wo[i]));
     } else {
-        // offsets from the 4-byte aligned address at or below the tile's first byte (tb: its
-        // misalignment); bit 0 set for chunk 13, which moves 4 bytes on when sh = 2
-        tb = (uint32_t)(uintptr_t)tp[0] & 3u;
-        tp[0] -= tb;
+        // offsets from the tile's first byte, which is 4-byte aligned (16 rows are a multiple of 4
+        // bytes, the table's matrices are checked); bit 0 set for chunk 13, which moves 4 bytes on
+        // when sh = 2
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int t = 64 * i + lane, row = t < 16 * kSlots6 ? t / kSlots6 : 15;
             const int ch = t < 16 * kSlots6 ? t % kSlots6 : 12;
-            wo[i] = row * wrow_bytes + tb + (ch <= 12 ? 16u * (uint32_t)ch : ch == 13 ? 192u + 1u : 192u);
+            wo[i] = row * wrow_bytes + (ch <= 12 ? 16u * (uint32_t)ch : ch == 13 ? 192u + 1u : 192u);
         }
-        roff = c * wrow_bytes + tb;
+        roff = c * wrow_bytes;
     }
     const uint8_t *area = L.w[wave];
     // LDS addresses of the copies' targets (scalars)
@@ -213,8 +212,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         const int j = min(j0 + r, n_rows - 1);
         return MODE == 1 ? g.perm[row_base + j] : row_base + j;
     };
-    // offsets from the tile's first row (gathered rows: from the first of all, which 16-byte units
-    // reach for every staged x that fits the memory beside its fp32 source)
+    // offsets from the tile's first row (gathered rows: from the first of all; 32 bits of 16-byte units
+    // reach 2^35 values of x, whose fp32 source, staged rows, down rows and output take 480 GB)
     const int row0 = MODE == 1 ? 0 : row_base + j0;
     const _Float16 *A0 = g.A + (size_t)row0 * K;
     const float *rho0 = g.a_rho + (size_t)row0 * (K / 32);
