@@ -48,6 +48,9 @@ constexpr int kRouteWaves = kRouteThreads / 64;
 constexpr int kRouteAhead = 8;  // steps whose loads are in flight together
 constexpr int kMaxMoeExperts = 512;
 constexpr int kMoeTileRows = kGroupTile;  // token rows per grouped GEMM tile
+constexpr long kMaxMoePairs = 1L << 22;   // of one call
+// a tile-list entry is (expert << 16) | tile
+static_assert(kMaxMoePairs <= 65536L * kMoeTileRows, "an expert's tiles stay below 65536");
 
 struct MoeLayout {
     size_t xs, xr, xds, xdl, counts, offsets, rank, inv, perm, tiles, act, acts, actr, actds, actdl, down, total;
@@ -265,9 +268,8 @@ int launch_moe_prefill(const void *experts, size_t expert_stride, size_t gate_of
     if (E > kMaxMoeExperts) return set_error(kErrBadArg, "moe_prefill: at most %d experts", kMaxMoeExperts);
     if (hidden % 256 != 0 || eff % 256 != 0)
         return set_error(kErrBadArg, "moe_prefill: hidden and eff must be multiples of 256");
-    // a tile-list entry is (expert << 16) | tile: an expert's tiles must stay below 65536
-    if ((long)T * k > 65536L * kMoeTileRows)
-        return set_error(kErrBadArg, "moe_prefill: more than %ld token-expert pairs", 65536L * kMoeTileRows);
+    if ((long)T * k > kMaxMoePairs)
+        return set_error(kErrBadArg, "moe_prefill: more than %ld token-expert pairs", kMaxMoePairs);
     if (down_type != kTypeQ4K && down_type != kTypeQ6K)
         return set_error(kErrUnsupportedType, "moe_prefill: unsupported down type %d", down_type);
     if ((((uintptr_t)ws | (uintptr_t)x | (uintptr_t)out) & 15) != 0)

@@ -85,3 +85,12 @@ def test_bad_arguments_are_reported_without_launching(L, call, capfd):
 def test_expert_fwd_rejects_bad_down_type(L):
     assert L.mnemo_expert_fwd(16, 1, 1, 4096, 1536, 13, 1.0, 16, 16, 16, 16, None) == 3
     assert L.mnemo_expert_fwd(None, 1, 1, 4096, 1536, 12, 1.0, 16, 16, 16, 16, None) == 1
+
+
+def test_moe_prefill_pair_limit(L):
+    """At most 4,194,304 token-expert pairs a call, whatever the tiles' size (a workspace of no bytes
+    ends the accepted call)."""
+    for pairs, message in ((1 << 22, b"workspace"), ((1 << 22) + 64, b"more than 4194304 token-expert pairs")):
+        assert L.mnemo_moe_prefill(16, 1 << 20, 0, 4, 8, 12, 16, 16, 16, pairs // 64, 256, 256, 128, 64, 16, 0, 16, None) == 1
+        assert message in L.mnemo_last_error_string()
+        L.mnemo_last_error()
