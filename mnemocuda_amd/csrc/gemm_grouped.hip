@@ -137,17 +137,24 @@ __device__ __forceinline__ Raw6 read6(const uint8_t *area, int c, int q, uint32_
     r.sc[1] = __builtin_amdgcn_perm(sc.w, sc.z, sel);
     return r;
 }
+// the lane's index, formed where it is used and not held in a register through the main loop
+__device__ __forceinline__ uint32_t lane_here() {
+    uint32_t l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
 // One token tile of NB 16-row columns against the workgroup's weight rows.
 template <int TYPE, int MODE, int NB>
-__device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int rb,
-                                        int wave, int lane, int tid, int e, int j0, int n_rows, int row_base) {
+__device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> &L, uint32_t lds, int rb, int wave,
+                                        int e, int j0, int n_rows, int row_base) {
     using T = Gw<TYPE>;
     constexpr int W = T::kWaves, R = T::kR;
     constexpr bool Q4 = TYPE == kTypeQ4K;
     constexpr int SK = gw_stage_k<NB>(), NS = 256 / SK, SJ = SK / 32;  // stages per block, sub-blocks per stage
     constexpr int CH = SK / 8;                                         // 16-byte chunks per staged row
     constexpr int P = (NB * 16 * CH + 64 * W - 1) / (64 * W);          // copies per wave and stage
-    const int q = lane >> 4, c = lane & 15;
+    // formed per instantiation: what the switch's arms share is held, and spilled, through their loops
+    const int lane = lane_here(), tid = 64 * wave + lane, q = lane >> 4, c = lane & 15;
     const int K = g.K, nkb = K / 256;
     const uint32_t wrow_bytes = (uint32_t)nkb * (Q4 ? kQ4KBytes : kQ6KBytes);
     const uint8_t *Wm = g.W + (size_t)e * g.expert_stride + g.w_off;
@@ -286,15 +293,44 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     };
     if constexpr (!Q4) load_d6(0);
 
-    // Q4_K's min term, sum_s -(dmin*m_s)_i * ds_js, is one product over the sub-block index:
-    // two MFMAs (hi + lo operand) per window of 32 sub-blocks (4 blocks).  Lane group q keeps the
-    // packed mins and dmin of the window's block 4 w + q as it reads the headers (K index 8 q + s
-    // of the MFMA = sub-block s of that block); at the window's end the accumulators become
-    // absolute, take the term and start the next window with unit scales, which is what the
-    // staged ratios assume.  (Adding the term before the main loop read every header's weight
-    // line twice: gate/up of 512 tokens ~1.04 against ~1.01 ms in all.)
-    uint2 mins[Q4 ? R : 1];
+    // Q4_K's min term, sum_s -(dmin*m_s)_i * ds_js, is one product over the sub-block index: two
+    // MFMAs (hi + lo operand) per window of 32 sub-blocks (4 blocks), lane group q holding the window's
+    // block 4 w + q (K index 8 q + s of the MFMA = sub-block s of that block).
+    // Gate/up: the lanes keep the packed mins and dmin as they read the headers; at the window's
+    // end the term is formed on zero and the accumulators join it by one fma, which makes them absolute
+    // (4.9e-7 relative L2 against 64 bits, 5.1e-7 with the term added to the absolute accumulators;
+    // SwiGLU rows of K = 4096).
+    // Down: the accumulators start as the whole term.  Where activations are large the term and the
+    // products are larger than their sum, and the roundings scale with the sum so far: K = 768 1.07e-7
+    // against 1.39e-7 with the term at the windows' ends, K = 512 9.0e-8 against 9.9e-8.  (Activations
+    // several times larger, near where ds leaves the f16 range, favour the other order.)  It reads the
+    // headers' lines once more: the launch takes 130 us instead of 123 at K = 768, M = 2048, 16,384
+    // rows; gate/up of 512 tokens would pay 3 %.
+    constexpr bool kLate = Q4 && MODE == 1;
+    uint2 mins[kLate ? R : 1];
     const int nwin = (nkb + 3) / 4;
+    if constexpr (Q4 && !kLate) {
+        for (int w = 0; w < nwin; w++) {
+            const bool valid = 4 * w + q < nkb;  // lane groups past the row's end add nothing
+            const int sb = min(4 * w + q, nkb - 1);
+            uint4 hd[R], bd[NB];
+#pragma unroll
+            for (int a = 0; a < R; a++) hd[a] = ld16(tp[a] + c * wrow_bytes + (size_t)sb * kQ4KBytes);
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                bd[b] = ld16((const uint8_t *)(g.a_ds + (size_t)stage_row(16 * b + c) * (K / 32) + 8 * sb));
+#pragma unroll
+            for (int a = 0; a < R; a++) {
+                h8 hi, lo;
+                q4k_min_operand_m(q4k_mins(hd[a]), valid ? hd[a].x >> 16 : 0u, hi, lo);
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const h8 bv = valid ? __builtin_bit_cast(h8, bd[b]) : h8{};
+                    acc[a][b] = mfma(lo, bv, mfma(hi, bv, acc[a][b]));
+                }
+            }
+        }
+    }
     // every wave's copies of the first stage and block have landed before any wave passes
     wait_vm<0>();
     pin_r();
@@ -332,10 +368,12 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
                     for (int a = 0; a < R; a++) {
                         d[a] = h2f(w4[a].h.x & 0xFFFFu);
-                        const bool cap = (k & 3) == q;
-                        const uint2 mn = q4k_min_pack(w4[a].h);
-                        mins[a].x = cap ? mn.x : mins[a].x;
-                        mins[a].y = cap ? mn.y : mins[a].y;
+                        if constexpr (kLate) {
+                            const bool cap = (k & 3) == q;
+                            const uint2 mn = q4k_min_pack(w4[a].h);
+                            mins[a].x = cap ? mn.x : mins[a].x;
+                            mins[a].y = cap ? mn.y : mins[a].y;
+                        }
                         if (d[a] == 0.0f) w4[a].h.y = w4[a].h.w = 0u;  // scales 0: the block's products are zero
                     }
                 } else if (d[0] == 0.0f) {
@@ -400,40 +438,44 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                 // the window's last blocks: lane groups past the row's end add nothing
                 const bool valid = 4 * w + q < nkb;
                 const int sb = min(4 * w + q, nkb - 1);
-                uint32_t rowa = lds + (uint32_t)offsetof(GwLds<TYPE>, row) + 4 * c;
-                asm volatile("" : "+v"(rowa));  // formed here, not held through the loop
-                float dr[R][4];
-#pragma unroll
-                for (int a = 0; a < R; a++) {
-#pragma unroll
-                    for (int x = 0; x < 4; x++) dr[a][x] = __shfl(deff[a], 4 * q + x);
-                    deff[a] = 1.0f;
-                }
-                // every operand is loaded before the first is used: the lane's fragments are dead
+                const uint32_t rowa = lds + (uint32_t)offsetof(GwLds<TYPE>, row) + 4 * (lane_here() & 15);
+                // a group's operands are loaded before the first is used: the lane's fragments are dead
                 // here, and their registers take them
-                float dt[NB];
-                h8 bd[Q4 ? NB : 1];
+                constexpr int NC = NB > 4 && kLate ? NB / 2 : NB;  // columns at a time
 #pragma unroll
-                for (int b = 0; b < NB; b++) {
-                    const size_t tok = lds_get<uint32_t>(rowa, 64 * b);
-                    dt[b] = g.a_dlast[tok * nwin + w];
-                    if constexpr (Q4) bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
-                }
+                for (int b0 = 0; b0 < NB; b0 += NC) {
+                    float dt[NC];
+                    h8 bd[kLate ? NC : 1];
 #pragma unroll
-                for (int a = 0; a < R; a++) {
-                    h8 hi, lo;
-                    if constexpr (Q4) q4k_min_operand(valid ? mins[a] : make_uint2(0u, 0u), hi, lo);
+                    for (int b = 0; b < NC; b++) {
+                        const size_t tok = lds_get<uint32_t>(rowa, 64 * (b0 + b));
+                        dt[b] = g.a_dlast[tok * nwin + w];
+                        if constexpr (kLate)
+                            bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
+                    }
 #pragma unroll
-                    for (int b = 0; b < NB; b++) {
-                        f4 &ac = acc[a][b];
+                    for (int a = 0; a < R; a++) {
+                        float dr[4];
 #pragma unroll
-                        for (int x = 0; x < 4; x++) ac[x] *= dr[a][x] * dt[b];
-                        if constexpr (Q4) {
-                            const h8 bv = valid ? bd[b] : h8{};
-                            ac = mfma(lo, bv, mfma(hi, bv, ac));
+                        for (int x = 0; x < 4; x++) dr[x] = __shfl(deff[a], 4 * q + x);
+                        h8 hi, lo;
+                        if constexpr (kLate) q4k_min_operand(valid ? mins[a] : make_uint2(0u, 0u), hi, lo);
+#pragma unroll
+                        for (int b = 0; b < NC; b++) {
+                            f4 &ac = acc[a][b0 + b];
+                            f4 to = {0.f, 0.f, 0.f, 0.f};
+                            if constexpr (kLate) {
+                                const h8 bv = valid ? bd[b] : h8{};
+                                to = mfma(lo, bv, mfma(hi, bv, to));
+                            }
+#pragma unroll
+                            for (int x = 0; x < 4; x++) ac[x] = __builtin_fmaf(ac[x], dr[x] * dt[b], to[x]);
                         }
                     }
+                    if constexpr (NC < NB) __builtin_amdgcn_sched_barrier(0);
                 }
+#pragma unroll
+                for (int a = 0; a < R; a++) deff[a] = 1.0f;
             }
             // the next stage's activations have landed for every wave (and, from the second
             // stage on, the next block's weights)
@@ -445,11 +487,12 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     }
 
     // D layout: lane holds weight rows 4q + x of each 16-row tile, token column c
+    const int le = lane_here();
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int j = j0 + 16 * b + c;
+        const int j = j0 + 16 * b + (le & 15);
         if (j >= n_rows) continue;
-        float *orow = g.out + (size_t)(row_base + j) * g.out_ld + base + 4 * q;
+        float *orow = g.out + (size_t)(row_base + j) * g.out_ld + base + 4 * (le >> 4);
         if constexpr (MODE == 1) {
             f4 v;
 #pragma unroll
@@ -472,7 +515,7 @@ __global__ void __launch_bounds__(64 * Gw<TYPE>::kWaves)
     __attribute__((amdgpu_waves_per_eu(Gw<TYPE>::kPerEu, Gw<TYPE>::kPerEu))) gemm_grouped_kernel(GroupedArgs g) {
     __shared__ __align__(16) GwLds<TYPE> L;
     const uint32_t lds = lds_addr(&L);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Workgroups go to the 8 XCDs in turn.  The row blocks of one tile share its activation rows, so
     // they run on one XCD (tiles are dealt to the XCDs in turn, heaviest first) and read them from
     // its L2; the last n % 8 tiles are spread over all XCDs.  With every tile spread, the rows came
@@ -494,7 +537,7 @@ __global__ void __launch_bounds__(64 * Gw<TYPE>::kWaves)
     const int e = tl >> 16, nt = tl & 0xFFFF;
     const int n_rows = g.counts[e], row_base = g.offsets[e], j0 = nt * kGroupTile;
     const int nvalid = min(kGroupTile, n_rows - j0);
-#define MNEMO_GW(NB_) gw_tile<TYPE, MODE, NB_>(g, L, lds, rb, wave, lane, tid, e, j0, n_rows, row_base)
+#define MNEMO_GW(NB_) gw_tile<TYPE, MODE, NB_>(g, L, lds, rb, wave, e, j0, n_rows, row_base)
     // one instantiation per count of 16-row column tiles, so every MFMA is unconditional (5
     // and 7 run padded to 6 and 8)
     switch ((nvalid + 15) >> 4) {
