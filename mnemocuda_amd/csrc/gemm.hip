@@ -178,7 +178,7 @@ struct RawW<kTypeQ6K> {
 };
 
 template <int TYPE, int R, int RG, int KS, int NB, bool ONCE>
-__global__ void __launch_bounds__(64 * RG * KS) __attribute__((amdgpu_waves_per_eu(R * NB <= 4 ? 4 : 2)))
+__global__ void __launch_bounds__(64 * RG * KS) __attribute__((amdgpu_waves_per_eu(R * NB <= 4 && KS * NB <= 8 ? 4 : 2)))
 gemm_q8_1_kernel(GemmArgs g) {
     using Lds = GemmLds<TYPE, R, RG, KS, NB>;
     constexpr bool Q4 = TYPE == kTypeQ4K;
@@ -626,27 +626,34 @@ static int device_cus_gemm() {
     return cus;
 }
 
-// The workgroup shapes and what each costs.  A launch of t tiles runs in ceil(t / CUs) rounds (one
-// workgroup per CU: the workgroups are latency-bound, a second one per CU gains nothing), and a
-// round takes c1 us per super-block of a K slice plus c2 us (first loads, the slices' sums,
-// the stores); c0: the launch.  Fitted to 520 sizes (M 512-8192, K 512-8192, N 1-2048, both
-// types; rms 6 %): the choice with the least cost is within 1.3 % of the fastest shape on
-// average and 29 % at worst (Q6_K, K = 1536, a slice per block).
+// The workgroup shapes and what each costs: t tiles on C CUs, nsb super-blocks in ks slices, take
+//   c0 + ceil(t / C) (c1 ceil(nsb / ks) + c2) + t / C (c3 nsb / ks + c4)  us:
+// the launch; the rounds, each as long as its longest slice; and what the tiles cost each other (a
+// wave's issue rate and the memory).  Where a shape's LDS and registers let two workgroups share a CU, a
+// second one is not free: two rounds of the 64 x 64 tile of two slices take 1.7 times one.  Constants
+// fitted to 891 sizes (M 64-10^4, K 256-12,288, N 1-2,350, both types; rms of the shapes near the
+// best 8 % Q4_K, 15 % Q6_K): the choice is 2 % slower than the fastest shape on average and 23 % at worst.
 // Large products take the wide tiles (fewest conversions and LDS reads per MFMA), small ones
-// narrow tiles with K in up to 8 slices, so that the launch still covers the chip.
+// narrow tiles with K in up to 16 slices, so that the launch still covers the chip.  Shapes 8 to 11 are
+// for few tiles of long rows, above all of Q6_K, whose super-blocks take a wave longest:
+// M = 1836, K = 8960, N = 39 38.3 us without them, 26 with; 1359 x 4352, N = 776 74 and 59.
 struct GemmShape {
     int r, rg, ks, nb;
-    double q4[3], q6[3];
+    double q4[5], q6[5];
 };
-#define MNEMO_GEMM_SHAPES(X)                                                      \
-    X(0, 2, 8, 1, 8, {-7.7, 5.82, 14.7}, {-8.3, 9.14, 16.2}) /* 256 x 128 */      \
-    X(1, 2, 4, 2, 8, {-2.5, 6.46, 9.3}, {-3.0, 10.3, 10.5})  /* 128 x 128 */      \
-    X(2, 2, 4, 2, 4, {0.8, 4.46, 4.6}, {0.6, 7.39, 5.5})     /* 128 x 64 */       \
-    X(3, 1, 4, 2, 4, {5.1, 2.84, 0.4}, {4.2, 3.96, 0.9})     /* 64 x 64 */        \
-    X(4, 1, 4, 4, 4, {1.5, 5.40, 1.6}, {1.0, 8.34, 0.1})     /* 64 x 64 */        \
-    X(5, 1, 4, 4, 2, {3.3, 3.96, 0.4}, {2.6, 6.96, -1.0})    /* 64 x 32 */        \
-    X(6, 1, 2, 8, 2, {3.2, 5.40, -0.2}, {3.9, 9.15, -3.6})   /* 32 x 32 */        \
-    X(7, 2, 1, 8, 1, {5.4, 4.16, -1.7}, {5.4, 7.99, -4.5})   /* 32 x 16 */
+#define MNEMO_GEMM_SHAPES(X) \
+    X(0, 2, 8, 1, 8, {0, 5.92, 5.13, 0.28, 20.42}, {5.99, 9.02, 0.81, 0.26, 21.96})     /* 256 x 128 */  \
+    X(1, 2, 4, 2, 8, {3.88, 6.19, 2.18, 0.43, 10.28}, {1.98, 10.28, 0.08, 0.24, 13.92}) /* 128 x 128 */  \
+    X(2, 2, 4, 2, 4, {4.18, 3.86, 0.91, 0.82, 4.56}, {3.09, 6.91, 0, 0.76, 6.43})       /* 128 x 64 */   \
+    X(3, 1, 4, 2, 4, {5.73, 2.5, 0, 0.14, 1.08}, {4.58, 4.06, 0, 0, 1.12})              /* 64 x 64 */    \
+    X(4, 1, 4, 4, 4, {2.87, 3.98, 1.95, 1.86, 0.5}, {1.13, 6.19, 2.13, 3.57, 0})        /* 64 x 64 */    \
+    X(5, 1, 4, 4, 2, {4.82, 2.6, 0.94, 1.44, 0}, {3.94, 4.85, 0, 3.38, 0})              /* 64 x 32 */    \
+    X(6, 1, 2, 8, 2, {4.97, 3.24, 0.26, 2.02, 0}, {2.34, 6.45, 0, 2.45, 0})             /* 32 x 32 */    \
+    X(7, 2, 1, 8, 1, {6.16, 2.17, 0, 1.07, 0}, {2.96, 5.78, 0, 1.34, 0})                /* 32 x 16 */    \
+    X(8, 1, 1, 16, 1, {5.98, 2.23, 0, 2.87, 0}, {6.27, 2.01, 0, 8.09, 0})               /* 16 x 16 */    \
+    X(9, 1, 4, 2, 8, {1.92, 4.37, 2.82, 0.84, 3.36}, {1.51, 5.22, 2.56, 0.83, 3.23})    /* 64 x 128 */   \
+    X(10, 1, 2, 4, 4, {3.57, 3.16, 1.69, 1.11, 0}, {4.74, 4.17, 0, 1.01, 0})            /* 32 x 64 */    \
+    X(11, 1, 1, 8, 2, {5.81, 2.33, 0, 1.9, 0}, {5.05, 3.3, 0, 1.52, 0})                 /* 16 x 32 */
 #define MNEMO_GEMM_SHAPE(I_, R_, RG_, KS_, NB_, ...) {R_, RG_, KS_, NB_, __VA_ARGS__},
 static const GemmShape kShapes[] = {MNEMO_GEMM_SHAPES(MNEMO_GEMM_SHAPE)};
 
@@ -689,7 +696,8 @@ static GemmPlan gemm_plan(int type, int M, int K, int N, int cus) {
             // only shape 0 has a form that rounds once)
             if (type == kTypeQ4K && nsb == 1 && h.r * h.nb > 8 && i) continue;
             const long tiles = (long)gemm_tiles(M, 16 * h.r * h.rg) * gemm_tiles(N, 16 * h.nb);
-            const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]);
+            const double t = c[0] + (double)((tiles + cus - 1) / cus) * (c[1] * ((nsb + h.ks - 1) / h.ks) + c[2]) +
+                             (double)tiles / cus * (c[3] * nsb / h.ks + c[4]);
             if (p.shape < 0 || t < least) {
                 p.shape = i;
                 least = t;

@@ -62,9 +62,11 @@ RAGGED = [
     (6001, 2304, 513), (2047, 4352, 1027), (8190, 1280, 1025), (4093, 5376, 2047),
     # at most one super-block per slice
     (8197, 256, 197), (8263, 512, 195), (8307, 256, 68), (8603, 256, 33), (8201, 768, 33), (4131, 1280, 17),
+    (8917, 256, 1), (4109, 256, 1), (5551, 256, 130), (10883, 256, 325), (8311, 512, 338), (2097, 768, 33),
     # more than four
     (33, 8448, 1), (33, 8704, 2070), (8219, 4352, 1), (8455, 4352, 33), (9395, 4864, 34), (8395, 2304, 34),
-    (5409, 2304, 337), (8225, 2304, 65), (8401, 2304, 104),
+    (5409, 2304, 337), (8225, 2304, 65), (8401, 2304, 104), (33, 16640, 1), (4123, 8448, 1), (4245, 8704, 17),
+    (4655, 4352, 34), (199, 4352, 2157), (8993, 2304, 129),
 ]
 
 
