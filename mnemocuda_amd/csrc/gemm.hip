@@ -535,9 +535,9 @@ gemm_q8_1_kernel(GemmArgs g) {
 // (per 32 values d = amax/127, q = rint(x*127/amax) clamped to +-127, ds = f16(d * sum x);
 // gemm_q4k.cu:327-358): q8 as f16 integers [N][K] in the operands' element order
 // (gemm_ops.hpp), the f16 ds [N][K/32], the running-scale
-// ratio rho_s = d8eff_{s-1} / d8eff_s [N][K/32] and d8eff at the end of every window of 32
-// sub-blocks (1024 values) [N][ceil(K/1024)].  d8eff is the last nonzero f16 d8 at or before s
-// in s's window, 1 before the window's first.  One wave per row.
+// ratio rho_s = d8eff_{s-1} / d8eff_s [N][K/32] and d8eff at the end of every 256 values
+// [N][K/256].  d8eff is the last nonzero f16 d8 at or before s in s's window of 32 sub-blocks
+// (1024 values), 1 before the window's first.  K a multiple of 256.  One wave per row.
 constexpr int kStageThreads = 256;
 
 __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *__restrict__ x, int K, int N,
@@ -602,7 +602,7 @@ __global__ void __launch_bounds__(kStageThreads) stage_f32_kernel(const float *_
         const float cur = d8 != 0.0f ? d8 : prev;
         if (b < nsub) {
             rho[(size_t)row * nsub + b] = prev / cur;
-            if ((b & 31) == 31 || b == nsub - 1) dlast[(size_t)row * ((nsub + 31) / 32) + b / 32] = cur;
+            if ((b & 7) == 7) dlast[(size_t)row * (nsub / 8) + b / 8] = cur;
         }
     }
 }

@@ -36,7 +36,7 @@ struct GroupedArgs {
     const _Float16 *A;       // staged q8 rows, f16 integers [rows][K]
     const float *a_rho;      // [rows][K/32] token scale ratios
     const uint16_t *a_ds;    // [rows][K/32] f16 ds
-    const float *a_dlast;    // [rows][ceil(K/1024)] d8 unit at the end of each window
+    const float *a_dlast;    // [rows][K/256] d8 unit at the end of each block
     float *out;
     int K, out_ld;           // K a multiple of 256
     int row_blocks;          // workgroups per token tile
@@ -272,12 +272,18 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     }
     asm volatile("" : "+v"(rra));
 
+    constexpr f4 kZero = {0.f, 0.f, 0.f, 0.f};
+    constexpr bool kTot = Q4 && MODE == 2 && NB <= 4;
     f4 acc[R][NB];
-    float deff[R];  // running d of the lane's A row c of each tile
+    f4 tot[kTot ? R : 1][kTot ? NB : 1];  // the sums of the blocks before
+    float deff[R];  // running d of the lane's A row c of each tile (kTot: the block's d)
 #pragma unroll
     for (int a = 0; a < R; a++) {
 #pragma unroll
-        for (int b = 0; b < NB; b++) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < NB; b++) {
+            acc[a][b] = kZero;
+            if constexpr (kTot) tot[a][b] = kZero;
+        }
         deff[a] = 1.0f;
     }
     if (tid < 16 * NB) lds_put<uint32_t>(lds + (uint32_t)offsetof(GwLds<TYPE>, row), 4 * tid, (uint32_t)stage_row(tid));
@@ -300,17 +306,19 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     // end the term is formed on zero and the accumulators join it by one fma, which makes them absolute
     // (4.9e-7 relative L2 against 64 bits, 5.1e-7 with the term added to the absolute accumulators;
     // SwiGLU rows of K = 4096).
-    // Down: the accumulators start as the whole term.  Where activations are large the term and the
-    // products are larger than their sum, and the roundings scale with the sum so far: K = 768 1.07e-7
-    // against 1.39e-7 with the term at the windows' ends, K = 512 9.0e-8 against 9.9e-8.  (Activations
-    // several times larger, near where ds leaves the f16 range, favour the other order.)  It reads the
-    // headers' lines once more: the launch takes 130 us instead of 123 at K = 768, M = 2048, 16,384
-    // rows; gate/up of 512 tokens would pay 3 %.
-    constexpr bool kLate = Q4 && MODE == 1;
-    uint2 mins[kLate ? R : 1];
-    const int nwin = (nkb + 3) / 4;
-    if constexpr (Q4 && !kLate) {
-        for (int w = 0; w < nwin; w++) {
+    // Down: the products are larger than their sum with the term where activations are large, and the
+    // roundings scale with the sum so far.  Up to 64 tokens the registers hold a total beside the
+    // block's sum, so that only one rounding per block is at the total's magnitude (K = 1024 7.5e-8;
+    // 1.6e-7 in one sum.  Gate/up would gain as much and take 1.4 % longer at 37 and 512 tokens).  Wider tiles
+    // start their accumulators as the whole term, which keeps the sum near the result all the way:
+    // K = 768 1.07e-7, 1.39e-7 with the term at the windows' ends; K = 512 9.0e-8 and 9.9e-8.
+    // (Activations several times larger, near where ds leaves the f16 range, favour the other order.)
+    // It reads the headers' lines once more: at K = 768, M = 2048 130 us instead of 123 for
+    // 16,384 rows; narrow tiles, which the weights' bytes bound, would take 10 % longer.
+    constexpr bool kMins = Q4 && (MODE == 1 || kTot);
+    uint2 mins[kMins ? R : 1];
+    if constexpr (Q4 && !kMins) {
+        for (int w = 0; 4 * w < nkb; w++) {
             const bool valid = 4 * w + q < nkb;  // lane groups past the row's end add nothing
             const int sb = min(4 * w + q, nkb - 1);
             uint4 hd[R], bd[NB];
@@ -336,6 +344,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
     pin_r();
     lds_barrier();
 
+    // LDS address of the token row of the lane's column
+    auto row_addr = [&] { return lds + (uint32_t)offsetof(GwLds<TYPE>, row) + 4 * (lane_here() & 15); };
     for (int k = 0; k < nkb; k++) {
         const int kn = min(k + 1, nkb - 1);  // past the end the last block is copied again
         // block k's weights into registers; the area is refilled once they are there
@@ -361,6 +371,14 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
             else if (W == 4 || wave < 4) lds_put<float>(lds_r + 4 * (uint32_t)tid, sizeof L.rho[0], rn);
             copy_b(tn, buf ^ 1);
             if (s == NS - 1) load_r(kn);
+            float dtk[kTot ? NB : 1];  // the tokens' units at the block's end
+            if constexpr (kTot) {
+                if (s == NS - 1) {
+                    const uint32_t rowa = row_addr();
+#pragma unroll
+                    for (int b = 0; b < NB; b++) dtk[b] = g.a_dlast[(size_t)lds_get<uint32_t>(rowa, 64 * b) * nkb + k];
+                }
+            }
             if (s == 0) {
                 copy_w(kn);
                 if constexpr (!Q4) load_d6(kn);
@@ -368,7 +386,7 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
                     for (int a = 0; a < R; a++) {
                         d[a] = h2f(w4[a].h.x & 0xFFFFu);
-                        if constexpr (kLate) {
+                        if constexpr (kMins) {
                             const bool cap = (k & 3) == q;
                             const uint2 mn = q4k_min_pack(w4[a].h);
                             mins[a].x = cap ? mn.x : mins[a].x;
@@ -383,6 +401,10 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                 // rows 4q + x, whose ratios come from lanes 4q + x
 #pragma unroll
                 for (int a = 0; a < R; a++) {
+                    if constexpr (kTot) {
+                        deff[a] = d[a];
+                        continue;
+                    }
                     const float nd = d[a] == 0.0f ? deff[a] : d[a];
                     const float sg = ratio(deff[a], nd);
                     deff[a] = nd;
@@ -426,7 +448,8 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
 #pragma unroll
                         for (int b = 0; b < NC; b++) {
                             f4 &ac = acc[a][NC * gr + b];
-                            ac *= rr[b];
+                            if (kTot && j == 0) ac = kZero;
+                            else ac *= rr[b];
                             ac = mfma(a1[a], bf[b], ac);
                             if constexpr (!Q4) ac = mfma(a2[a], bf[b], ac);
                         }
@@ -434,48 +457,69 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
                 }
             }
             if (s == NS - 1 && ((k & 3) == 3 || k == nkb - 1)) {  // uniform: the window's end
-                const int w = k >> 2;
                 // the window's last blocks: lane groups past the row's end add nothing
-                const bool valid = 4 * w + q < nkb;
-                const int sb = min(4 * w + q, nkb - 1);
-                const uint32_t rowa = lds + (uint32_t)offsetof(GwLds<TYPE>, row) + 4 * (lane_here() & 15);
+                const bool valid = (k & ~3) + q < nkb;
+                const int sb = min((k & ~3) + q, nkb - 1);
+                const uint32_t rowa = row_addr();
                 // a group's operands are loaded before the first is used: the lane's fragments are dead
                 // here, and their registers take them
-                constexpr int NC = NB > 4 && kLate ? NB / 2 : NB;  // columns at a time
+                constexpr int NC = NB > 4 && kMins ? NB / 2 : NB;  // columns at a time
 #pragma unroll
                 for (int b0 = 0; b0 < NB; b0 += NC) {
                     float dt[NC];
-                    h8 bd[kLate ? NC : 1];
+                    h8 bd[kMins ? NC : 1];
 #pragma unroll
                     for (int b = 0; b < NC; b++) {
                         const size_t tok = lds_get<uint32_t>(rowa, 64 * (b0 + b));
-                        dt[b] = g.a_dlast[tok * nwin + w];
-                        if constexpr (kLate)
+                        if constexpr (!kTot) dt[b] = (g.a_dlast + k)[(uint32_t)tok * (uint32_t)nkb];
+                        if constexpr (kMins)
                             bd[b] = __builtin_bit_cast(h8, ld16((const uint8_t *)(g.a_ds + tok * (K / 32) + 8 * sb)));
                     }
 #pragma unroll
                     for (int a = 0; a < R; a++) {
                         float dr[4];
+                        if constexpr (!kTot) {
 #pragma unroll
-                        for (int x = 0; x < 4; x++) dr[x] = __shfl(deff[a], 4 * q + x);
+                            for (int x = 0; x < 4; x++) dr[x] = __shfl(deff[a], 4 * q + x);
+                        }
                         h8 hi, lo;
-                        if constexpr (kLate) q4k_min_operand(valid ? mins[a] : make_uint2(0u, 0u), hi, lo);
+                        if constexpr (kMins) q4k_min_operand(valid ? mins[a] : make_uint2(0u, 0u), hi, lo);
 #pragma unroll
                         for (int b = 0; b < NC; b++) {
                             f4 &ac = acc[a][b0 + b];
-                            f4 to = {0.f, 0.f, 0.f, 0.f};
-                            if constexpr (kLate) {
+                            f4 to = kZero;
+                            if constexpr (kTot) to = tot[a][b0 + b];
+                            if constexpr (kMins) {
                                 const h8 bv = valid ? bd[b] : h8{};
                                 to = mfma(lo, bv, mfma(hi, bv, to));
                             }
+                            if constexpr (kTot) {
+                                tot[a][b0 + b] = to;
+                            } else {
 #pragma unroll
-                            for (int x = 0; x < 4; x++) ac[x] = __builtin_fmaf(ac[x], dr[x] * dt[b], to[x]);
+                                for (int x = 0; x < 4; x++) ac[x] = __builtin_fmaf(ac[x], dr[x] * dt[b], to[x]);
+                            }
                         }
                     }
                     if constexpr (NC < NB) __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int a = 0; a < R; a++) deff[a] = 1.0f;
+                for (int a = 0; a < R; a++)
+                    if constexpr (!kTot) deff[a] = 1.0f;
+            }
+            if constexpr (kTot) {
+                if (s == NS - 1)  // the block's sum, absolute, joins the total
+#pragma unroll
+                    for (int a = 0; a < R; a++) {
+                        float dr[4];
+#pragma unroll
+                        for (int x = 0; x < 4; x++) dr[x] = __shfl(deff[a], 4 * q + x);
+#pragma unroll
+                        for (int b = 0; b < NB; b++)
+#pragma unroll
+                            for (int x = 0; x < 4; x++)
+                                tot[a][b][x] = __builtin_fmaf(acc[a][b][x], dr[x] * dtk[b], tot[a][b][x]);
+                    }
             }
             // the next stage's activations have landed for every wave (and, from the second
             // stage on, the next block's weights)
@@ -486,6 +530,12 @@ __device__ __forceinline__ void gw_tile(const GroupedArgs &g, const GwLds<TYPE> 
         }
     }
 
+    if constexpr (kTot) {
+#pragma unroll
+        for (int a = 0; a < R; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = tot[a][b];
+    }
     // D layout: lane holds weight rows 4q + x of each 16-row tile, token column c
     const int le = lane_here();
 #pragma unroll

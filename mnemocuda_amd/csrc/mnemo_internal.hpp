@@ -13,7 +13,7 @@ constexpr int kGroupTile = 128;
 // Activation rows staged for the grouped GEMM (gemm.hip, stage_f32_kernel): the Q8_1 values
 // of each row as f16 integers [rows][K], the f16 ds of each 32-value sub-block [rows][K/32],
 // the running-scale ratio of each sub-block [rows][K/32] and the d8 unit at the end of every
-// 1024-value window [rows][ceil(K/1024)].
+// 256 values [rows][K/256].
 struct StagedAct {
     _Float16 *q8;
     float *rho;

@@ -13,7 +13,7 @@
 //
 // Workspace layout (each part 256-byte aligned), sizes for T tokens, k slots, E experts:
 //   xs      T staged rows of x (StagedAct: q8 [T][hidden] f16, rho and ds [T][hidden/32],
-//           dlast [T][ceil(hidden/1024)])
+//           dlast [T][hidden/256])
 //   counts  E ints, offsets E ints
 //   rank    T*k ints   (rank of a pair within its expert and wave range; -1 for dropped slots)
 //   inv     T*k ints   (pair -> expert-sorted row, -1 for dropped slots)
@@ -72,7 +72,7 @@ static MoeLayout moe_layout(int T, int hidden, int eff, int E, int k) {
     L.xs = take((size_t)T * hidden * 2);
     L.xr = take((size_t)T * (hidden / 32) * 4);
     L.xds = take((size_t)T * (hidden / 32) * 2);
-    L.xdl = take((size_t)T * ((hidden + 1023) / 1024) * 4);
+    L.xdl = take((size_t)T * (hidden / 256) * 4);
     L.counts = take((size_t)E * 4);
     L.offsets = take((size_t)E * 4);
     L.rank = take(pairs * 4);
@@ -83,7 +83,7 @@ static MoeLayout moe_layout(int T, int hidden, int eff, int E, int k) {
     L.acts = take(pairs * eff * 2);
     L.actr = take(pairs * (eff / 32) * 4);
     L.actds = take(pairs * (eff / 32) * 2);
-    L.actdl = take(pairs * ((eff + 1023) / 1024) * 4);
+    L.actdl = take(pairs * (eff / 256) * 4);
     L.down = take(pairs * hidden * 4);
     L.total = o;
     return L;

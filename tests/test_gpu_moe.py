@@ -533,7 +533,7 @@ def test_moe_decode_unaligned_table(gpu, oracle):
 
 
 def test_moe_prefill_q4k_down_rounding(gpu):
-    """The Q4_K down projection's roundings.  Its sum starts as the min term, M, and takes the products
+    """The Q4_K down projection's roundings, in tiles of 128 and 72 tokens.  Its sum starts as the min term, M, and takes the products
     P_s of the 24 sub-blocks one by one, two roundings each, so the error's square is the sum of
     2 (2^-24 / sqrt(3))^2 S_s^2 at most, S_s = M + P_1 + .. + P_s; over mantissas in [1, 2) the mean is
     0.54 of that (0.74 in the error), and 15 % more is left for the last few roundings and the draw.
