@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the quantized-matmul hot path on one MI355X.
 
-Headline workload (BASELINE.json configs[1]): Qwen3-235B-shape attention projections,
+Headline workload: Qwen3-235B-shape attention projections,
 decode batch 1, hidden 4096.  One step = the projections of all 94 layers for one token:
 Q Q4_K 4096->8192 with K (Q4_K) + V (Q6_K) 4096->512 each in one launch
 (mnemo_matvec_qkv), then O Q4_K 8192->4096 with fp32 residual -- 188 launches over
@@ -214,7 +214,7 @@ def gpu_bench(args):
 
 
 def decode_bench(gen, stream, layers, tokens, ctx_pos, cache_ctx=40960, long_pos=0):
-    """configs[2] inside a full decode step (forward.c:687-1077 per layer, then the lm_head
+    """The MoE block inside a full decode step (forward.c:687-1077 per layer, then the lm_head
     and sampling, forward.c:1601-1707), one token at cache position ctx_pos, ctx_pos+1, ...:
     per layer  fused Q/K/V with the attention RMS norm -> GQA decode attention over 0..pos
     with the QK norm, RoPE and f16 KV store in its launch (position in device memory) -> O (+ residual) ->
@@ -343,7 +343,7 @@ def attention_bench(stream, lengths=(1024, 4096, 16384, 32768)):
 
 
 def moe_prefill_bench(gen, stream):
-    """grouped-expert prefill, 512 tokens x top-8 of 128 experts (Zipf 1.1),
+    """Grouped-expert prefill, 512 tokens x top-8 of 128 experts (Zipf 1.1),
     gate+up Q4_K 4096->1536, down Q6_K 1536->4096, router-weighted scatter-add."""
     import numpy as np
     import torch
@@ -449,7 +449,7 @@ def main():
         "vs_baseline": None,
         "dtype": "i8 dot4 (q4/q6 weights x int8 digits of x), fp32 rescale and accumulate",
         "data": "synthetic (seeded GGUF Q4_K/Q6_K blocks with the benchmark configs' value distributions, generated in HBM)",
-        "config": {"workload": "configs[1]: Qwen3-235B attention projections, decode batch=1, hidden 4096, "
+        "config": {"workload": "Qwen3-235B attention projections, decode batch=1, hidden 4096, "
                                "94 layers per step (Q 4096->8192 Q4_K + K Q4_K + V Q6_K 4096->512 in one "
                                "launch, O 8192->4096 Q4_K + residual), hipGraph replay",
                    "global_batch": 1, "layers": LAYERS, "parallelism": "single GPU"},

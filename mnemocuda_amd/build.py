@@ -2,8 +2,7 @@
 
 HIP sources are compiled with hipcc for gfx950 only; the C host composition
 (csrc/host/mnemo_host.c) with the system C compiler; both link into one shared library
-whose exported symbols are exactly the declarations of include/mnemo_kernels.h and
-include/mnemo_host.h.
+that exports the declarations of the headers under include/ (and internal symbols).
 """
 from __future__ import annotations
 

@@ -26,7 +26,7 @@
 //     is a window of 1024 values, acc is also multiplied by d_prev / d of the rows at super-block
 //     boundaries, becomes absolute at the window's end, and the scales start again from 1.  Q4_K's
 //     wide tiles form acc * rho and let the MFMA add the products to it (two roundings): forming t
-//     first costs them 5 % (M = 4096, K = 4096, N = 1024: 69.0 against 73.2 us).  A zero scale
+//     first costs them 5 % (M = 4096, K = 4096, N = 1024: 69.0 against 73.2 us with the quantizer).  A zero scale
 //     leaves the running scale unchanged and zeroes its block's operand (its products are zero).
 //   * Q4_K's min term, sum_s -(dmin*m_s) * ds_js, is one more product over the sub-block
 //     index: -dmin*m (an f16 times a 6-bit integer, 17 significant bits) is split into an
@@ -66,8 +66,8 @@ namespace mnemo {
 // that a stage or window waited for was moved out of it: the Q4_K min term's operands come from
 // LDS (read from memory at each window's end they cost 8 400 cycles per window), the conversion
 // of the next stage sits in front of the multiplication in the same basic block (so the two
-// interleave), addresses are scalars plus constants.  M = 8192, K = 4096, N = 512: 81.4 -> 64 us
-// (540 TOPS); M = 4096, K = 8192, N = 1999: 319 -> 200 us (670 TOPS); N = 7: 25.5 -> 12 us, with
+// interleave), addresses are scalars plus constants.  M = 8192, K = 4096, N = 512: 81.4 -> 62 us
+// (550 TOPS); M = 4096, K = 8192, N = 1999: 319 -> 198 us (677 TOPS); N = 7: 25.5 -> 13 us, with
 // the tiled kernel before (128 x 128 tiles, operands of both sides through LDS, K split over
 // workgroups by atomics) on the left.
 constexpr int kStageK = 64;  // K per stage

@@ -16,12 +16,12 @@
 // weights ~12 operations to form the operand, and 4 per 16 x 16 outputs for the running
 // scale, against one 16-cycle MFMA).  Both need work in flight from phases that do not
 // coincide, so the kernel runs as several small workgroups per CU (Q4_K: three of 4 waves,
-// 52 KB of LDS and 168 registers each; Q6_K: two of 8 waves, 128 registers): one workgroup's
+// 52 KB of LDS and at most 168 registers each; Q6_K: two of 8 waves, 128 registers): one workgroup's
 // copies, barriers, first loads and final stores pass while the others multiply.  No
 // instantiation spills: a reload in the loop waits for every copy issued before it (14 spilled
 // registers in the 128-token tiles: 423 against 398 us, below).
-// MoE prefill of 512 tokens (128 experts of 4096 -> 1536, top-8, Q6_K down): 830 -> 618 us; of 37
-// tokens 363 -> 275; of 2048 (64 experts of 2048 -> 768, Q4_K down) 654 -> 382; before: one
+// MoE prefill of 512 tokens (128 experts of 4096 -> 1536, top-8, Q6_K down): 830 -> 609 us; of 37
+// tokens 363 -> 277; of 2048 (2048 -> 768, Q4_K down) 654 -> 388; before: one
 // workgroup of 8 or 16 waves per CU, 64-token tiles.
 #include <cstddef>
 

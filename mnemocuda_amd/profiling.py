@@ -9,7 +9,7 @@
   qkv  -- the fused QKV GEMV of bench.py's workload (one layer's weights, 4 launches);
   gemm -- the M=512 Q4_K prefill GEMMs of bench.py (N=8192 and N=1536, one launch per weight
           buffer over 600 MB of distinct buffers);
-  moe  -- bench.py's grouped-expert prefill (configs[4], 3 calls);
+  moe  -- bench.py's grouped-expert prefill (512 tokens, 3 calls);
   decode -- bench.py's decode layer (fused QKV with the norm, attention at position 2048, O +
           residual, the MoE block with 128 resident experts) over 4 layers of distinct
           weights, 3 tokens, then the lm_head Q6_K 151,936 x 4096 GEMV and top-p sampling.

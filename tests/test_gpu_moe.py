@@ -4,11 +4,11 @@ Reference for the added delta out - out0: the reference's expert chain applied t
 (src/forward.c:876-893 per expert, src/forward.c:1783-1830 per token) in the Q8_1 GEMM
 semantics -- Oracle.moe_prefill (fp64, C) at test sizes and its torch restatement
 (tests/torch_ref.py, fp64 on the GPU, pinned against the oracle on the CPU) at the benchmark
-cfg5 shape.  Bar: relative L2 <= 1e-3 (north_star).  The GEMMs sum every sub-block exactly,
+cfg5 shape.  Bar: relative L2 <= 1e-3.  The GEMMs sum every sub-block exactly,
 so the remaining difference is the SwiGLU's exp rounding moving a requantized value by one
 step now and then (measured ~1e-6); a wrong expert, slot or weight is an O(1) error.
 The per-expert composition of the plain entry points is a second reference at the same bar.
-Routing edge cases: experts with no tokens, an expert spanning several 64-row tiles, dropped
+Routing edge cases: experts with no tokens, an expert spanning several 128-row tiles, dropped
 slots (id -1 or >= n_experts), one token.  The cfg5 shape is also checked for bitwise
 run-to-run determinism."""
 import numpy as np
@@ -67,11 +67,10 @@ def _compose_plain(gpu, table, lay, DT, x, idx, w, T, H, EFF, out0):
     (300, 256, 512, 4, 2, 12, 3.0),    # expert 0 spans several tiles
     (1, 256, 256, 8, 8, 14, 1.1),      # one token, every expert once
     (37, 768, 256, 32, 3, 14, 0.0),    # most experts empty or single-row
-    # experts of 1-3 full 64-row tiles plus a ragged one
+    # experts of one ragged tile, of a full one and a ragged one
     (130, 256, 256, 2, 1, 14, 0.0),
     (200, 512, 256, 5, 2, 12, 0.5),
-    # Q4_K K in whole 1024-value windows (1-3 of them; the min term formed after the main
-    # loop), and K = 5120 (five windows: the min term before the loop, in two passes)
+    # K in whole 1024-value windows, one to five of them
     (48, 1024, 1024, 4, 2, 12, 0.5),
     (24, 2048, 256, 3, 2, 14, 1.1),
     (70, 3072, 256, 2, 1, 14, 0.0),
@@ -145,8 +144,7 @@ def test_moe_prefill_tile_widths(gpu, counts, H, EFF, k, down_type):
 @pytest.mark.parametrize("H", [512, 2048])
 def test_moe_prefill_zero_d_blocks(gpu, oracle, H):
     """Gate/up Q4_K blocks with d = 0 (dmin kept, so only the min term survives), scattered
-    and over whole rows, with K below one 1024-value window (min term before the main loop)
-    and K in two whole windows (min term after it, from the headers the loop reads)."""
+    and over whole rows, with K below one 1024-value window and K in two whole windows."""
     T, EFF, E, k, DT = 96, 256, 4, 2, 14
     rng = np.random.default_rng(H + 7)
     table = synth.expert_table(rng, E, H, EFF, DT)
