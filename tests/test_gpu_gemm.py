@@ -108,6 +108,31 @@ def test_gemm_rounds_once_per_sub_block(gpu, type_id, M, K, N):
     assert err < bar
 
 
+# Wide tiles keep one running sum per slice.  Per sub-block Q6_K's is rounded once (an fma), Q4_K's
+# twice, and the scale ratio carries a rounding of its own; one more per super-block (the row's
+# scale), all at the running sum's magnitude (half of them, as above); two at the end.  The root mean square over
+# mantissas in [1, 2) is 0.74 of a rounding's 2^-24 / sqrt(3); 15 % on top.
+@pytest.mark.parametrize("type_id", [12, 14])
+@pytest.mark.parametrize("M,K,N", [(8192, 4096, 512), (4096, 8192, 1999)])
+def test_gemm_wide_tiles_rounding(gpu, type_id, M, K, N):
+    from tests.test_gemm_plan import plan
+    case(f"gemm wide rounding type={type_id} M={M} K={K} N={N}")
+    shape, _, _, slices, *_ = plan(type_id, M, K, N)
+    assert shape < 2
+    rng = np.random.default_rng(M + K + N)
+    w = dev(synth.weights(rng, type_id, M, K))
+    x = torch.randn((N, K), device="cuda", generator=torch.Generator("cuda").manual_seed(M))
+    act = torch.zeros(N * (K // 128) * 144, dtype=torch.uint8, device="cuda")
+    gpu.ops.quantize_q8_1(x, act, K, N)
+    out = _run(gpu, type_id, w, act, M, K, N)
+    sub = K // 32 / slices
+    roundings = (3 if type_id == 12 else 2) * sub / 2 + sub / 8 / 2 + 2
+    bar = 1.15 * 0.74 * 2.0**-24 * (roundings / 3) ** 0.5
+    err = rel_l2(host(out), torch_ref.gemm(type_id, w, act, M, K, N).cpu().numpy())
+    print(f"rel_l2={err:.3e} bar {bar:.3e}")
+    assert err < bar
+
+
 @pytest.mark.parametrize("type_id", [12, 14])
 def test_gemm_zero_scales_and_range(gpu, oracle, type_id):
     """Zero weight blocks (d = 0 with nonzero quants), zero activation sub-blocks and sub-blocks
@@ -185,8 +210,11 @@ def test_gemm_large_activations(gpu, oracle, type_id):
 
 
 def test_gemm_rows_over_4_gib(gpu):
-    """33 Q6_K rows of 137.6 MB: one workgroup's rows would span more than a 32-bit offset."""
-    M, K, N = 33, 5 << 25, 1
+    """17 Q6_K rows of 275 MB: even the smallest tile's rows would span more than a 32-bit offset."""
+    from tests.test_gemm_plan import plan
+    M, K, N = 17, 5 << 26, 1
+    _, _, _, slices, rows1, _ = plan(14, M, K, N)
+    assert rows1 < M  # two launches
     nsb = K // 256
     gen = torch.Generator("cuda").manual_seed(3)
     w = torch.randint(0, 256, (M, nsb, 210), dtype=torch.uint8, device="cuda", generator=gen)
@@ -195,7 +223,7 @@ def test_gemm_rows_over_4_gib(gpu):
     act[:, :, :16] = torch.tensor([0.01, 0.0] * 4, dtype=torch.float16).view(torch.uint8).cuda()
     case(f"gemm long rows M={M} K={K} N={N}")
     out = _run(gpu, 14, w.view(-1), act.view(-1), M, K, N)
-    rows = [0, 1, 15, 27, 28, 30, 31, 32]  # both launches, the first and last of each among them
+    rows = [0, 1, 7, rows1 - 1, rows1, 14, 15, 16]  # the first and last of both launches among them
     ref = torch.zeros((N, len(rows)), dtype=torch.float64, device="cuda")
     var = torch.zeros_like(ref)
     w = w[rows]
@@ -205,13 +233,13 @@ def test_gemm_rows_over_4_gib(gpu):
         part = torch_ref.gemm(14, w[:, b:b + n].reshape(-1), act[:, 2 * b:2 * (b + n)].reshape(-1), len(rows), 256 * n, N)
         ref += part
         var += part * part
-    # A slice sums n = 81,920 super-blocks of either sign, one rounding each (2^-24 / sqrt(3) of the sum
+    # A slice sums n super-blocks of either sign, one rounding each (2^-24 / sqrt(3) of the sum
     # so far at most): the sum's square grows evenly to the slice's share of var, so the error's square is
     # n / 2 * 2^-48 / 3 of var on average.  Over 8 outputs it is spread like a chi-square of 8 degrees
     # (half of it): twice the error is six spreads.  A row read 4 GiB away is an error of the result's
     # size, 10^5 times that.
     err = float((out[:, rows].double() - ref).norm() / var.sum().sqrt())
-    bar = 2 * 2.0**-24 * (nsb / 8 / 6) ** 0.5
+    bar = 2 * 2.0**-24 * (nsb / slices / 6) ** 0.5
     print(f"err={err:.2e} bar {bar:.2e}")
     assert err < bar
 
